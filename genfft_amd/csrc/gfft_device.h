@@ -411,6 +411,12 @@ __device__ __forceinline__ void stockham_passes(cx<T> *lds, const cx<T> *__restr
 }
 
 template <int R, int... RS>
+constexpr int first_radix()
+{
+    return R;
+}
+
+template <int R, int... RS>
 constexpr int last_radix()
 {
     if constexpr (sizeof...(RS) == 0) return R;

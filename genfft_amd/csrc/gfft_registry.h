@@ -7,6 +7,7 @@
 #include <type_traits>
 
 #include "gfft_device.h"
+#include "gfft_regtile.h"
 #include "gfft_wave.h"
 
 namespace gfft {
@@ -27,6 +28,8 @@ struct KernelEntry {
     int store;       // 0: complex T in memory; 1: FP16 pairs; 2: BF16 pairs (FP32 arithmetic)
     int gen_tw;      // 1: the last pass builds its twiddles from TileArgs::gen_lo / gen_hi (W_L)
     int wave;        // 1: one wavefront per row, lanes exchanged without LDS (wave_rows1024_kernel)
+    int reg;         // 1: tile held in registers (reg_tile_kernel); its own pass twiddle table layout
+    int long_row;    // 1: a row longer than the LDS row tiles (the planner takes it by its own rule)
     int wide;        // 1: double-width row tile the planner takes for batches past the Infinity Cache
 };
 
@@ -117,6 +120,68 @@ constexpr KernelEntry make_pipe_entry()
 {
     KernelEntry e = pipe_shape<T, L, M, NT, LAY, INP, OUTP, RS...>();
     e.fn = &tile_fft_pipe_kernel<T, L, M, NT, LAY, INP, OUTP, RS...>;
+    return e;
+}
+
+template <typename T, int L, int M, int NT, int LAY, int INP, int OUTP, int... RS>
+constexpr KernelEntry make_pipe_variant()
+{
+    KernelEntry e = make_pipe_entry<T, L, M, NT, LAY, INP, OUTP, RS...>();
+    e.tune_only = 1;
+    return e;
+}
+
+// A tile held in registers (reg_tile_kernel), with its stores streamed.
+template <typename T, int L, int M, int NT, int INP, int OUTP, int HINT, int... RS>
+constexpr KernelEntry reg_shape()
+{
+    static_assert(((RS * ...) == L), "radices must multiply to L");
+    static_assert(NT % 64 == 0 && NT <= 1024, "whole wavefronts, at most 1024 threads");
+    using G = PlaneGeom<T, L, M, first_radix<RS...>(), INP == PAT_ROW>;
+    static_assert(G::ELEMS * sizeof(T) <= 160 * 1024, "exchange plane exceeds gfx950 LDS");
+    KernelEntry e{};
+    e.prec = sizeof(T) == 8 ? 1 : 0;
+    e.L = L;
+    e.M = M;
+    e.NT = NT;
+    e.layout = INP == PAT_ROW ? LAY_SEQ : LAY_ELEM;
+    e.inp = INP;
+    e.outp = OUTP;
+    e.nrad = sizeof...(RS);
+    const int r[] = {RS...};
+    for (int i = 0; i < (int)sizeof...(RS); i++) e.rad[i] = r[i];
+    e.lds_bytes = (int)(G::ELEMS * sizeof(T));
+    e.gen_tw = sizeof(T) == 4;
+    e.reg = 1;
+    e.fn = &reg_tile_kernel<T, L, M, NT, INP, OUTP, HINT, RS...>;
+    return e;
+}
+
+template <typename T, int L, int M, int NT, int INP, int OUTP, int... RS>
+constexpr KernelEntry make_reg_entry()
+{
+    return reg_shape<T, L, M, NT, INP, OUTP, HINT_ST, RS...>();
+}
+
+// The row tile with streaming loads as well, which the planner takes for
+// batches past the Infinity Cache (KernelEntry::wide).
+template <typename T, int L, int M, int NT, int... RS>
+constexpr KernelEntry make_reg_wide()
+{
+    KernelEntry e = reg_shape<T, L, M, NT, PAT_ROW, PAT_ROW, HINT_LD | HINT_ST, RS...>();
+    e.tune_only = 1;
+    e.wide = 1;
+    return e;
+}
+
+// A row longer than the LDS row tiles.
+template <typename T, int L, int NT, int HINT, int... RS>
+constexpr KernelEntry make_reg_long()
+{
+    KernelEntry e = reg_shape<T, L, 1, NT, PAT_ROW, PAT_ROW, HINT, RS...>();
+    e.tune_only = 1;
+    e.long_row = 1;
+    e.wide = (HINT & HINT_LD) ? 1 : 0;
     return e;
 }
 

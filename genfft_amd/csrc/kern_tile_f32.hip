@@ -1,15 +1,15 @@
 // kern_tile_f32.hip -- complex64 tile-kernel shapes.
 //
 // Rows (PAT_ROW -> PAT_ROW, sequence-major LDS): batched 1D transforms and
-// the 2D row pass; a tile holds 4096 complex (32 KB) up to L = 4096, then a
-// single sequence up to L = 16384 (136 KB of gfx950's 160 KB LDS).
+// the 2D row pass; a tile holds 4096 complex (32 KB) up to L = 4096.
 // Columns (PAT_COL -> PAT_COL, element-major LDS): the first pass of a
 // four-step transform and the 2D column pass; M adjacent columns give
 // >= 64-byte contiguous row segments.
 // Transposing rows (PAT_ROW -> PAT_COL): the second four-step pass, writing
 // element k of row k1 to k1 + N1*k, M rows wide.
-// Every default shape keeps 16 elements per thread, so radix-16 butterflies
-// live entirely in registers (the radix-32 alternatives hold 32).
+// Every default LDS shape keeps 16 elements per thread, so radix-16 butterflies
+// live entirely in registers (the radix-32 alternatives hold 32).  Rows from
+// 8192 points on are held in registers (gfft_regtile.h).
 #include "gfft_registry.h"
 
 namespace gfft {
@@ -30,9 +30,9 @@ const KernelEntry kTable[] = {
     make_entry<T, 512, 8, 256, S_, R_, R_, 8, 8, 8>(),
     make_entry<T, 1024, 4, 256, S_, R_, R_, 16, 16, 4>(),
     make_entry<T, 2048, 2, 256, S_, R_, R_, 16, 16, 8>(),
-    make_entry<T, 4096, 1, 256, S_, R_, R_, 16, 16, 16>(),
-    make_entry<T, 8192, 1, 512, S_, R_, R_, 16, 16, 8, 4>(),
-    make_entry<T, 16384, 1, 1024, S_, R_, R_, 16, 16, 16, 4>(),
+    make_variant<T, 4096, 1, 256, S_, R_, R_, 16, 16, 16>(),
+    make_variant<T, 8192, 1, 512, S_, R_, R_, 16, 16, 8, 4>(),
+    make_variant<T, 16384, 1, 1024, S_, R_, R_, 16, 16, 16, 4>(),
     // --- column tiles ---
     make_entry<T, 2, 512, 64, E_, C_, C_, 2>(),
     make_entry<T, 4, 256, 64, E_, C_, C_, 4>(),
@@ -67,12 +67,13 @@ const KernelEntry kTable[] = {
     // 0.479, 16*16*4: 0.493; the transposing row pass does not move with order)
     make_pipe_entry<T, 1024, 16, 1024, E_, C_, C_, 16, 4, 16>(),
     make_pipe_entry<T, 1024, 16, 1024, S_, R_, C_, 16, 16, 4>(),
-    // single 16384-point sequences (tile: 136 KB of LDS); radix 16*4*16*16:
+    // (tuner alternative) single 16384-point sequences (tile: 136 KB of LDS);
+    // radix 16*4*16*16:
     // c64 2^14 x 8192 0.500 ms with the pass twiddles read from global memory
     // (16*16*16*4: 0.509, 16*16*4*16: 0.502, 4*16*16*16: 0.521), 0.442 ms with
     // the last pass's twiddles generated from a 4 KB table in LDS
     // (PassTw::GEN: the first three passes' 8 KB of tables fit beside it)
-    make_pipe_entry<T, 16384, 1, 1024, S_, R_, R_, 16, 4, 16, 16>(),
+    make_pipe_variant<T, 16384, 1, 1024, S_, R_, R_, 16, 4, 16, 16>(),
     // --- autotuner alternatives: radix order, tile width, threads per tile.
     // The double-width row tiles (64 KB, 512 threads; make_wide_variant) are
     // also the planner's choice for batches of >= 512 MiB: measured on MI355X
@@ -91,11 +92,26 @@ const KernelEntry kTable[] = {
     make_variant<T, 2048, 2, 256, S_, R_, R_, 8, 16, 16>(),
     make_wide_variant<T, 2048, 4, 512, S_, R_, R_, 16, 16, 8>(),
     make_variant<T, 4096, 2, 512, S_, R_, R_, 16, 16, 16>(),
-    make_variant<T, 4096, 1, 512, S_, R_, R_, 8, 8, 8, 8>(),
+    // 512 threads of radix 8: 4096-point rows 5.5 -> 5.0 us (one), 12.9 -> 12.9
+    // (1024), 0.388 -> 0.384 ms (1 GiB) against 16*16*16 with 256 threads
+    make_entry<T, 4096, 1, 512, S_, R_, R_, 8, 8, 8, 8>(),
     make_variant<T, 8192, 1, 512, S_, R_, R_, 16, 16, 16, 2>(),
     make_variant<T, 16384, 1, 1024, S_, R_, R_, 16, 16, 8, 8>(),
     // one wavefront per 1024-point row, lanes exchanged by DPP / permlane swaps
     make_wave_entry<256>(),
+    // --- rows held in registers (LDS plane 34 / 69 / 135 KB: four / two / one
+    // workgroup per CU).  MI355X, 1 GiB batches, streaming loads: 8192 points
+    // 0.427 -> 0.364 ms, 16384 0.435 -> 0.360-0.387 ms, 32768 0.72 -> 0.46 ms
+    // (four-step); 256 MiB batches, plain loads: 0.087 -> 0.067 ms (8192) and
+    // 0.104 -> 0.079 ms (16384); from one row up to 16 the LDS tiles' time.
+    // The streaming 16384-point tile runs 16*4*16*16 with 1024 threads, the
+    // order of the LDS tile before it: 0.387 ms (32*32*16 with 512: 0.375) ---
+    make_reg_entry<T, 8192, 1, 256, R_, R_, 32, 16, 16>(),
+    make_reg_wide<T, 8192, 1, 256, 32, 16, 16>(),
+    make_reg_entry<T, 16384, 1, 512, R_, R_, 32, 32, 16>(),
+    make_reg_wide<T, 16384, 1, 1024, 16, 4, 16, 16>(),
+    make_reg_long<T, 32768, 1024, HINT_ST, 32, 32, 32>(),
+    make_reg_long<T, 32768, 1024, HINT_LD | HINT_ST, 32, 32, 32>(),
 };
 // The 2^20 four-step's two pipelined passes paired in one launch (column pass
 // of chunk k, transposing row pass of chunk k - 1).

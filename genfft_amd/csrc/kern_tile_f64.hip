@@ -2,9 +2,9 @@
 //
 // Same three families as complex64 (rows, column tiles, transposing rows)
 // with half the elements per tile, since each element is 16 bytes: rows hold
-// 2048 complex (32 KB) up to L = 2048 and a single sequence up to L = 8192;
-// column tiles are >= 8 columns (128-byte segments) where LDS allows.  The
-// batched rows use radix-8 passes (FP64 register pressure, see below).
+// 2048 complex (32 KB) up to L = 128 and are held in registers from L = 256 on
+// (gfft_regtile.h); column tiles are >= 8 columns (128-byte segments) where
+// LDS allows.
 #include "gfft_registry.h"
 
 namespace gfft {
@@ -21,16 +21,18 @@ const KernelEntry kTable[] = {
     make_entry<T, 32, 64, 128, S_, R_, R_, 8, 4>(),
     make_entry<T, 64, 32, 128, S_, R_, R_, 8, 8>(),
     make_entry<T, 128, 16, 128, S_, R_, R_, 16, 8>(),
-    // radix <= 8 and 8 elements per thread from L = 256 on: an FP64 radix-16
-    // butterfly holds 64 VGPRs of data plus 60 of twiddles (148-190 VGPRs per
-    // kernel); the radix-8 forms use 83-116 and run 25-30% faster (MI355X,
-    // 1 GiB batches: L = 1024 0.624 -> 0.449 ms, 8192 0.787 -> 0.569 ms)
-    make_entry<T, 256, 8, 256, S_, R_, R_, 8, 8, 4>(),
-    make_entry<T, 512, 4, 256, S_, R_, R_, 8, 8, 8>(),
-    make_entry<T, 1024, 2, 256, S_, R_, R_, 8, 4, 8, 4>(),
-    make_entry<T, 2048, 1, 256, S_, R_, R_, 8, 8, 8, 4>(),
-    make_entry<T, 4096, 1, 512, S_, R_, R_, 8, 8, 8, 8>(),
-    make_entry<T, 8192, 1, 1024, S_, R_, R_, 8, 8, 8, 8, 2>(),
+    // tuner alternatives to the register-held rows below, and the kernels of
+    // layouts past their 32-bit offsets; radix <= 8 and 8 elements per thread:
+    // an FP64 radix-16 butterfly holds 64 VGPRs of data plus 60 of twiddles
+    // (148-190 VGPRs per kernel); the radix-8 forms use 83-116 and run 25-30%
+    // faster (MI355X, 1 GiB batches: L = 1024 0.624 -> 0.449 ms, 8192 0.787 ->
+    // 0.569 ms)
+    make_variant<T, 256, 8, 256, S_, R_, R_, 8, 8, 4>(),
+    make_variant<T, 512, 4, 256, S_, R_, R_, 8, 8, 8>(),
+    make_variant<T, 1024, 2, 256, S_, R_, R_, 8, 4, 8, 4>(),
+    make_variant<T, 2048, 1, 256, S_, R_, R_, 8, 8, 8, 4>(),
+    make_variant<T, 4096, 1, 512, S_, R_, R_, 8, 8, 8, 8>(),
+    make_variant<T, 8192, 1, 1024, S_, R_, R_, 8, 8, 8, 8, 2>(),
     // --- column tiles ---
     make_entry<T, 2, 256, 64, E_, C_, C_, 2>(),
     make_entry<T, 4, 256, 64, E_, C_, C_, 4>(),
@@ -67,6 +69,26 @@ const KernelEntry kTable[] = {
     make_variant<T, 2048, 1, 128, S_, R_, R_, 16, 16, 8>(),
     make_variant<T, 4096, 1, 256, S_, R_, R_, 16, 16, 16>(),
     make_variant<T, 8192, 1, 512, S_, R_, R_, 16, 16, 8, 4>(),
+    // --- rows held in registers.  MI355X against the LDS tiles above, 1 GiB
+    // batches (streaming loads) / 256 MiB batches (plain loads) / one row:
+    // 256 points 0.374 -> 0.350 ms / 0.101 -> 0.063 ms / 4.1 -> 3.9 us, 1024
+    // 0.378 -> 0.349 / 0.101 -> 0.068 / 4.9 -> 4.6, 4096 0.417 -> 0.362 /
+    // 0.116 -> 0.090 / 7.5 -> 6.2, 8192 0.579 -> 0.345 / 0.157 -> 0.083 /
+    // 12.8 -> 10.3; 16384 points against the four-step 0.77 -> 0.435 ms ---
+    make_reg_entry<T, 256, 8, 256, R_, R_, 8, 4, 8>(),
+    make_reg_wide<T, 256, 8, 256, 8, 4, 8>(),
+    make_reg_entry<T, 512, 4, 256, R_, R_, 8, 8, 8>(),
+    make_reg_wide<T, 512, 4, 256, 8, 8, 8>(),
+    make_reg_entry<T, 1024, 2, 256, R_, R_, 8, 4, 4, 8>(),
+    make_reg_wide<T, 1024, 2, 256, 8, 4, 4, 8>(),
+    make_reg_entry<T, 2048, 1, 128, R_, R_, 16, 16, 8>(),
+    make_reg_wide<T, 2048, 1, 128, 16, 16, 8>(),
+    make_reg_entry<T, 4096, 1, 256, R_, R_, 16, 16, 16>(),
+    make_reg_wide<T, 4096, 1, 256, 16, 16, 16>(),
+    make_reg_entry<T, 8192, 1, 512, R_, R_, 8, 16, 8, 8>(),
+    make_reg_wide<T, 8192, 1, 512, 8, 16, 8, 8>(),
+    make_reg_long<T, 16384, 1024, HINT_ST, 16, 16, 8, 8>(),
+    make_reg_long<T, 16384, 1024, HINT_LD | HINT_ST, 16, 16, 8, 8>(),
 };
 // The 2^20 four-step's two pipelined passes paired in one launch (column pass
 // of chunk k, transposing row pass of chunk k - 1).

@@ -113,8 +113,8 @@ void twiddle_ld(int64_t m, int64_t n, long double *c, long double *s)
 
 struct DeviceTables {
     std::mutex mu;
-    // (device, prec, L, radices) -> pass twiddles
-    std::map<std::tuple<int, int, int, std::vector<int>>, void *> pass;
+    // (device, prec, L, entry order, radices) -> pass twiddles
+    std::map<std::tuple<int, int, int, int, std::vector<int>>, void *> pass;
     // (device, N) -> two-level FP64 table {lo, hi}
     std::map<std::pair<int, int64_t>, std::pair<void *, void *>> two_level;
 };
@@ -133,7 +133,9 @@ int upload(void **dst, const void *src, size_t bytes)
 }
 
 // Stockham pass twiddles of one tile shape: for each pass with NS > 1,
-// entries [m*(R-1) + r-1] = W_{NS*R}^(r*m), m < NS, r = 1..R-1.
+// entries [m*(R-1) + r-1] = W_{NS*R}^(r*m), m < NS, r = 1..R-1; at
+// [(r-1)*NS + m] for the kernels that hold their tile in registers, whose
+// lanes read consecutive m.
 int get_pass_twiddles(int dev, const KernelEntry &k, const void **out, bool dry)
 {
     if (dry) {
@@ -143,7 +145,7 @@ int get_pass_twiddles(int dev, const KernelEntry &k, const void **out, bool dry)
     auto &T = tables();
     std::lock_guard<std::mutex> lk(T.mu);
     std::vector<int> rad(k.rad, k.rad + k.nrad);
-    auto key = std::make_tuple(dev, k.prec, k.L, rad);
+    auto key = std::make_tuple(dev, k.prec, k.L, k.reg, rad);
     auto it = T.pass.find(key);
     if (it != T.pass.end()) {
         *out = it->second;
@@ -154,13 +156,13 @@ int get_pass_twiddles(int dev, const KernelEntry &k, const void **out, bool dry)
     for (int p = 0; p < k.nrad; p++) {
         const int R = k.rad[p];
         if (ns > 1)
-            for (int64_t m = 0; m < ns; m++)
-                for (int r = 1; r < R; r++) {
-                    long double c, s;
-                    twiddle_ld((int64_t)r * m, ns * R, &c, &s);
-                    re.push_back(c);
-                    im.push_back(s);
-                }
+            for (int64_t e = 0; e < ns * (R - 1); e++) {
+                const int64_t m = k.reg ? e % ns : e / (R - 1), r = 1 + (k.reg ? e / ns : e % (R - 1));
+                long double c, s;
+                twiddle_ld(r * m, ns * R, &c, &s);
+                re.push_back(c);
+                im.push_back(s);
+            }
         ns *= R;
     }
     if (re.empty()) {  // single-pass shapes read no twiddles; keep a valid pointer
@@ -298,12 +300,15 @@ const KernelEntry *tile_table(int prec, int store, int *cnt)
     return prec ? tile_kernels_f64(cnt) : tile_kernels_f32(cnt);
 }
 
+// With `lds` only tiles kept in LDS count (layouts whose offsets the register-
+// held tiles cannot address, and the shapes the tuning alternatives vary).
 const KernelEntry *find_tile(int prec, int L, int inp, int outp, int prefer_m = 0, int pipe_mask = 3,
-                             int variant = -1, int store = 0)
+                             int variant = -1, int store = 0, bool lds = false)
 {
     int cnt = 0;
     const KernelEntry *tab = tile_table(prec, store, &cnt);
-    if (variant >= 0 && variant < cnt && tab[variant].L == L && tab[variant].inp == inp && tab[variant].outp == outp)
+    if (variant >= 0 && variant < cnt && tab[variant].L == L && tab[variant].inp == inp &&
+        tab[variant].outp == outp && !(lds && tab[variant].reg))
         return &tab[variant];
     const bool pipe = (inp == PAT_COL ? (pipe_mask & 1) : (pipe_mask & 2)) != 0;
     const KernelEntry *best = nullptr;
@@ -315,7 +320,8 @@ const KernelEntry *find_tile(int prec, int L, int inp, int outp, int prefer_m = 
     };
     for (int i = 0; i < cnt; i++) {
         const KernelEntry &e = tab[i];
-        if (e.L != L || e.inp != inp || e.outp != outp || e.tune_only) continue;
+        if (e.L != L || e.inp != inp || e.outp != outp) continue;
+        if (lds ? e.reg || e.wide || e.wave : e.tune_only) continue;
         if (better(e)) best = &e;
     }
     return best;
@@ -335,7 +341,7 @@ int narrow_row_variant(int prec, int L, int64_t batch, int num_cus)
     const KernelEntry *tab = tile_table(prec, 0, &cnt);
     for (int i = 0; i < cnt; i++) {
         const KernelEntry &e = tab[i];
-        if (e.L != L || e.inp != PAT_ROW || e.outp != PAT_ROW || e.wave || e.wide || e.persistent) continue;
+        if (e.L != L || e.inp != PAT_ROW || e.outp != PAT_ROW || e.wave || e.wide || e.reg || e.persistent) continue;
         if (e.M < d->M && (best < 0 || e.M < tab[best].M)) best = i;
     }
     return best;
@@ -348,7 +354,18 @@ int row_variant_of(int prec, int L, int KernelEntry::*flag)
     int cnt = 0;
     const KernelEntry *tab = tile_table(prec, 0, &cnt);
     for (int i = 0; i < cnt; i++)
-        if (tab[i].*flag && tab[i].L == L && tab[i].inp == PAT_ROW && tab[i].outp == PAT_ROW) return i;
+        if (tab[i].*flag && !tab[i].long_row && tab[i].L == L && tab[i].inp == PAT_ROW && tab[i].outp == PAT_ROW) return i;
+    return -1;
+}
+
+// Registry index of the register-held tile of a row one length past the LDS
+// row tiles (KernelEntry::long_row), with or without streaming loads, or -1.
+int long_row_index(int prec, int64_t n, bool wide)
+{
+    int cnt = 0;
+    const KernelEntry *tab = tile_table(prec, 0, &cnt);
+    for (int i = 0; i < cnt; i++)
+        if (tab[i].long_row && tab[i].L == n && (tab[i].wide != 0) == wide) return i;
     return -1;
 }
 
@@ -380,7 +397,7 @@ int max_len(int prec, int inp, int outp, int store = 0)
     int cnt = 0, best = 0;
     const KernelEntry *tab = tile_table(prec, store, &cnt);
     for (int i = 0; i < cnt; i++)
-        if (tab[i].inp == inp && tab[i].outp == outp) best = std::max(best, tab[i].L);
+        if (tab[i].inp == inp && tab[i].outp == outp && !tab[i].long_row) best = std::max(best, tab[i].L);
     return best;
 }
 
@@ -588,10 +605,16 @@ struct gfft_plan_s {
     // input is read: a launch that reads the input and writes the output
     // (its workgroups store while others have yet to load), or an output
     // write ahead of a later input read (a batch run in chunks).  Overlapping
-    // buffers are then staged (needs_stage) unless every transform is in
+    // buffers are then staged (route) unless every transform is in
     // place: in == out with equal byte distances in_step / out_step (batch
     // members, or rows) and in_step2 / out_step2 (2D images).
     bool overlap_hazard = false;
+    // The launches of the same plan without register-held long rows (none: it
+    // has none).  They read every input before they write an output wherever
+    // the four-step does, so a call on overlapping buffers runs these, through
+    // the workspace they were sized for, and no staging copy is needed.
+    std::vector<gfft::Launch> alt;
+    bool alt_hazard = false;
     int64_t in_step = 0, out_step = 0, in_step2 = 0, out_step2 = 0;
     void *stage = nullptr;  // copy of an input that overlaps the output (allocated on first use)
     std::mutex host_mu;
@@ -617,6 +640,15 @@ bool tile_offsets_fit(int pat, int64_t L, int64_t M, int64_t inner, int64_t elem
     return last * (int64_t)csize < ((int64_t)1 << 31);
 }
 
+// Batches of at least this many bytes a side stream through HBM: row tiles
+// with the `wide` flag.
+constexpr int64_t kStreamBytes = (int64_t)512 << 20;
+// Rows from which a register-held tile per row beats the four-step (MI355X, us
+// per call at 64 / 96 / 128 / 256 rows: c64 32768 points 18.1 / 18.3 / 19.5 /
+// 32 against 16.0 / 23.3 / 28 / 54, c128 16384 points 17.4 / 18.2 / 20.9 / 33
+// against 19.5 / 24.6 / 30 / 51).
+constexpr int64_t kLongRows = 96;
+
 struct Builder {
     gfft_plan_s *p;
     int prec;
@@ -626,6 +658,8 @@ struct Builder {
     PlanOpts opts = resolve_opts(prec, 0, forced);
     int64_t scratch_elems = 0;  // complex elements of scratch needed
     int store = 0;              // 16-bit storage format (tile_kernels_f16 / _bf16), default shapes only
+    bool no_long_rows = false;  // rows past the LDS tiles run as a four-step (gfft_plan_s::alt)
+    bool long_rows = false;     // set when some took the register-held tile
 
     void need_scratch(int64_t elems) { scratch_elems = std::max(scratch_elems, elems); }
 
@@ -647,6 +681,9 @@ struct Builder {
              int tw_mode, int64_t tw_n, bool first, bool last, int variant = -1)
     {
         const KernelEntry *k = find_tile(prec, L, inp, outp, prefer_m, opts.pipe_mask, variant, store);
+        if (k && k->reg && !(tile_offsets_fit(inp, k->L, k->M, in_inner, in_elem, csize) &&
+                             tile_offsets_fit(outp, k->L, k->M, out_inner, out_elem, csize)))
+            k = find_tile(prec, L, inp, outp, prefer_m, opts.pipe_mask, -1, store, true);
         if (!k) return fail(GFFT_ERR_UNSUPPORTED, "no tile kernel for L=%d pattern %d->%d", L, inp, outp);
         Launch l;
         l.type = LT_TILE;
@@ -734,6 +771,22 @@ struct Builder {
         return GFFT_OK;
     }
 
+    // Register-held row tile for `batch` rows of length n, one past the LDS
+    // row tiles, or -1 (four-step).  One workgroup owns a row, so below half
+    // the CUs the four-step's shorter tiles spread a small batch wider.
+    int long_row_variant(int64_t n, int64_t batch) const
+    {
+        if (store || no_long_rows || opts.dual || opts.n1_log2) return -1;
+        if (opts.row_variant >= 0) {  // tuned
+            int cnt = 0;
+            const KernelEntry *tab = tile_table(prec, 0, &cnt);
+            const int v = opts.row_variant;
+            return v < cnt && tab[v].long_row && tab[v].L == n ? v : -1;
+        }
+        if (batch < kLongRows) return -1;
+        return long_row_index(prec, n, n * batch * (int64_t)csize >= kStreamBytes);
+    }
+
     // Batched 1D complex transforms of length n; `batch` transforms at
     // distances in_dist / out_dist (complex elements).
     int c2c_1d(int64_t n, int64_t batch, int in_buf, int64_t in_off, int64_t in_dist, int out_buf,
@@ -771,12 +824,18 @@ struct Builder {
             int variant = opts.row_variant;
             if (variant < 0 && !store) {
                 if (batch == 1) variant = row_variant_of(prec, (int)n, &KernelEntry::wave);
-                else if (n * batch * (int64_t)csize >= ((int64_t)512 << 20))
+                else if (n * batch * (int64_t)csize >= kStreamBytes)
                     variant = row_variant_of(prec, (int)n, &KernelEntry::wide);
                 else variant = narrow_row_variant(prec, (int)n, batch, p->num_cus);
             }
             return tile((int)n, PAT_ROW, PAT_ROW, 0, in_buf, in_off, out_buf, out_off, batch, 1, 1, 0, 0,
                         in_dist, 1, 0, 0, out_dist, 1, TW_NONE, 0, first, last, variant);
+        }
+        // one length past the LDS row tiles a row still fits a workgroup's registers
+        if (const int v = long_row_variant(n, batch); v >= 0) {
+            long_rows = true;
+            return tile((int)n, PAT_ROW, PAT_ROW, 0, in_buf, in_off, out_buf, out_off, batch, 1, 1, 0, 0,
+                        in_dist, 1, 0, 0, out_dist, 1, TW_NONE, 0, first, last, v);
         }
         // four-step: n = N1 (column length) * N2 (row length)
         const int lg = ilog2(n);
@@ -1125,11 +1184,12 @@ bool output_before_input_done(const std::vector<Launch> &launches)
 int plan_via_dense_copy(gfft_plan_s *p, bool dry, const PlanOpts *forced, const gfft_desc &dense, bool input_side,
                         const RepackArgs &rp);
 
-int build_plan(gfft_plan_s *p, bool dry, const PlanOpts *forced = nullptr)
+int build_plan(gfft_plan_s *p, bool dry, const PlanOpts *forced = nullptr, bool no_long_rows = false)
 {
     const gfft_desc &d = p->d;
     Builder b{p, p->prec, csize_of(p->prec, p->store), dry, forced};
     b.store = p->store;
+    b.no_long_rows = no_long_rows;
     if (p->store) b.opts = PlanOpts{};
     const size_t cs = b.csize, rs = cs / 2;
     const int64_t n = d.n, batch = d.batch;
@@ -1431,6 +1491,18 @@ int build_plan(gfft_plan_s *p, bool dry, const PlanOpts *forced = nullptr)
     b.scratch_elems = std::max<int64_t>(b.scratch_elems, 0);
     p->scratch_bytes = (size_t)b.scratch_elems * cs;
     p->overlap_hazard = output_before_input_done(p->launches);
+    if (b.long_rows) {
+        std::vector<Launch> direct;
+        direct.swap(p->launches);
+        const bool hazard = p->overlap_hazard;
+        const size_t scratch = p->scratch_bytes;
+        if ((st = build_plan(p, dry, forced, true))) return st;
+        p->alt.swap(p->launches);
+        p->alt_hazard = p->overlap_hazard;
+        p->launches.swap(direct);
+        p->overlap_hazard = hazard;
+        p->scratch_bytes = std::max(scratch, p->scratch_bytes);
+    }
     return GFFT_OK;
 }
 
@@ -1495,7 +1567,15 @@ int plan_via_dense_copy(gfft_plan_s *p, bool dry, const PlanOpts *forced, const 
 // Plan-time bounds proof: the largest byte offset each launch can touch,
 // from the same index formulas the kernels use, must lie inside its buffer.
 // A planner mistake becomes an error here instead of a device fault.
+int validate_list(const gfft_plan_s *p, const std::vector<Launch> &launches);
+
 int validate(const gfft_plan_s *p)
+{
+    const int st = validate_list(p, p->launches);
+    return st ? st : validate_list(p, p->alt);
+}
+
+int validate_list(const gfft_plan_s *p, const std::vector<Launch> &launches)
 {
     const int64_t cs = (int64_t)csize_of(p->prec, p->store), rs = cs / 2;
     const int64_t ext[3] = {(int64_t)p->in_bytes, (int64_t)p->out_bytes, (int64_t)p->scratch_bytes};
@@ -1524,7 +1604,7 @@ int validate(const gfft_plan_s *p)
         if (k->lds_bytes > 160 * 1024) return fail(GFFT_ERR_UNSUPPORTED, "internal: LDS");
         return GFFT_OK;
     };
-    for (const Launch &l : p->launches) {
+    for (const Launch &l : launches) {
         int st = GFFT_OK;
         idx++;
         switch (l.type) {
@@ -1646,7 +1726,11 @@ int describe(const gfft_plan_s *p, char *buf, size_t len)
     char line[256];
     snprintf(line, sizeof(line), "plan in_bytes=%zu out_bytes=%zu scratch_bytes=%zu\n", p->in_bytes,
              p->out_bytes, p->scratch_bytes);
-    return describe_launches(p->launches, line, buf, len);
+    if (p->alt.empty()) return describe_launches(p->launches, line, buf, len);
+    int st = describe_launches(p->launches, line, buf, len);
+    if (st) return st;
+    const std::string head = std::string(buf) + "on overlapping buffers:\n";
+    return describe_launches(p->alt, head, buf, len);
 }
 
 int describe_launches(const std::vector<Launch> &launches, const std::string &head, char *buf, size_t len)
@@ -1659,11 +1743,11 @@ int describe_launches(const std::vector<Launch> &launches, const std::string &he
         case LT_TILE: {
             const TileArgs &a = l.ta;
             snprintf(line, sizeof(line),
-                     "tile L=%d M=%d NT=%d layout=%d inp=%d outp=%d lds=%d pipe=%d grid=%lld rad=%d,%d,%d,%d tiles=%d "
+                     "%s L=%d M=%d NT=%d layout=%d inp=%d outp=%d lds=%d pipe=%d grid=%lld rad=%d,%d,%d,%d tiles=%d "
                      "n_inner=%d tiles_inner=%d n_outer1=%d in=%s+%lld out=%s+%lld "
                      "in_strides=%lld,%lld,%lld,%lld out_strides=%lld,%lld,%lld,%lld tw=%d first=%d last=%d vin=%d vout=%d runs=%d\n",
-                     l.k->L, l.k->M, l.k->NT, l.k->layout, l.k->inp, l.k->outp, l.k->lds_bytes, l.k->persistent,
-                     (long long)l.grid, l.k->rad[0],
+                     l.k->long_row ? "long_row" : "tile", l.k->L, l.k->M, l.k->NT, l.k->layout, l.k->inp, l.k->outp,
+                     l.k->lds_bytes, l.k->persistent, (long long)l.grid, l.k->rad[0],
                      l.k->nrad > 1 ? l.k->rad[1] : 0, l.k->nrad > 2 ? l.k->rad[2] : 0,
                      l.k->nrad > 3 ? l.k->rad[3] : 0, a.n_tiles, a.n_inner, a.tiles_inner, a.n_outer1,
                      bn[l.in_buf], (long long)l.in_off, bn[l.out_buf], (long long)l.out_off,
@@ -1752,14 +1836,26 @@ int run_launches(const std::vector<Launch> &launches, int prec, int xcd_remap, c
                  const float *scale = nullptr, int64_t scale_div = 1, hipEvent_t stop = nullptr,
                  bool *stopped = nullptr);
 
-// Whether this call's buffers overlap in a way the plan's launch order can
-// corrupt (see gfft_plan_s::overlap_hazard).
-bool needs_stage(const gfft_plan_s *p, const void *in, const void *out)
+// The launches this call runs, and whether its buffers overlap in a way their
+// order can corrupt (see gfft_plan_s::overlap_hazard), so that the input has
+// to be staged.
+const std::vector<Launch> &route(const gfft_plan_s *p, const void *in, const void *out, bool *stage)
 {
-    if (!p->overlap_hazard) return false;
+    *stage = false;
+    if (!p->overlap_hazard) return p->launches;
     const uintptr_t i0 = (uintptr_t)in, o0 = (uintptr_t)out;
-    if (!(i0 < o0 + p->out_bytes && o0 < i0 + p->in_bytes)) return false;
-    return !(i0 == o0 && p->in_step == p->out_step && p->in_step2 == p->out_step2);
+    if (!(i0 < o0 + p->out_bytes && o0 < i0 + p->in_bytes)) return p->launches;
+    if (i0 == o0 && p->in_step == p->out_step && p->in_step2 == p->out_step2) return p->launches;
+    *stage = p->alt.empty() || p->alt_hazard;
+    return p->alt.empty() ? p->launches : p->alt;
+}
+
+// Whether a launch of the list works in the plan's shared workspace.
+bool uses_scratch(const std::vector<Launch> &launches)
+{
+    for (const Launch &l : launches)
+        if (l.reads(B_SCR) || l.writes(B_SCR)) return true;
+    return false;
 }
 
 int run(gfft_plan_s *p, const void *in, void *out, int direction, hipStream_t s,
@@ -1768,9 +1864,10 @@ int run(gfft_plan_s *p, const void *in, void *out, int direction, hipStream_t s,
     if (p->scratch_bytes && !p->scratch)
         return fail(GFFT_ERR_INVALID_ARG, "plan created with GFFT_FLAG_NO_WORKSPACE holds no workspace: "
                                           "run it with gfft_execute_noalloc");
-    const bool stage = needs_stage(p, in, out);
-    if (!p->scratch && !stage)  // no shared workspace: calls on any streams are independent
-        return run_launches(p->launches, p->prec, p->xcd_remap, in, out, p->scratch, direction, s, events, scale,
+    bool stage = false;
+    const std::vector<Launch> &launches = route(p, in, out, &stage);
+    if ((!p->scratch || !uses_scratch(launches)) && !stage)  // no shared workspace: calls on any streams are independent
+        return run_launches(launches, p->prec, p->xcd_remap, in, out, p->scratch, direction, s, events, scale,
                             p->scale_div);
     std::lock_guard<std::mutex> lk(p->order.mu);
     if (stage && !p->stage) {
@@ -1788,7 +1885,7 @@ int run(gfft_plan_s *p, const void *in, void *out, int direction, hipStream_t s,
         in = p->stage;
     }
     bool stopped = false;
-    int st = run_launches(p->launches, p->prec, p->xcd_remap, in, out, p->scratch, direction, s, events, scale,
+    int st = run_launches(launches, p->prec, p->xcd_remap, in, out, p->scratch, direction, s, events, scale,
                           p->scale_div, p->order.stop_event(s), &stopped);
     if (st) return st;
     if (stopped) p->order.mark(s);
@@ -2142,11 +2239,12 @@ int build_batch(gfft_batch_plan_s *p)
         // each length class takes the kernel choices a single plan of that
         // length would: the tuning table's entry, or the defaults
         b.opts = resolve_opts(prec, L, nullptr);
-        if (L <= maxrow) {
+        const int lv = L > maxrow ? b.long_row_variant(L, c.count) : -1;
+        if (L <= maxrow || lv >= 0) {
             // one transform per tile (job tables give each its own offsets): a
             // tuned single-pass kernel counts only when it holds one sequence
             const int v = b.opts.row_variant;
-            const int variant = v >= 0 && v < cnt && tab[v].M == 1 ? v : -1;
+            const int variant = lv >= 0 ? lv : v >= 0 && v < cnt && tab[v].M == 1 ? v : -1;
             if ((st = b.tile((int)L, PAT_ROW, PAT_ROW, 1, B_IN, 0, B_OUT, 0, 1, c.count, 1, 0, 0, 0, 1, 0, 0, 0, 1,
                              TW_NONE, 0, false, false, variant)))
                 return st;
@@ -2247,6 +2345,12 @@ std::vector<PlanOpts> tune_candidates(int prec, int64_t n)
             }
         return out;
     }
+    for (int i = 0; i < cnt; i++)  // one row in a workgroup's registers
+        if (tab[i].long_row && tab[i].L == n) {
+            PlanOpts o;
+            o.row_variant = i;
+            out.push_back(o);
+        }
     const int lg = ilog2(n), maxcol = max_len(prec, PAT_COL, PAT_COL), maxtr = max_len(prec, PAT_ROW, PAT_COL);
     for (int l1 = 1; l1 < lg; l1++) {
         const int64_t N1 = (int64_t)1 << l1, N2 = (int64_t)1 << (lg - l1);
@@ -2585,13 +2689,15 @@ int gfft_execute_noalloc(gfft_plan plan, const void *in, void *out, int directio
                     "this plan needs %zu bytes of workspace, more than the %lld bytes of the static workspace "
                     "(create it with GFFT_FLAG_NO_WORKSPACE to chunk its batch)",
                     plan->scratch_bytes, (long long)GFFT_NOALLOC_SCRATCH_BYTES);
-    if (needs_stage(plan, in, out))
+    bool stage = false;
+    const std::vector<Launch> &launches = route(plan, in, out, &stage);
+    if (stage)
         return fail(GFFT_ERR_UNSUPPORTED, "the buffers overlap other than exactly in place, which needs a staging "
                                           "copy this entry point cannot allocate");
     void *scr = nullptr;
     if (plan->scratch_bytes)
         if (int st = noalloc_scratch_ptr(plan->device, &scr)) return st;
-    return run_launches(plan->launches, plan->prec, plan->xcd_remap, in, out, scr, direction, (hipStream_t)stream);
+    return run_launches(launches, plan->prec, plan->xcd_remap, in, out, scr, direction, (hipStream_t)stream);
 }
 
 int gfft_execute_scaled(gfft_plan plan, const void *in, void *out, int direction, float *scales, int scale_mode,
@@ -2747,7 +2853,8 @@ int gfft_plan_profile(gfft_plan plan, const void *in, void *out, int direction, 
     if ((direction != GFFT_FORWARD && direction != GFFT_INVERSE) || !(plan->dir_mask & (1 << direction)))
         return fail(GFFT_ERR_INVALID_ARG, "direction %d is not one this plan runs", direction);
     if (int st = on_plan_device(plan->device)) return st;
-    const int n = (int)plan->launches.size();
+    bool stage = false;
+    const int n = (int)route(plan, in, out, &stage).size();
     *count = n;
     std::vector<hipEvent_t> ev(2 * n);
     for (auto &e : ev) HIP_TRY(hipEventCreate(&e));

@@ -1,0 +1,117 @@
+"""Tiles held in registers (genfft_amd/csrc/gfft_regtile.h).
+
+Parity with the long-double oracle at the library's bounds (rel-L2 2e-7*log2 N
+complex64, 1e-15*log2 N complex128) at the edges of the shapes: tiles with
+missing sequences, padded pitches, the smallest batch that takes a row past
+the LDS tiles, and overlapping buffers there.
+"""
+import numpy as np
+import pytest
+import torch
+
+import oracle_lib as O
+from genfft_amd import _capi as C
+from test_capi_cpu import desc, explain, field, tiles
+
+PREC = {"c64": (C.GFFT_F32, np.complex64, torch.complex64, O.tol_c64),
+        "c128": (C.GFFT_F64, np.complex128, torch.complex128, O.tol_c128)}
+
+
+def _rand(shape, dt, seed):
+    rng = np.random.default_rng(seed)
+    return (rng.uniform(-1, 1, shape) + 1j * rng.uniform(-1, 1, shape)).astype(dt)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("prec,n,batch,pin,pout", [
+    ("c64", 8192, 1, 0, 0), ("c64", 8192, 5, 3, 1), ("c64", 16384, 3, 0, 7), ("c64", 32768, 96, 0, 0),
+    ("c64", 32768, 97, 5, 3),
+    ("c128", 256, 1, 0, 0), ("c128", 256, 13, 1, 0), ("c128", 512, 7, 0, 3), ("c128", 1024, 3, 1, 1),
+    ("c128", 2048, 2, 0, 0), ("c128", 4096, 3, 3, 0), ("c128", 8192, 2, 0, 1), ("c128", 16384, 96, 0, 0),
+    ("c128", 16384, 97, 1, 5)])
+def test_rows_vs_oracle(gpu, prec, n, batch, pin, pout):
+    import genfft_amd as G
+    p, ndt, tdt, tol = PREC[prec]
+    x = _rand((batch, n + pin), ndt, n + batch)
+    tx = torch.from_numpy(x).to(gpu)
+    plan = G.Plan(C.GFFT_C2C, n, precision=p, batch=batch, in_dist=n + pin, out_dist=n + pout)
+    rows = sorted({0, 1, batch // 2, batch - 1} & set(range(batch)))
+    for inv in (False, True):
+        y = torch.full((batch, n + pout), 7 + 5j, dtype=tdt, device=gpu)
+        plan.execute(tx, y, inverse=inv)
+        h = y.cpu().numpy()
+        ref = O.fft_ld(np.ascontiguousarray(x[rows, :n]).astype(np.complex128), inv)
+        assert O.rel_l2_rows(h[rows, :n], ref).max() <= tol(n)
+        full = np.fft.ifft(x[:, :n].astype(np.complex128)) * n if inv else np.fft.fft(x[:, :n].astype(np.complex128))
+        assert O.rel_l2_rows(h[:, :n], full).max() <= tol(n)
+        if pout:
+            assert np.all(h[:-1, n:] == 7 + 5j)  # the gaps stay untouched
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("prec,n", [("c64", 32768), ("c128", 16384)])
+def test_long_rows_on_overlapping_buffers(gpu, prec, n):
+    """Exactly in place, and with the output shifted against the input by part
+    of a row and by whole rows, through both execute entry points."""
+    import genfft_amd as G
+    p, ndt, tdt, tol = PREC[prec]
+    batch = 97
+    x = _rand((batch, n), ndt, 3)
+    ref = np.fft.fft(x.astype(np.complex128))
+    plan = G.Plan(C.GFFT_C2C, n, precision=p, batch=batch)
+    for shift in (0, 2, n // 2, 3 * n):
+        buf = torch.zeros(batch * n + shift, dtype=tdt, device=gpu)
+        for at_in, at_out in ((0, shift), (shift, 0)):
+            src = buf[at_in:at_in + batch * n]
+            src.copy_(torch.from_numpy(x.reshape(-1)))
+            out = buf[at_out:at_out + batch * n]
+            plan.execute(src, out)
+            assert O.rel_l2_rows(out.cpu().numpy().reshape(batch, n), ref).max() <= tol(n)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("prec,lg", [("c64", (13, 14, 15)), ("c128", (12, 13, 14))])
+@pytest.mark.parametrize("count", [3, 96])
+def test_uneven_batches_of_long_rows(gpu, prec, lg, count):
+    """Job tables with odd offsets through the register-held rows."""
+    import genfft_amd as G
+    p, ndt, tdt, tol = PREC[prec]
+    sizes = [1 << (lg[i % 3] if count < 96 else lg[2] if i else lg[0]) for i in range(count + 1)]
+    offs = np.cumsum([1] + [s + 1 for s in sizes[:-1]])
+    inv = np.arange(len(sizes)) % 2 == 1
+    x = _rand(int(offs[-1] + sizes[-1]), ndt, 9)
+    tx = torch.from_numpy(x).to(gpu)
+    y = torch.zeros_like(tx)
+    b = G.UnevenBatch(sizes, offs, offs, inv, tdt)
+    for mode in ("graph", "eager"):
+        y.zero_()
+        b.execute(tx, y, mode=mode)
+        h = y.cpu().numpy()
+        for o, s, i in zip(offs, sizes, inv):
+            v = x[o:o + s].astype(np.complex128)
+            ref = np.fft.ifft(v) * s if i else np.fft.fft(v)
+            assert O.rel_l2(h[o:o + s], ref) <= tol(s)
+
+
+def test_long_rows_route():
+    """From 96 rows on a row past the LDS tiles is one launch; smaller batches,
+    lengths beyond and a tuned split keep the four-step.  The plan's workspace
+    stays the four-step's, which calls on overlapping buffers run in."""
+    for prec, n in ((C.GFFT_F32, 1 << 15), (C.GFFT_F64, 1 << 14)):
+        for batch, one in ((95, False), (96, True), (400, True)):
+            st, text = explain(desc(prec=prec, n=n, batch=batch))
+            assert st == C.GFFT_OK
+            assert text.count("long_row ") == (1 if one else 0)
+            assert ("on overlapping buffers" in text) == one
+            assert f"scratch_bytes={batch * n * (8 << prec)}\n" in text
+        st, text = explain(desc(prec=prec, n=2 * n, batch=400))
+        assert st == C.GFFT_OK and "long_row" not in text
+
+
+def test_layouts_past_32_bit_offsets_keep_the_lds_tiles():
+    """A tile of several rows whose last row lies 2^31 bytes or more from its
+    first is not register-held (its accesses are 32-bit offsets)."""
+    for dist, reg in ((256, True), (1 << 24, True), (1 << 25, False)):
+        st, text = explain(desc(prec=C.GFFT_F64, n=256, batch=8, ind=dist, outd=dist))
+        assert st == C.GFFT_OK
+        assert (field(tiles(text)[0], "rad") == "8,4,8,0") == reg
