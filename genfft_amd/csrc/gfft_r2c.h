@@ -110,9 +110,19 @@ struct RealRowsArgs {
 
 enum RealRowsMode { RR_R2C = 0, RR_C2R = 1 };
 
-// Shape for n/2 = L (the row-tile shape of that length; nullptr: none).
-const KernelEntry *real_rows_entry(int prec, int L);
-hipError_t launch_real_rows(int prec, int L, int mode, const RealRowsArgs &a, int64_t grid, hipStream_t s,
+// One mode of one row length: shape and kernel.
+struct RowsEntry {
+    KernelEntry entry;
+    int mode;
+    int64_t most;  // input bytes up to which this shape is taken (0: any)
+    void (*fn)(RealRowsArgs);
+};
+
+// The kernel of n/2 = L for `bytes` of input (nullptr: none).  `lds`: only
+// tiles kept in LDS; `long_row`: the register-held tile of a row one length
+// past the c2c row tiles.
+const RowsEntry *real_rows_entry(int prec, int L, int mode, int64_t bytes, bool lds = false, bool long_row = false);
+hipError_t launch_real_rows(const RowsEntry *e, const RealRowsArgs &a, int64_t grid, hipStream_t s,
                             hipEvent_t stop = nullptr);
 
 }  // namespace gfft

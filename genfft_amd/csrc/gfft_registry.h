@@ -29,6 +29,7 @@ struct KernelEntry {
     int gen_tw;      // 1: the last pass builds its twiddles from TileArgs::gen_lo / gen_hi (W_L)
     int wave;        // 1: one wavefront per row, lanes exchanged without LDS (wave_rows1024_kernel)
     int reg;         // 1: tile held in registers (reg_tile_kernel); its own pass twiddle table layout
+    int cached;      // 1: row tile the planner takes for batches within the Infinity Cache
     int long_row;    // 1: a row longer than the LDS row tiles (the planner takes it by its own rule)
     int wide;        // 1: double-width row tile the planner takes for batches past the Infinity Cache
 };
@@ -171,6 +172,25 @@ constexpr KernelEntry make_reg_wide()
     KernelEntry e = reg_shape<T, L, M, NT, PAT_ROW, PAT_ROW, HINT_LD | HINT_ST, RS...>();
     e.tune_only = 1;
     e.wide = 1;
+    return e;
+}
+
+// A narrow row tile for batches that would leave CUs idle (the planner's
+// narrow_row_variant).
+template <typename T, int L, int M, int NT, int... RS>
+constexpr KernelEntry make_reg_narrow()
+{
+    KernelEntry e = make_reg_entry<T, L, M, NT, PAT_ROW, PAT_ROW, RS...>();
+    e.tune_only = 1;
+    return e;
+}
+
+// A row tile for batches that stay within the Infinity Cache.
+template <typename T, int L, int M, int NT, int... RS>
+constexpr KernelEntry make_reg_cached()
+{
+    KernelEntry e = make_reg_narrow<T, L, M, NT, RS...>();
+    e.cached = 1;
     return e;
 }
 

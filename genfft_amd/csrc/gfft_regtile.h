@@ -52,24 +52,32 @@ struct PlaneGeom {
 // the sequence first (MAP_J), across the sequences first (MAP_S), or across
 // pairs of adjacent sequences (MAP_P: butterflies 2q and 2q + 1 of a thread
 // are the same j of sequences s and s + 1, so their HBM accesses join into
-// 16 bytes and they share their twiddles).
-enum : int { MAP_J = 0, MAP_S = 1, MAP_P = 2 };
+// 16 bytes and they share their twiddles), or along the sequence in mirror
+// pairs (MAP_M, two butterflies per thread: thread t of a sequence has j = t
+// and L/R - t, whose elements are k and L - k; t = 0 has 0 and L/2R, which
+// mirror themselves).
+enum : int { MAP_J = 0, MAP_S = 1, MAP_P = 2, MAP_M = 3 };
 template <int L, int M, int NT, int MAP, int R>
 struct Bfly {
     static constexpr int LR = L / R;
     static constexpr int W = MAP == MAP_P ? 2 : 1;  // butterflies that share j
     static constexpr int N = M * L / NT / R / W;    // groups of them per thread
     static_assert(N >= 1 && N * W * R * NT == M * L, "whole butterflies per thread");
+    static_assert(MAP != MAP_M || N == 2, "mirror pairs");
     static __device__ __forceinline__ int s(int tid, int q)
     {
         const int b = tid + q * NT;
         if constexpr (M == 1) return 0;
+        else if constexpr (MAP == MAP_M) return tid / (LR / 2);
         else return MAP == MAP_J ? b / LR : MAP == MAP_S ? b % M : b % (M / 2) * 2;
     }
     static __device__ __forceinline__ int j(int tid, int q)
     {
         const int b = tid + q * NT;
-        if constexpr (M == 1) return b;
+        if constexpr (MAP == MAP_M) {
+            const int t = tid % (LR / 2);
+            return q == 0 ? t : t ? LR - t : LR / 2;
+        } else if constexpr (M == 1) return b;
         else return MAP == MAP_J ? b % LR : MAP == MAP_S ? b / M : b / (M / 2);
     }
 };
@@ -175,11 +183,11 @@ struct TwWalk {
     }
 };
 
-// The passes from (NS, R) on: mapping MP for this one, MPL for the later
-// ones.  complex64 builds a butterfly's twiddles as FP64 powers of its base,
+// The passes from (NS, R) on: mapping MP for this one, MPL for the last one
+// and MPM for those between.  complex64 builds a butterfly's twiddles as FP64 powers of its base,
 // rounded once; complex128 reads them from `tw`, W_{NS*R}^(r*m) at
 // [(r - 1) * NS + m] for each pass with NS > 1.
-template <typename T, int L, int M, int NT, class G, int MP, int MPL, int NS, int R, int... RS>
+template <typename T, int L, int M, int NT, class G, int MP, int MPM, int MPL, int NS, int R, int... RS>
 __device__ __forceinline__ void reg_passes(T *plane, cx<T> (&v)[M * L / NT], const cx<T> *__restrict__ tw, int tid,
                                            const TileArgs &a, const RegTw<T, L, M, NT, NS, R, MP> &w)
 {
@@ -210,10 +218,11 @@ __device__ __forceinline__ void reg_passes(T *plane, cx<T> (&v)[M * L / NT], con
     }
     if constexpr (sizeof...(RS) > 0) {
         constexpr int R2 = first_radix<RS...>();
-        RegTw<T, L, M, NT, NS * R, R2, MPL> w2;
+        constexpr int MP2 = sizeof...(RS) == 1 ? MPL : MPM;
+        RegTw<T, L, M, NT, NS * R, R2, MP2> w2;
         w2.load(a, tid);
-        reg_exchange<T, L, M, NT, G, NS, R, MP, R2, MPL, NS == 1>(plane, v, tid);
-        reg_passes<T, L, M, NT, G, MPL, MPL, NS * R, RS...>(plane, v, tw + (NS > 1 ? NS * (R - 1) : 0), tid, a, w2);
+        reg_exchange<T, L, M, NT, G, NS, R, MP, R2, MP2, NS == 1>(plane, v, tid);
+        reg_passes<T, L, M, NT, G, MP2, MPM, MPL, NS * R, RS...>(plane, v, tw + (NS > 1 ? NS * (R - 1) : 0), tid, a, w2);
     }
 }
 
@@ -326,7 +335,7 @@ __global__ void __launch_bounds__(NT, 4) reg_tile_kernel(TileArgs a)
             for (int k = 0; k < E; k++) v[k] = swap_ri(v[k]);
         }
     }
-    reg_passes<T, L, M, NT, G, MP, MPL, 1, RS...>(plane, v, reinterpret_cast<const cx<T> *>(a.pass_tw), tid, a,
+    reg_passes<T, L, M, NT, G, MP, MPL, MPL, 1, RS...>(plane, v, reinterpret_cast<const cx<T> *>(a.pass_tw), tid, a,
                                                   RegTw<T, L, M, NT, 1, R1, MP>{});
     {
         using A = Bfly<L, M, NT, MPL, RL>;

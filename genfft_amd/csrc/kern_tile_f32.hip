@@ -1,15 +1,17 @@
 // kern_tile_f32.hip -- complex64 tile-kernel shapes.
 //
 // Rows (PAT_ROW -> PAT_ROW, sequence-major LDS): batched 1D transforms and
-// the 2D row pass; a tile holds 4096 complex (32 KB) up to L = 4096.
+// the 2D row pass; a tile holds 4096 complex (32 KB)
+// up to L = 2048.
 // Columns (PAT_COL -> PAT_COL, element-major LDS): the first pass of a
 // four-step transform and the 2D column pass; M adjacent columns give
 // >= 64-byte contiguous row segments.
 // Transposing rows (PAT_ROW -> PAT_COL): the second four-step pass, writing
 // element k of row k1 to k1 + N1*k, M rows wide.
 // Every default LDS shape keeps 16 elements per thread, so radix-16 butterflies
-// live entirely in registers (the radix-32 alternatives hold 32).  Rows from
-// 8192 points on are held in registers (gfft_regtile.h).
+// live entirely in registers (the radix-32 alternatives hold 32).  Rows
+// within the Infinity Cache and from 4096 points on are held in registers
+// (gfft_regtile.h).
 #include "gfft_registry.h"
 
 namespace gfft {
@@ -25,10 +27,10 @@ const KernelEntry kTable[] = {
     make_entry<T, 16, 256, 256, S_, R_, R_, 16>(),
     make_entry<T, 32, 128, 256, S_, R_, R_, 8, 4>(),
     make_entry<T, 64, 64, 256, S_, R_, R_, 8, 8>(),
-    make_entry<T, 128, 32, 256, S_, R_, R_, 16, 8>(),
+    make_variant<T, 128, 32, 256, S_, R_, R_, 16, 8>(),
     make_entry<T, 256, 16, 256, S_, R_, R_, 16, 16>(),
     make_entry<T, 512, 8, 256, S_, R_, R_, 8, 8, 8>(),
-    make_entry<T, 1024, 4, 256, S_, R_, R_, 16, 16, 4>(),
+    make_variant<T, 1024, 4, 256, S_, R_, R_, 16, 16, 4>(),
     make_entry<T, 2048, 2, 256, S_, R_, R_, 16, 16, 8>(),
     make_variant<T, 4096, 1, 256, S_, R_, R_, 16, 16, 16>(),
     make_variant<T, 8192, 1, 512, S_, R_, R_, 16, 16, 8, 4>(),
@@ -92,22 +94,39 @@ const KernelEntry kTable[] = {
     make_variant<T, 2048, 2, 256, S_, R_, R_, 8, 16, 16>(),
     make_wide_variant<T, 2048, 4, 512, S_, R_, R_, 16, 16, 8>(),
     make_variant<T, 4096, 2, 512, S_, R_, R_, 16, 16, 16>(),
-    // 512 threads of radix 8: 4096-point rows 5.5 -> 5.0 us (one), 12.9 -> 12.9
-    // (1024), 0.388 -> 0.384 ms (1 GiB) against 16*16*16 with 256 threads
-    make_entry<T, 4096, 1, 512, S_, R_, R_, 8, 8, 8, 8>(),
+    make_variant<T, 4096, 1, 512, S_, R_, R_, 8, 8, 8, 8>(),
     make_variant<T, 8192, 1, 512, S_, R_, R_, 16, 16, 16, 2>(),
     make_variant<T, 16384, 1, 1024, S_, R_, R_, 16, 16, 8, 8>(),
     // one wavefront per 1024-point row, lanes exchanged by DPP / permlane swaps
     make_wave_entry<256>(),
-    // --- rows held in registers (LDS plane 34 / 69 / 135 KB: four / two / one
-    // workgroup per CU).  MI355X, 1 GiB batches, streaming loads: 8192 points
-    // 0.427 -> 0.364 ms, 16384 0.435 -> 0.360-0.387 ms, 32768 0.72 -> 0.46 ms
-    // (four-step); 256 MiB batches, plain loads: 0.087 -> 0.067 ms (8192) and
-    // 0.104 -> 0.079 ms (16384); from one row up to 16 the LDS tiles' time.
-    // The streaming 16384-point tile runs 16*4*16*16 with 1024 threads, the
-    // order of the LDS tile before it: 0.387 ms (32*32*16 with 512: 0.375) ---
-    make_reg_entry<T, 8192, 1, 256, R_, R_, 32, 16, 16>(),
-    make_reg_wide<T, 8192, 1, 256, 32, 16, 16>(),
+    // --- rows held in registers.  Short ones: few elements per thread and no
+    // load, store or pass sweep through LDS, so a small batch's one round of
+    // tiles ends sooner and within the Infinity Cache the loads and stores of
+    // more workgroups overlap.  Past it the LDS tiles' 16-byte accesses win up
+    // to 2048 points.  MI355X, us per call, one row / 4 MiB / 64 MiB, LDS tile
+    // -> register tile: 64 points 4.9 -> 3.5 / 5.4 -> 4.1 (8192 rows; LDS
+    // beyond), 256: 4.9 -> 4.2 / 5.5 -> 4.8 / 25.8 -> 24.1, 512: 5.3 -> 4.3 /
+    // 5.8 -> 4.9 / 25.9 -> 24.1, 2048: 6.1 -> 4.7 / 6.4 -> 5.4 / 27.1 -> 24.1,
+    // 4096: 5.9 -> 5.5 / 6.6 -> 6.1 / 28.5 -> 25.0.  Long ones (LDS plane 34 /
+    // 69 / 135 KB: four / two / one workgroup per CU), 1 GiB batches with
+    // streaming loads: 4096 points 0.392 -> 0.369 ms, 8192 0.427 -> 0.352,
+    // 16384 0.435 -> 0.378, 32768 0.72 -> 0.46 (four-step); 256 MiB batches:
+    // 8192 0.087 -> 0.067, 16384 0.104 -> 0.080.  The streaming 16384-point
+    // tile runs 16*4*16*16 with 1024 threads, the order of the LDS tile before
+    // it: 0.387 ms (32*32*16 with 512: 0.375) ---
+    make_reg_narrow<T, 16, 32, 64, 4, 4>(),
+    make_reg_narrow<T, 32, 16, 64, 8, 4>(),
+    make_reg_narrow<T, 64, 8, 64, 8, 8>(),
+    make_reg_entry<T, 128, 16, 256, R_, R_, 8, 2, 8>(),
+    make_reg_cached<T, 256, 8, 256, 8, 4, 8>(),
+    make_reg_cached<T, 512, 4, 256, 8, 8, 8>(),
+    make_reg_narrow<T, 1024, 2, 128, 16, 4, 16>(),
+    make_reg_entry<T, 1024, 4, 256, R_, R_, 16, 8, 8>(),
+    make_reg_cached<T, 2048, 1, 128, 16, 8, 16>(),
+    make_reg_entry<T, 4096, 1, 256, R_, R_, 16, 16, 16>(),
+    make_reg_wide<T, 4096, 1, 256, 16, 16, 16>(),
+    make_reg_entry<T, 8192, 1, 512, R_, R_, 16, 8, 8, 8>(),
+    make_reg_wide<T, 8192, 1, 512, 8, 16, 8, 8>(),
     make_reg_entry<T, 16384, 1, 512, R_, R_, 32, 32, 16>(),
     make_reg_wide<T, 16384, 1, 1024, 16, 4, 16, 16>(),
     make_reg_long<T, 32768, 1024, HINT_ST, 32, 32, 32>(),

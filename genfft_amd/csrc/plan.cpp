@@ -341,8 +341,8 @@ int narrow_row_variant(int prec, int L, int64_t batch, int num_cus)
     const KernelEntry *tab = tile_table(prec, 0, &cnt);
     for (int i = 0; i < cnt; i++) {
         const KernelEntry &e = tab[i];
-        if (e.L != L || e.inp != PAT_ROW || e.outp != PAT_ROW || e.wave || e.wide || e.reg || e.persistent) continue;
-        if (e.M < d->M && (best < 0 || e.M < tab[best].M)) best = i;
+        if (e.L != L || e.inp != PAT_ROW || e.outp != PAT_ROW || e.wave || e.wide || e.persistent || e.long_row) continue;
+        if (e.M < d->M && (best < 0 || e.M < tab[best].M || (e.M == tab[best].M && e.reg > tab[best].reg))) best = i;
     }
     return best;
 }
@@ -507,6 +507,7 @@ struct Launch {
     RealRowsArgs rr{};
     RepackArgs rp{};
     int rr_mode = RR_R2C;
+    const RowsEntry *rre = nullptr;
     int in_buf = B_IN, out_buf = B_OUT;
     int64_t in_off = 0, out_off = 0;  // bytes
     bool vin_ok = false, vout_ok = false;
@@ -643,6 +644,9 @@ bool tile_offsets_fit(int pat, int64_t L, int64_t M, int64_t inner, int64_t elem
 // Batches of at least this many bytes a side stream through HBM: row tiles
 // with the `wide` flag.
 constexpr int64_t kStreamBytes = (int64_t)512 << 20;
+// Row batches of at most this many bytes a side take the `cached` row tiles
+// (c64 2048 points on MI355X: 64 MiB 59.8 -> 55.8 us, 128 MiB 101.3 -> 101.4).
+constexpr int64_t kCachedBytes = (int64_t)128 << 20;
 // Rows from which a register-held tile per row beats the four-step (MI355X, us
 // per call at 64 / 96 / 128 / 256 rows: c64 32768 points 18.1 / 18.3 / 19.5 /
 // 32 against 16.0 / 23.3 / 28 / 54, c128 16384 points 17.4 / 18.2 / 20.9 / 33
@@ -771,6 +775,16 @@ struct Builder {
         return GFFT_OK;
     }
 
+    // Row tile for `rows` rows of length n within the Infinity Cache: the one
+    // registered for that (KernelEntry::cached), else the narrowest while the
+    // default tiles would leave CUs idle; -1: the default.
+    int cached_row_variant(int n, int64_t rows) const
+    {
+        if (store) return -1;
+        const int v = n * rows * (int64_t)csize <= kCachedBytes ? row_variant_of(prec, n, &KernelEntry::cached) : -1;
+        return v >= 0 ? v : narrow_row_variant(prec, n, rows, p->num_cus);
+    }
+
     // Register-held row tile for `batch` rows of length n, one past the LDS
     // row tiles, or -1 (four-step).  One workgroup owns a row, so below half
     // the CUs the four-step's shorter tiles spread a small batch wider.
@@ -826,7 +840,7 @@ struct Builder {
                 if (batch == 1) variant = row_variant_of(prec, (int)n, &KernelEntry::wave);
                 else if (n * batch * (int64_t)csize >= kStreamBytes)
                     variant = row_variant_of(prec, (int)n, &KernelEntry::wide);
-                else variant = narrow_row_variant(prec, (int)n, batch, p->num_cus);
+                if (variant < 0) variant = cached_row_variant((int)n, batch);
             }
             return tile((int)n, PAT_ROW, PAT_ROW, 0, in_buf, in_off, out_buf, out_off, batch, 1, 1, 0, 0,
                         in_dist, 1, 0, 0, out_dist, 1, TW_NONE, 0, first, last, variant);
@@ -1068,7 +1082,15 @@ struct Builder {
     // single-pass row length from 2 on): unpack or pack fused in.
     bool rows_fusable(int64_t n) const
     {
-        return !store && opts.r2c_fuse && is_pow2(n) && n / 2 >= 2 && real_rows_entry(prec, (int)(n / 2));
+        return !store && opts.r2c_fuse && is_pow2(n) && n / 2 >= 2 && real_rows_entry(prec, (int)(n / 2), RR_R2C, 0);
+    }
+
+    // Whether `rows` real transforms of length n, n/2 one past the LDS row
+    // tiles, run in one pass on register-held rows.
+    bool long_real_rows(int64_t n, int64_t rows) const
+    {
+        return !store && opts.r2c_fuse && !no_long_rows && rows >= kLongRows && is_pow2(n) && n <= INT32_MAX &&
+               real_rows_entry(prec, (int)(n / 2), RR_R2C, 0, false, true);
     }
 
     // `rows` real transforms of length n in one launch: mode RR_R2C reads
@@ -1076,12 +1098,20 @@ struct Builder {
     // apart; n/2 + 1 of them with `half`, else n); RR_C2R reads n/2 + 1 bins
     // per row and writes n reals (out_row apart, complex units).
     int real_rows(int mode, int64_t n, int64_t rows, int in_buf, int64_t in_off_el, int64_t in_row, int out_buf,
-                  int64_t out_off_el, int64_t out_row, bool half)
+                  int64_t out_off_el, int64_t out_row, bool half, bool long_row = false)
     {
-        const KernelEntry *fe = real_rows_entry(prec, (int)(n / 2));
+        const RowsEntry *re = real_rows_entry(prec, (int)(n / 2), mode, rows * (n / 2) * (int64_t)csize, false, long_row);
+        // 32-bit byte offsets within a tile; a full spectrum spans n bins
+        if (re && re->entry.reg && !(tile_offsets_fit(PAT_ROW, n / 2 + 1, re->entry.M, in_row, 1, csize) &&
+                                     tile_offsets_fit(PAT_ROW, n, re->entry.M, out_row, 1, csize)))
+            re = real_rows_entry(prec, (int)(n / 2), mode, 0, true);
+        if (!re) return fail(GFFT_ERR_UNSUPPORTED, "no real-row kernel for n=%lld", (long long)n);
+        if (long_row) long_rows = true;
+        const KernelEntry *fe = &re->entry;
         Launch l;
         l.type = LT_RROWS;
         l.k = fe;
+        l.rre = re;
         l.rr_mode = mode;
         TileArgs &a = l.rr.t;
         const int64_t tiles = (rows + fe->M - 1) / fe->M;
@@ -1100,6 +1130,12 @@ struct Builder {
         int st;
         if ((st = get_pass_twiddles(p->device, *fe, &a.pass_tw, dry))) return st;
         if ((st = get_two_level(p->device, n, &l.rr.tw, dry))) return st;
+        if (fe->gen_tw) {
+            TwTable g;
+            if ((st = get_two_level(p->device, fe->L, &g, dry))) return st;
+            a.gen_lo = g.lo;
+            a.gen_hi = g.hi;
+        }
         auto even = [](int64_t v) { return (v & 1) == 0; };
         if (prec == 0) {
             l.vin_ok = mode == RR_R2C && even(in_row) && even(in_off_el) &&
@@ -1233,6 +1269,10 @@ int build_plan(gfft_plan_s *p, bool dry, const PlanOpts *forced = nullptr, bool 
             st = b.real_rows(RR_R2C, n, batch, B_IN, 0, id / 2, B_OUT, 0, od, half);
             break;
         }
+        if (b.long_real_rows(n, batch)) {
+            st = b.real_rows(RR_R2C, n, batch, B_IN, 0, id / 2, B_OUT, 0, od, half, true);
+            break;
+        }
         // The fused path needs scratch for the whole batch.  The separate
         // unpack with an odd output distance needs the same; with an even
         // one it chunks the transform through at most GFFT_CHUNK_BYTES, so a
@@ -1288,6 +1328,10 @@ int build_plan(gfft_plan_s *p, bool dry, const PlanOpts *forced = nullptr, bool 
         }
         if (b.rows_fusable(n)) {
             st = b.real_rows(RR_C2R, n, batch, B_IN, 0, id, B_OUT, 0, od / 2, false);
+            break;
+        }
+        if (b.long_real_rows(n, batch)) {
+            st = b.real_rows(RR_C2R, n, batch, B_IN, 0, id, B_OUT, 0, od / 2, false, true);
             break;
         }
         if (b.c2r_fusable(n) && b.opts.r2c_fuse) {
@@ -1367,7 +1411,7 @@ int build_plan(gfft_plan_s *p, bool dry, const PlanOpts *forced = nullptr, bool 
         }
         // rows: H rows of batch matrices (two outer levels)
         st = b.tile((int)W, PAT_ROW, PAT_ROW, 0, B_IN, 0, B_OUT, 0, H, batch, 1, 0, id, ip, 1, 0, od, op, 1,
-                    TW_NONE, 0, true, H == 1);
+                    TW_NONE, 0, true, H == 1, b.cached_row_variant((int)W, H * batch));
         if (!st && H > 1) st = b.columns(H, W, batch, B_OUT, op, od, B_OUT, op, od, false, true);
         break;
     }
@@ -1982,7 +2026,7 @@ int run_launches(const std::vector<Launch> &launches, int prec, int xcd_remap, c
             a.t.vec_in = l.vin_ok && (((uintptr_t)ip & 15) == 0);
             a.t.vec_out = l.vout_ok && (((uintptr_t)op & 15) == 0);
             a.t.xcd_remap = p->xcd_remap;
-            HIP_TRY(launch_real_rows(p->prec, l.k->L, l.rr_mode, a, l.grid, s, tail));
+            HIP_TRY(launch_real_rows(l.rre, a, l.grid, s, tail));
             if (tail && stopped) *stopped = true;
             break;
         }

@@ -24,7 +24,9 @@ def _rand(shape, dt, seed):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("prec,n,batch,pin,pout", [
-    ("c64", 8192, 1, 0, 0), ("c64", 8192, 5, 3, 1), ("c64", 16384, 3, 0, 7), ("c64", 32768, 96, 0, 0),
+    ("c64", 16, 33, 1, 0), ("c64", 32, 17, 0, 3), ("c64", 64, 9, 1, 1), ("c64", 128, 17, 0, 0), ("c64", 256, 9, 3, 0),
+    ("c64", 512, 5, 0, 1), ("c64", 1024, 3, 0, 0), ("c64", 1024, 1025, 1, 0), ("c64", 2048, 3, 5, 0),
+    ("c64", 4096, 2, 0, 1), ("c64", 8192, 1, 0, 0), ("c64", 8192, 5, 3, 1), ("c64", 16384, 3, 0, 7), ("c64", 32768, 96, 0, 0),
     ("c64", 32768, 97, 5, 3),
     ("c128", 256, 1, 0, 0), ("c128", 256, 13, 1, 0), ("c128", 512, 7, 0, 3), ("c128", 1024, 3, 1, 1),
     ("c128", 2048, 2, 0, 0), ("c128", 4096, 3, 3, 0), ("c128", 8192, 2, 0, 1), ("c128", 16384, 96, 0, 0),
@@ -115,3 +117,59 @@ def test_layouts_past_32_bit_offsets_keep_the_lds_tiles():
         st, text = explain(desc(prec=C.GFFT_F64, n=256, batch=8, ind=dist, outd=dist))
         assert st == C.GFFT_OK
         assert (field(tiles(text)[0], "rad") == "8,4,8,0") == reg
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("prec,n,batch,pin,pout", [
+    ("c64", 128, 9, 0, 1), ("c64", 256, 5, 2, 0), ("c64", 512, 3, 2, 2), ("c64", 512, 1, 0, 0), ("c64", 512, 8193, 0, 0), ("c64", 1024, 9, 0, 2), ("c64", 2048, 5, 0, 0), ("c64", 4096, 3, 2, 4),
+    ("c64", 8192, 2, 0, 0), ("c64", 16384, 3, 4, 2), ("c64", 32768, 2, 0, 0), ("c64", 65536, 96, 0, 0),
+    ("c64", 65536, 97, 2, 4), ("c128", 256, 5, 0, 1), ("c128", 512, 3, 2, 0), ("c128", 1024, 2, 0, 0),
+    ("c128", 2048, 3, 0, 2), ("c128", 4096, 3, 0, 0), ("c128", 8192, 2, 2, 0),
+    ("c128", 16384, 2, 0, 2), ("c128", 32768, 96, 0, 0), ("c128", 32768, 97, 2, 2)])
+def test_real_rows_vs_float64(gpu, prec, n, batch, pin, pout):
+    """Half and full spectra and the way back, dense and padded (pin: reals,
+    pout: bins), against numpy's float64 transform at the complex bounds."""
+    import genfft_amd as G
+    p, ndt, tdt, tol = PREC[prec]
+    rdt = np.float32 if prec == "c64" else np.float64
+    rng = np.random.default_rng(n)
+    x = rng.uniform(-1, 1, (batch, n + pin)).astype(rdt)
+    tx = torch.from_numpy(x).to(gpu)
+    ref = np.fft.fft(x[:, :n].astype(np.float64))
+    for half in (True, False):
+        bins = n // 2 + 1 if half else n
+        y = torch.full((batch, bins + pout), 7 + 5j, dtype=tdt, device=gpu)
+        G.Plan(C.GFFT_R2C, n, precision=p, batch=batch, in_dist=n + pin, out_dist=bins + pout, half=half).execute(tx, y)
+        h = y.cpu().numpy()
+        assert O.rel_l2_rows(h[:, :bins], ref[:, :bins]).max() <= tol(n)
+        if pout:
+            assert np.all(h[:-1, bins:] == 7 + 5j)
+    X = ref[:, :n // 2 + 1].astype(ndt)
+    X[:, 0] += 3j  # ignored, as in any c2r
+    X[:, -1] -= 2j
+    z = torch.full((batch, n + pin), 9, dtype=torch.float32 if prec == "c64" else torch.float64, device=gpu)
+    G.Plan(C.GFFT_C2R, n, precision=p, batch=batch, out_dist=n + pin).execute(torch.from_numpy(X).to(gpu), z, inverse=True)
+    h = z.cpu().numpy()
+    assert O.rel_l2_rows(h[:, :n] / n, x[:, :n]).max() <= 2 * tol(n)
+    if pin:
+        assert np.all(h[:-1, n:] == 9)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("prec,n", [("c64", 65536), ("c128", 32768)])
+def test_long_real_rows_in_place(gpu, prec, n):
+    """Dense half spectra over their own reals: bins of one row lie where the
+    next row's reals are, so the call runs the plan's two-launch form."""
+    import genfft_amd as G
+    p, ndt, tdt, tol = PREC[prec]
+    rdt = torch.float32 if prec == "c64" else torch.float64
+    batch, bins = 96, n // 2 + 1
+    x = np.random.default_rng(1).uniform(-1, 1, (batch, n)).astype(np.float32 if prec == "c64" else np.float64)
+    buf = torch.zeros(batch * bins, dtype=tdt, device=gpu)
+    reals = torch.view_as_real(buf).reshape(-1)[:batch * n]
+    reals.copy_(torch.from_numpy(x.reshape(-1)))
+    G.Plan(C.GFFT_R2C, n, precision=p, batch=batch, half=True).execute(reals, buf)
+    h = buf.cpu().numpy().reshape(batch, bins)
+    assert O.rel_l2_rows(h, np.fft.rfft(x.astype(np.float64))).max() <= tol(n)
+    G.Plan(C.GFFT_C2R, n, precision=p, batch=batch).execute(buf, reals, inverse=True)
+    assert O.rel_l2_rows(reals.cpu().numpy().reshape(batch, n) / n, x).max() <= 2 * tol(n)
