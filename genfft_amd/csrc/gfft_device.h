@@ -229,6 +229,11 @@ struct TileArgs {
     // scale[] of that transform.  Null: no scaling.
     const float *scale;
     int64_t scale_div, scale_off;
+    // Automatic scale (kernels that hold a whole transform, reg_rows_kernel_h):
+    // the kernel computes the scale of transform s (scale_from_max with gain
+    // and limit), applies it and writes it to auto_scale[s].  Null: off.
+    float *auto_scale;
+    float gain, limit;
 };
 
 // FP64 twiddle W_Ntw^m from the two-level table.

@@ -132,8 +132,8 @@ constexpr KernelEntry make_pipe_variant()
     return e;
 }
 
-// A tile held in registers (reg_tile_kernel), with its stores streamed.
-template <typename T, int L, int M, int NT, int INP, int OUTP, int HINT, int... RS>
+// Shape of a tile held in registers, without its kernel.
+template <typename T, int L, int M, int NT, int INP, int OUTP, int... RS>
 constexpr KernelEntry reg_shape()
 {
     static_assert(((RS * ...) == L), "radices must multiply to L");
@@ -154,14 +154,22 @@ constexpr KernelEntry reg_shape()
     e.lds_bytes = (int)(G::ELEMS * sizeof(T));
     e.gen_tw = sizeof(T) == 4;
     e.reg = 1;
+    return e;
+}
+
+template <typename T, int L, int M, int NT, int INP, int OUTP, int HINT, int... RS>
+constexpr KernelEntry reg_entry()
+{
+    KernelEntry e = reg_shape<T, L, M, NT, INP, OUTP, RS...>();
     e.fn = &reg_tile_kernel<T, L, M, NT, INP, OUTP, HINT, RS...>;
     return e;
 }
 
+// reg_tile_kernel with its stores streamed.
 template <typename T, int L, int M, int NT, int INP, int OUTP, int... RS>
 constexpr KernelEntry make_reg_entry()
 {
-    return reg_shape<T, L, M, NT, INP, OUTP, HINT_ST, RS...>();
+    return reg_entry<T, L, M, NT, INP, OUTP, HINT_ST, RS...>();
 }
 
 // The row tile with streaming loads as well, which the planner takes for
@@ -169,7 +177,7 @@ constexpr KernelEntry make_reg_entry()
 template <typename T, int L, int M, int NT, int... RS>
 constexpr KernelEntry make_reg_wide()
 {
-    KernelEntry e = reg_shape<T, L, M, NT, PAT_ROW, PAT_ROW, HINT_LD | HINT_ST, RS...>();
+    KernelEntry e = reg_entry<T, L, M, NT, PAT_ROW, PAT_ROW, HINT_LD | HINT_ST, RS...>();
     e.tune_only = 1;
     e.wide = 1;
     return e;
@@ -198,7 +206,7 @@ constexpr KernelEntry make_reg_cached()
 template <typename T, int L, int NT, int HINT, int... RS>
 constexpr KernelEntry make_reg_long()
 {
-    KernelEntry e = reg_shape<T, L, 1, NT, PAT_ROW, PAT_ROW, HINT, RS...>();
+    KernelEntry e = reg_entry<T, L, 1, NT, PAT_ROW, PAT_ROW, HINT, RS...>();
     e.tune_only = 1;
     e.long_row = 1;
     e.wide = (HINT & HINT_LD) ? 1 : 0;
@@ -213,6 +221,36 @@ constexpr KernelEntry make_entry_h()
     e.lds_bytes += M * (int)sizeof(float);
     e.store = std::is_same<S, st_f16>::value ? 1 : 2;
     e.fn = &tile_fft_kernel_h<S, L, M, NT, LAY, INP, OUTP, RS...>;
+    return e;
+}
+
+// A row tile kept for layouts the register-held one cannot address.
+template <class S, int L, int M, int NT, int LAY, int INP, int OUTP, int... RS>
+constexpr KernelEntry make_variant_h()
+{
+    KernelEntry e = make_entry_h<S, L, M, NT, LAY, INP, OUTP, RS...>();
+    e.tune_only = 1;
+    return e;
+}
+
+// 16-bit rows held in registers (reg_rows_kernel_h).
+template <class S, int HINT, int L, int M, int NT, int... RS>
+constexpr KernelEntry make_reg_rows_h()
+{
+    KernelEntry e = reg_shape<float, L, M, NT, PAT_ROW, PAT_ROW, RS...>();
+    e.lds_bytes += (NT / M > 64 ? NT / M / 64 : 1) * (int)sizeof(float);
+    e.store = std::is_same<S, st_f16>::value ? 1 : 2;
+    e.fn = &reg_rows_kernel_h<S, L, M, NT, HINT, RS...>;
+    return e;
+}
+
+// The same for batches within the Infinity Cache only.
+template <class S, int HINT, int L, int M, int NT, int... RS>
+constexpr KernelEntry make_reg_cached_h()
+{
+    KernelEntry e = make_reg_rows_h<S, HINT, L, M, NT, RS...>();
+    e.tune_only = 1;
+    e.cached = 1;
     return e;
 }
 

@@ -55,20 +55,21 @@ struct PlaneGeom {
 // 16 bytes and they share their twiddles), or along the sequence in mirror
 // pairs (MAP_M, two butterflies per thread: thread t of a sequence has j = t
 // and L/R - t, whose elements are k and L - k; t = 0 has 0 and L/2R, which
-// mirror themselves).
-enum : int { MAP_J = 0, MAP_S = 1, MAP_P = 2, MAP_M = 3 };
+// mirror themselves), or in pairs of neighbours (MAP_N: thread t of a sequence
+// has j = 2t and 2t + 1, whose HBM accesses join).
+enum : int { MAP_J = 0, MAP_S = 1, MAP_P = 2, MAP_M = 3, MAP_N = 4 };
 template <int L, int M, int NT, int MAP, int R>
 struct Bfly {
     static constexpr int LR = L / R;
     static constexpr int W = MAP == MAP_P ? 2 : 1;  // butterflies that share j
     static constexpr int N = M * L / NT / R / W;    // groups of them per thread
     static_assert(N >= 1 && N * W * R * NT == M * L, "whole butterflies per thread");
-    static_assert(MAP != MAP_M || N == 2, "mirror pairs");
+    static_assert((MAP != MAP_M && MAP != MAP_N) || N == 2, "pairs of butterflies");
     static __device__ __forceinline__ int s(int tid, int q)
     {
         const int b = tid + q * NT;
         if constexpr (M == 1) return 0;
-        else if constexpr (MAP == MAP_M) return tid / (LR / 2);
+        else if constexpr (MAP == MAP_M || MAP == MAP_N) return tid / (LR / 2);
         else return MAP == MAP_J ? b / LR : MAP == MAP_S ? b % M : b % (M / 2) * 2;
     }
     static __device__ __forceinline__ int j(int tid, int q)
@@ -77,6 +78,8 @@ struct Bfly {
         if constexpr (MAP == MAP_M) {
             const int t = tid % (LR / 2);
             return q == 0 ? t : t ? LR - t : LR / 2;
+        } else if constexpr (MAP == MAP_N) {
+            return tid % (LR / 2) * 2 + q;
         } else if constexpr (M == 1) return b;
         else return MAP == MAP_J ? b % LR : MAP == MAP_S ? b / M : b / (M / 2);
     }
@@ -383,6 +386,100 @@ __global__ void __launch_bounds__(NT, 4) reg_tile_kernel(TileArgs a)
                     for (int e = 0; e < A::W; e++)
                         if (s + e < nvalid) p[e] = x[e * RL + r];
                 }
+            }
+        }
+    }
+}
+
+// scale of a 16-bit transform from the largest |re| + |im| of its input: the
+// largest power of two up to 1 with m * gain * scale <= limit
+__device__ __forceinline__ float scale_from_max(float m, float gain, float limit)
+{
+    const float q = m * gain / limit;  // limit is a power of two: exact division
+    if (!(q > 1.0f) || !(q <= 3.0e38f)) return 1.0f;  // fits already, or not finite
+    const uint32_t u = __float_as_uint(q);
+    const int k = (int)((u >> 23) & 255u) - 127 + ((u & 0x7fffffu) ? 1 : 0);  // ceil(log2 q), q normal
+    return __uint_as_float((uint32_t)(127 - k) << 23);
+}
+
+// Rows of 16-bit storage (FP16 / BF16 pairs, FP32 arithmetic), a whole row per
+// workgroup, so the automatic scale (TileArgs::auto_scale) needs no pass of its
+// own: each thread takes the largest |re| + |im| of the elements it loads, the
+// row's threads reduce it, and the store multiplies by the scale.
+template <class S, int L, int M, int NT, int HINT, int... RS>
+__global__ void __launch_bounds__(NT, 4) reg_rows_kernel_h(TileArgs a)
+{
+    using T = float;
+    constexpr int E = M * L / NT;
+    constexpr int R1 = first_radix<RS...>(), RL = last_radix<RS...>();
+    static_assert(E == 2 * R1 && E == 2 * RL, "one pair of butterflies per thread at both ends");
+    using G = PlaneGeom<T, L, M, R1, true>;
+    using A = Bfly<L, M, NT, MAP_N, R1>;
+    using B = Bfly<L, M, NT, MAP_N, RL>;
+    constexpr int TPS = NT / M;  // threads of a row
+    typedef uint32_t word2 __attribute__((ext_vector_type(2), aligned(4)));
+    __shared__ __align__(16) T plane[G::ELEMS];
+    __shared__ float red[TPS > 64 ? TPS / 64 : 1];
+    const int tid = threadIdx.x;
+    const int tile = a.xcd_remap ? xcd_tile(blockIdx.x, gridDim.x) : (int)blockIdx.x;
+    const int t2 = tile / a.tiles_inner;
+    const int ti = tile - t2 * a.tiles_inner;
+    const int o2 = t2 / a.n_outer1;
+    const int o = t2 - o2 * a.n_outer1;
+    const int s0 = ti * M;
+    const int nvalid = min(M, a.n_inner - s0);
+    const int s = A::s(tid, 0), j = A::j(tid, 0);
+    const int64_t ibase = in_base(a, o2, o) + (int64_t)s0 * a.in_inner;
+    cx<T> v[E];
+    float m = 0.0f;
+    {
+        const bool sw = swap_in_of(a, o);
+        const char *ib = reinterpret_cast<const char *>(reinterpret_cast<const uint32_t *>(a.in) + ibase);
+        const uint32_t to = ((uint32_t)s * (uint32_t)a.in_inner + (uint32_t)j) * 4u;
+#pragma unroll
+        for (int r = 0; r < R1; r++) {
+            word2 w = {0u, 0u};
+            if (M == 1 || s < nvalid) {
+                const word2 *p = reinterpret_cast<const word2 *>(ib + r * A::LR * 4 + to);
+                w = (HINT & HINT_LD) ? __builtin_nontemporal_load(p) : *p;
+            }
+            const cx<T> x0 = hdec<S>(w.x), x1 = hdec<S>(w.y);
+            m = fmaxf(m, fmaxf(fabsf(x0.re) + fabsf(x0.im), fabsf(x1.re) + fabsf(x1.im)));
+            v[r] = sw ? swap_ri(x0) : x0;
+            v[R1 + r] = sw ? swap_ri(x1) : x1;
+        }
+    }
+    if (a.auto_scale) {
+#pragma unroll
+        for (int off = (TPS < 64 ? TPS : 64) / 2; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
+        if (TPS > 64 && (tid & 63) == 0) red[tid >> 6] = m;  // read after the passes' barriers
+    }
+    reg_passes<T, L, M, NT, G, MAP_N, MAP_J, MAP_N, 1, RS...>(plane, v, nullptr, tid, a, RegTw<T, L, M, NT, 1, R1, MAP_N>{});
+    float scl = 1.0f;
+    if (a.auto_scale) {
+        if constexpr (TPS > 64) {
+            static_assert(M == 1 && sizeof...(RS) > 1, "the row's waves are the workgroup's, with barriers between the passes");
+#pragma unroll
+            for (int i = 0; i < TPS / 64; i++) m = fmaxf(m, red[i]);
+        }
+        scl = scale_from_max(m, a.gain, a.limit);
+        if (tid % TPS == 0 && s < nvalid) a.auto_scale[s0 + s] = scl;
+    } else if (a.scale && s < nvalid) {
+        scl = a.scale[(a.scale_off + ibase + (int64_t)s * a.in_inner) / a.scale_div];
+    }
+    {
+        const bool sw = swap_out_of(a, o);
+        char *ob = reinterpret_cast<char *>(reinterpret_cast<uint32_t *>(a.out) + out_base(a, o2, o) +
+                                            (int64_t)s0 * a.out_inner);
+        const uint32_t to = ((uint32_t)s * (uint32_t)a.out_inner + (uint32_t)B::j(tid, 0)) * 4u;
+        if (M == 1 || s < nvalid) {
+#pragma unroll
+            for (int r = 0; r < RL; r++) {
+                const cx<T> x0 = {v[r].re * scl, v[r].im * scl}, x1 = {v[RL + r].re * scl, v[RL + r].im * scl};
+                const word2 w = {henc<S>(sw ? swap_ri(x0) : x0), henc<S>(sw ? swap_ri(x1) : x1)};
+                word2 *p = reinterpret_cast<word2 *>(ob + r * B::LR * 4 + to);
+                if constexpr (HINT & HINT_ST) __builtin_nontemporal_store(w, p);
+                else *p = w;
             }
         }
     }

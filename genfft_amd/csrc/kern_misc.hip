@@ -18,6 +18,7 @@
 // All of them are grid-stride loops over (pair, batch) with 64-bit indices
 // and read each input element once.
 #include "gfft_misc.h"
+#include "gfft_regtile.h"
 
 namespace gfft {
 
@@ -212,15 +213,6 @@ __global__ void __launch_bounds__(256) repack_kernel(RepackArgs a)
 }
 
 // ---- per-transform scale of 16-bit storage transforms -------------------
-__device__ __forceinline__ float scale_from_max(float m, float gain, float limit)
-{
-    const float q = m * gain / limit;  // limit is a power of two: exact division
-    if (!(q > 1.0f) || !(q <= 3.0e38f)) return 1.0f;  // fits already, or not finite
-    const uint32_t u = __float_as_uint(q);
-    const int k = (int)((u >> 23) & 255u) - 127 + ((u & 0x7fffffu) ? 1 : 0);  // ceil(log2 q), q normal
-    return __uint_as_float((uint32_t)(127 - k) << 23);
-}
-
 template <class S>
 __device__ __forceinline__ float l1_of(uint32_t w)
 {
@@ -228,18 +220,43 @@ __device__ __forceinline__ float l1_of(uint32_t w)
     return fabsf(v.re) + fabsf(v.im);
 }
 
-// small transforms (rows * width <= 1024): one thread per transform writes
-// its scale directly
-template <class S>
-__global__ void __launch_bounds__(256) amax_small_kernel(AmaxArgs a)
+// small transforms (rows * width <= 1024): `lanes` neighbouring threads (a
+// power of two up to 64) per transform read it together, 16 bytes each where
+// the layout allows, reduce its largest value and write its scale directly.
+// U transforms' loads are in flight at a time.
+template <class S, int U>
+__global__ void __launch_bounds__(256) amax_small_kernel(AmaxArgs a, int lanes)
 {
     const uint32_t *in = reinterpret_cast<const uint32_t *>(a.in);
-    for (int64_t b = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; b < a.batch;
-         b += (int64_t)gridDim.x * blockDim.x) {
-        float m = 0.0f;
-        for (int64_t r = 0; r < a.rows; r++)
-            for (int64_t w = 0; w < a.width; w++) m = fmaxf(m, l1_of<S>(in[b * a.dist + r * a.pitch + w]));
-        reinterpret_cast<float *>(a.bits)[b] = scale_from_max(m, a.gain, a.limit);
+    const int per = 256 / lanes, lane = threadIdx.x & (lanes - 1);
+    const int w = a.vec ? 4 : 1;
+    const int elems = (int)(a.rows * a.width), width = (int)a.width;
+    const int64_t stride = (int64_t)gridDim.x * per;
+    for (int64_t b0 = blockIdx.x * (int64_t)per + threadIdx.x / lanes; b0 - threadIdx.x / lanes < a.batch; b0 += U * stride) {
+        float m[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) m[u] = 0.0f;
+        for (int e = lane * w; e < elems; e += lanes * w) {
+            const int r = e / width;
+            const int64_t at = r * a.pitch + (e - r * width);
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const int64_t b = b0 + u * stride;
+                if (b >= a.batch) continue;
+                if (a.vec) {
+                    const uint4 q = *reinterpret_cast<const uint4 *>(in + b * a.dist + at);
+                    m[u] = fmaxf(m[u], fmaxf(fmaxf(l1_of<S>(q.x), l1_of<S>(q.y)), fmaxf(l1_of<S>(q.z), l1_of<S>(q.w))));
+                } else {
+                    m[u] = fmaxf(m[u], l1_of<S>(in[b * a.dist + at]));
+                }
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int64_t b = b0 + u * stride;
+            for (int off = lanes >> 1; off > 0; off >>= 1) m[u] = fmaxf(m[u], __shfl_xor(m[u], off, 64));
+            if (lane == 0 && b < a.batch) reinterpret_cast<float *>(a.bits)[b] = scale_from_max(m[u], a.gain, a.limit);
+        }
     }
 }
 
@@ -338,9 +355,20 @@ hipError_t launch_amax_scale(AmaxArgs a, hipStream_t s)
     const int64_t E = a.rows * a.width;
     const bool f16 = a.store == 1;
     if (E <= 1024) {
-        const unsigned g = grid_for(a.batch);
-        if (f16) hipLaunchKernelGGL(amax_small_kernel<st_f16>, dim3(g), dim3(256), 0, s, a);
-        else hipLaunchKernelGGL(amax_small_kernel<st_bf16>, dim3(g), dim3(256), 0, s, a);
+        a.vec = (a.width % 4 == 0) && (a.pitch % 4 == 0) && (a.dist % 4 == 0) && (((uintptr_t)a.in & 15) == 0);
+        int lanes = 1;
+        while (lanes < 64 && lanes * (a.vec ? 4 : 1) < E) lanes <<= 1;
+        // MI355X, FP16, 2^20 transforms of 16 elements with their scales: 68 us
+        // with a thread per transform and one load in flight, 44 us so (images
+        // of up to 1024 elements, whose rows a thread walked alone, gain more);
+        // batches that one round of threads covers want no more in flight
+        if (a.batch * lanes <= ((int64_t)1 << 18)) {
+            const unsigned g = grid_for(a.batch * lanes);
+            hipLaunchKernelGGL((f16 ? amax_small_kernel<st_f16, 1> : amax_small_kernel<st_bf16, 1>), dim3(g), dim3(256), 0, s, a, lanes);
+        } else {
+            const unsigned g = grid_for((a.batch * lanes + 3) / 4);
+            hipLaunchKernelGGL((f16 ? amax_small_kernel<st_f16, 4> : amax_small_kernel<st_bf16, 4>), dim3(g), dim3(256), 0, s, a, lanes);
+        }
         return hipGetLastError();
     }
     // 64 Ki elements (256 KiB) per block: with 8 Ki, FP16 2^20 x 64 with the

@@ -263,9 +263,7 @@ constexpr RowsEntry lds_rows()
 template <typename T, int MODE, int HINT, int L, int M, int NT, int... RS>
 constexpr RowsEntry reg_rows(int64_t most = 0)
 {
-    KernelEntry e = reg_shape<T, L, M, NT, PAT_ROW, PAT_ROW, HINT, RS...>();
-    e.fn = nullptr;
-    return {e, MODE, most, &real_rows_reg_kernel<T, L, M, NT, MODE, HINT, RS...>};
+    return {reg_shape<T, L, M, NT, PAT_ROW, PAT_ROW, RS...>(), MODE, most, &real_rows_reg_kernel<T, L, M, NT, MODE, HINT, RS...>};
 }
 
 template <typename T, int MODE, int HINT, int L, int NT, int... RS>

@@ -349,10 +349,10 @@ int narrow_row_variant(int prec, int L, int64_t batch, int num_cus)
 
 // Registry index of the row -> row entry of length L with `flag` set
 // (KernelEntry::wave or ::wide), or -1.
-int row_variant_of(int prec, int L, int KernelEntry::*flag)
+int row_variant_of(int prec, int L, int KernelEntry::*flag, int store = 0)
 {
     int cnt = 0;
-    const KernelEntry *tab = tile_table(prec, 0, &cnt);
+    const KernelEntry *tab = tile_table(prec, store, &cnt);
     for (int i = 0; i < cnt; i++)
         if (tab[i].*flag && !tab[i].long_row && tab[i].L == L && tab[i].inp == PAT_ROW && tab[i].outp == PAT_ROW) return i;
     return -1;
@@ -780,9 +780,8 @@ struct Builder {
     // default tiles would leave CUs idle; -1: the default.
     int cached_row_variant(int n, int64_t rows) const
     {
-        if (store) return -1;
-        const int v = n * rows * (int64_t)csize <= kCachedBytes ? row_variant_of(prec, n, &KernelEntry::cached) : -1;
-        return v >= 0 ? v : narrow_row_variant(prec, n, rows, p->num_cus);
+        const int v = n * rows * (int64_t)csize <= kCachedBytes ? row_variant_of(prec, n, &KernelEntry::cached, store) : -1;
+        return v >= 0 || store ? v : narrow_row_variant(prec, n, rows, p->num_cus);
     }
 
     // Register-held row tile for `batch` rows of length n, one past the LDS
@@ -840,8 +839,8 @@ struct Builder {
                 if (batch == 1) variant = row_variant_of(prec, (int)n, &KernelEntry::wave);
                 else if (n * batch * (int64_t)csize >= kStreamBytes)
                     variant = row_variant_of(prec, (int)n, &KernelEntry::wide);
-                if (variant < 0) variant = cached_row_variant((int)n, batch);
             }
+            if (variant < 0) variant = cached_row_variant((int)n, batch);
             return tile((int)n, PAT_ROW, PAT_ROW, 0, in_buf, in_off, out_buf, out_off, batch, 1, 1, 0, 0,
                         in_dist, 1, 0, 0, out_dist, 1, TW_NONE, 0, first, last, variant);
         }
@@ -1873,12 +1872,18 @@ int describe_launches(const std::vector<Launch> &launches, const std::string &he
 
 // Executes the plan's launches in order on stream s.  With `events`, records
 // events[2i] / events[2i+1] on s around launch i (per-kernel timing).
-// With `scale` (16-bit storage plans), the tile launches that read the plan's
-// input multiply transform b's values by scale[b] on their store.
+// 16-bit storage plans: the tile launches that read the plan's input multiply
+// transform b's values by given[b] on their store, or (scales_itself plans)
+// compute the scale with `gain` and `limit` and write it to automatic[b].
+struct ScaleArgs {
+    const float *given = nullptr;
+    float *automatic = nullptr;
+    int64_t div = 1;  // input elements from one transform to the next
+    float gain = 0, limit = 0;
+};
 int run_launches(const std::vector<Launch> &launches, int prec, int xcd_remap, const void *in, void *out,
                  void *scratch, int direction, hipStream_t s, hipEvent_t *events = nullptr,
-                 const float *scale = nullptr, int64_t scale_div = 1, hipEvent_t stop = nullptr,
-                 bool *stopped = nullptr);
+                 const ScaleArgs &scale = ScaleArgs{}, hipEvent_t stop = nullptr, bool *stopped = nullptr);
 
 // The launches this call runs, and whether its buffers overlap in a way their
 // order can corrupt (see gfft_plan_s::overlap_hazard), so that the input has
@@ -1894,6 +1899,15 @@ const std::vector<Launch> &route(const gfft_plan_s *p, const void *in, const voi
     return p->alt.empty() ? p->launches : p->alt;
 }
 
+// Whether the plan's one launch holds every transform whole in a workgroup's
+// registers and so can find its automatic scale by itself.
+bool scales_itself(const gfft_plan_s *p)
+{
+    const gfft_desc &d = p->d;
+    return d.kind == GFFT_C2C && p->launches.size() == 1 && p->launches[0].type == LT_TILE && p->launches[0].k->reg &&
+           p->launches[0].k->store;
+}
+
 // Whether a launch of the list works in the plan's shared workspace.
 bool uses_scratch(const std::vector<Launch> &launches)
 {
@@ -1903,7 +1917,7 @@ bool uses_scratch(const std::vector<Launch> &launches)
 }
 
 int run(gfft_plan_s *p, const void *in, void *out, int direction, hipStream_t s,
-        hipEvent_t *events = nullptr, const float *scale = nullptr)
+        hipEvent_t *events = nullptr, const ScaleArgs &scale = ScaleArgs{})
 {
     if (p->scratch_bytes && !p->scratch)
         return fail(GFFT_ERR_INVALID_ARG, "plan created with GFFT_FLAG_NO_WORKSPACE holds no workspace: "
@@ -1911,8 +1925,7 @@ int run(gfft_plan_s *p, const void *in, void *out, int direction, hipStream_t s,
     bool stage = false;
     const std::vector<Launch> &launches = route(p, in, out, &stage);
     if ((!p->scratch || !uses_scratch(launches)) && !stage)  // no shared workspace: calls on any streams are independent
-        return run_launches(launches, p->prec, p->xcd_remap, in, out, p->scratch, direction, s, events, scale,
-                            p->scale_div);
+        return run_launches(launches, p->prec, p->xcd_remap, in, out, p->scratch, direction, s, events, scale);
     std::lock_guard<std::mutex> lk(p->order.mu);
     if (stage && !p->stage) {
         hipError_t e = hipMalloc(&p->stage, p->in_bytes);
@@ -1930,7 +1943,7 @@ int run(gfft_plan_s *p, const void *in, void *out, int direction, hipStream_t s,
     }
     bool stopped = false;
     int st = run_launches(launches, p->prec, p->xcd_remap, in, out, p->scratch, direction, s, events, scale,
-                          p->scale_div, p->order.stop_event(s), &stopped);
+                          p->order.stop_event(s), &stopped);
     if (st) return st;
     if (stopped) p->order.mark(s);
     else HIP_TRY(p->order.after(s));
@@ -1938,8 +1951,8 @@ int run(gfft_plan_s *p, const void *in, void *out, int direction, hipStream_t s,
 }
 
 int run_launches(const std::vector<Launch> &launches, int prec, int xcd_remap, const void *in, void *out,
-                 void *scratch, int direction, hipStream_t s, hipEvent_t *events, const float *scale,
-                 int64_t scale_div, hipEvent_t stop, bool *stopped)
+                 void *scratch, int direction, hipStream_t s, hipEvent_t *events, const ScaleArgs &scale,
+                 hipEvent_t stop, bool *stopped)
 {
     struct {
         int prec, xcd_remap;
@@ -1969,10 +1982,13 @@ int run_launches(const std::vector<Launch> &launches, int prec, int xcd_remap, c
             // hardware's block order (measured: c64 2^20 column pass 0.441 ->
             // 0.435 ms); interleaved tiles keep neighbours on one XCD
             a.xcd_remap = p->xcd_remap && a.runs >= 0;
-            if (scale && l.in_buf == B_IN) {
-                a.scale = scale;
-                a.scale_div = scale_div;
+            if (l.in_buf == B_IN) {
+                a.scale = scale.given;
+                a.scale_div = scale.div;
                 a.scale_off = l.in_off / (int64_t)csize_of(l.k->prec, l.k->store);
+                a.auto_scale = scale.automatic;
+                a.gain = scale.gain;
+                a.limit = scale.limit;
             }
             void *args[] = {&a};
             HIP_TRY(hipExtLaunchKernel((const void *)l.k->fn, dim3((unsigned)l.grid), dim3(l.k->NT), args, 0, s,
@@ -2756,6 +2772,16 @@ int gfft_execute_scaled(gfft_plan plan, const void *in, void *out, int direction
         return fail(GFFT_ERR_INVALID_ARG, "scale_mode must be GFFT_SCALE_GIVEN or GFFT_SCALE_AUTO");
     if (int st = on_plan_device(plan->device)) return st;
     hipStream_t s = (hipStream_t)stream;
+    ScaleArgs sc;
+    sc.div = plan->scale_div;
+    sc.gain = (float)plan->amax_gain;
+    // largest bound a stored value may reach: 2^15 keeps FP16 (max 65504)
+    // finite with room for rounding; BF16 shares FP32's exponent range
+    sc.limit = plan->store == 1 ? 32768.0f : 0x1p120f;
+    if (scale_mode == GFFT_SCALE_AUTO && scales_itself(plan)) {
+        sc.automatic = scales;
+        return run(plan, in, out, direction, s, nullptr, sc);
+    }
     if (scale_mode == GFFT_SCALE_AUTO) {
         AmaxArgs a{};
         a.in = in;
@@ -2766,13 +2792,12 @@ int gfft_execute_scaled(gfft_plan plan, const void *in, void *out, int direction
         a.width = plan->amax_width;
         a.pitch = plan->amax_pitch;
         a.dist = plan->scale_div;
-        a.gain = (float)plan->amax_gain;
-        // largest bound a stored value may reach: 2^15 keeps FP16 (max 65504)
-        // finite with room for rounding; BF16 shares FP32's exponent range
-        a.limit = plan->store == 1 ? 32768.0f : 0x1p120f;
+        a.gain = sc.gain;
+        a.limit = sc.limit;
         HIP_TRY(launch_amax_scale(a, s));
     }
-    return run(plan, in, out, direction, s, nullptr, scales);
+    sc.given = scales;
+    return run(plan, in, out, direction, s, nullptr, sc);
 }
 
 int gfft_execute_scrambled(gfft_plan plan, const void *in, void *out, int direction, void *stream)
@@ -2813,7 +2838,7 @@ int gfft_execute_scrambled(gfft_plan plan, const void *in, void *out, int direct
     a.out = plan->perm;
     HIP_TRY(launch_bitrev(plan->prec, a, s));
     int st = run_launches(plan->launches, plan->prec, plan->xcd_remap, plan->perm, out, plan->scratch, direction, s,
-                          nullptr, nullptr, plan->scale_div);
+                          nullptr);
     if (st) return st;
     HIP_TRY(plan->order.after(s));
     return GFFT_OK;

@@ -173,3 +173,68 @@ def test_long_real_rows_in_place(gpu, prec, n):
     assert O.rel_l2_rows(h, np.fft.rfft(x.astype(np.float64))).max() <= tol(n)
     G.Plan(C.GFFT_C2R, n, precision=p, batch=batch).execute(buf, reals, inverse=True)
     assert O.rel_l2_rows(reals.cpu().numpy().reshape(batch, n) / n, x).max() <= 2 * tol(n)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fmt", ["f16", "bf16"])
+@pytest.mark.parametrize("n,batch,pin,pout", [
+    (32, 33, 0, 0), (32, 5, 1, 3), (64, 17, 0, 2), (128, 9, 1, 0), (256, 5, 0, 1), (512, 3, 3, 3), (512, 5, 0, 0),
+    (1024, 3, 0, 0), (2048, 2, 1, 1), (4096, 1, 0, 0), (8192, 2, 0, 5), (16384, 2, 3, 0)])
+def test_half_rows_and_their_scale(gpu, fmt, n, batch, pin, pout):
+    """16-bit rows with the automatic scale, a given scale and none, at padded
+    pitches, both directions.  The scale is exactly the largest power of two up
+    to 1 with n * max(|re| + |im|) * scale <= 2^15 (FP16) or 2^120 (BF16); the
+    values are within one storage rounding plus the FP32 transform's bound."""
+    import genfft_amd as G
+    prec, tdt, u, top = (C.GFFT_F16, torch.float16, 2.0 ** -11, 2.0 ** 15) if fmt == "f16" else \
+        (C.GFFT_BF16, torch.bfloat16, 2.0 ** -8, 2.0 ** 120)
+    g = torch.Generator().manual_seed(n + batch)
+    x = (torch.randn(batch, n + pin, 2, generator=g) * 10.0 ** torch.arange(batch).remainder(4).view(-1, 1, 1)).to(tdt)
+    v = torch.view_as_complex(x[:, :n].double())
+    l1 = x[:, :n].float().abs().sum(-1).amax(-1).double() * n / top
+    auto = torch.exp2(-torch.ceil(torch.log2(l1.clamp(min=1.0))))
+    plan = G.Plan(C.GFFT_C2C, n, precision=prec, batch=batch, in_dist=n + pin, out_dist=n + pout)
+    tx = x.to(gpu)
+    for inv in (False, True):
+        ref = torch.fft.ifft(v, norm="forward") if inv else torch.fft.fft(v)
+        for mode in ("auto", "given", "none"):
+            y = torch.full((batch, n + pout, 2), 5.0, dtype=tdt, device=gpu)
+            s = (auto / 4).float().to(gpu) if mode == "given" else torch.zeros(batch, device=gpu)
+            if mode == "none":
+                if fmt == "f16" and float(auto.min()) < 1:
+                    continue  # would overflow
+                plan.execute(tx, y, inverse=inv)
+                want = torch.ones(batch, dtype=torch.float64)
+            else:
+                plan.execute_scaled(tx, y, s, mode == "auto", inverse=inv)
+                want = s.cpu().double()
+            if mode == "auto":
+                assert torch.equal(want, auto)
+            h = torch.view_as_complex(y.cpu()[:, :n].double().contiguous())
+            r = ref * want[:, None]
+            err = (h - r).abs().square().sum(-1).sqrt() / r.abs().square().sum(-1).sqrt()
+            # FP16 outputs below 2^-14 round to multiples of 2^-24
+            floor = 2.0 ** -25 * (2 * n) ** 0.5 / r.abs().square().sum(-1).sqrt() if fmt == "f16" else 0.0
+            assert bool((err <= u + O.tol_c64(n) + floor).all())
+            if pout:
+                assert bool((y.cpu()[:-1, n:] == 5.0).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("w,h,pitch", [(4, 4, 4), (8, 16, 11), (32, 32, 32), (16, 64, 20), (2, 64, 3)])
+def test_scale_of_small_images(gpu, w, h, pitch):
+    """The scale pass of images of up to 1024 elements, dense and padded."""
+    import genfft_amd as G
+    batch = 37
+    g = torch.Generator().manual_seed(w * h)
+    x = (torch.randn(batch, h, pitch, 2, generator=g) * 10.0 ** torch.arange(batch).remainder(4).view(-1, 1, 1, 1)).half()
+    x[:, :, w:] = 60000.0  # gaps don't count
+    l1 = x[:, :, :w].float().abs().sum(-1).amax((-1, -2)).double() * (w * h) / 2.0 ** 15
+    plan = G.Plan(C.GFFT_C2C_2D, w, precision=C.GFFT_F16, n2=h, batch=batch, in_stride=pitch, out_stride=w)
+    y = torch.empty(batch, h, w, 2, dtype=torch.float16, device=gpu)
+    s = torch.zeros(batch, device=gpu)
+    plan.execute_scaled(x.to(gpu), y, s, True)
+    assert torch.equal(s.cpu().double(), torch.exp2(-torch.ceil(torch.log2(l1.clamp(min=1.0)))))
+    ref = torch.fft.fft2(torch.view_as_complex(x[:, :, :w].double().contiguous())) * s.cpu().double().view(-1, 1, 1)
+    got = torch.view_as_complex(y.cpu().double())
+    assert float((got - ref).norm() / ref.norm()) <= 2 * 2.0 ** -11 + O.tol_c64(max(2, w * h))
