@@ -25,10 +25,15 @@ struct KernelEntry {
     int persistent;  // 1: tile_fft_pipe_kernel (grid sized to the device, loops over tiles)
     int tune_only;   // 1: an alternative (radix order / tile width / threads) only the autotuner selects
     void (*fn)(TileArgs);
+    void (*fn_plain)(TileArgs);  // reg: the same with plain stores, where one is compiled
     int store;       // 0: complex T in memory; 1: FP16 pairs; 2: BF16 pairs (FP32 arithmetic)
     int gen_tw;      // 1: the last pass builds its twiddles from TileArgs::gen_lo / gen_hi (W_L)
     int wave;        // 1: one wavefront per row, lanes exchanged without LDS (wave_rows1024_kernel)
     int reg;         // 1: tile held in registers (reg_tile_kernel); its own pass twiddle table layout
+    int many;        // tiles per CU from which this one is taken instead of the LDS tile of its width
+    int64_t most;    // cols: bytes a side up to which it is taken (0: any)
+    int64_t least;   // cols: bytes a side from which it is taken
+    int cols;        // 1: column tile for whole column transforms only; 2: but not those of complex 2D planes
     int cached;      // 1: row tile the planner takes for batches within the Infinity Cache
     int long_row;    // 1: a row longer than the LDS row tiles (the planner takes it by its own rule)
     int wide;        // 1: double-width row tile the planner takes for batches past the Infinity Cache
@@ -165,11 +170,13 @@ constexpr KernelEntry reg_entry()
     return e;
 }
 
-// reg_tile_kernel with its stores streamed.
+// reg_tile_kernel with its stores streamed or plain (KernelEntry::fn_plain).
 template <typename T, int L, int M, int NT, int INP, int OUTP, int... RS>
 constexpr KernelEntry make_reg_entry()
 {
-    return reg_entry<T, L, M, NT, INP, OUTP, HINT_ST, RS...>();
+    KernelEntry e = reg_entry<T, L, M, NT, INP, OUTP, HINT_ST, RS...>();
+    e.fn_plain = &reg_tile_kernel<T, L, M, NT, INP, OUTP, HINT_NONE, RS...>;
+    return e;
 }
 
 // The row tile with streaming loads as well, which the planner takes for
@@ -180,6 +187,36 @@ constexpr KernelEntry make_reg_wide()
     KernelEntry e = reg_entry<T, L, M, NT, PAT_ROW, PAT_ROW, HINT_LD | HINT_ST, RS...>();
     e.tune_only = 1;
     e.wide = 1;
+    return e;
+}
+
+// Taken from `many` tiles per CU on.
+template <typename T, int L, int M, int NT, int INP, int OUTP, int... RS>
+constexpr KernelEntry make_reg_many(int many)
+{
+    KernelEntry e = make_reg_entry<T, L, M, NT, INP, OUTP, RS...>();
+    e.many = many;
+    return e;
+}
+
+// A column tile of a whole column transform (not of a four-step pass), which
+// the planner picks by width (Builder::col_variant).
+template <typename T, int L, int M, int NT, int... RS>
+constexpr KernelEntry make_reg_cols(int64_t most = 0)
+{
+    KernelEntry e = make_reg_entry<T, L, M, NT, PAT_COL, PAT_COL, RS...>();
+    e.most = most;
+    e.tune_only = 1;
+    e.cols = 1;
+    return e;
+}
+
+template <typename T, int L, int M, int NT, int... RS>
+constexpr KernelEntry make_reg_cols_big(int64_t least)
+{
+    KernelEntry e = make_reg_cols<T, L, M, NT, RS...>();
+    e.least = least;
+    e.cols = 2;
     return e;
 }
 

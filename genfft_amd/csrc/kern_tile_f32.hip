@@ -44,7 +44,7 @@ const KernelEntry kTable[] = {
     make_entry<T, 64, 64, 256, E_, C_, C_, 8, 8>(),
     make_entry<T, 128, 32, 256, E_, C_, C_, 16, 8>(),
     make_entry<T, 256, 16, 256, E_, C_, C_, 16, 16>(),
-    make_entry<T, 512, 16, 512, E_, C_, C_, 8, 8, 8>(),
+    make_variant<T, 512, 16, 512, E_, C_, C_, 8, 8, 8>(),
     make_entry<T, 1024, 16, 1024, E_, C_, C_, 16, 16, 4>(),
     make_entry<T, 1024, 8, 512, E_, C_, C_, 16, 16, 4>(),
     make_entry<T, 2048, 8, 1024, E_, C_, C_, 16, 8, 16>(),  // c64 2^22 column pass 0.550 ms (16*16*8: 0.592, 8*16*16: 0.565)
@@ -131,6 +131,34 @@ const KernelEntry kTable[] = {
     make_reg_wide<T, 16384, 1, 1024, 16, 4, 16, 16>(),
     make_reg_long<T, 32768, 1024, HINT_ST, 32, 32, 32>(),
     make_reg_long<T, 32768, 1024, HINT_LD | HINT_ST, 32, 32, 32>(),
+    // --- column tiles held in registers.  Four-step passes (MI355X, 1 GiB a
+    // pass): 512 rows 0.476 -> 0.421 ms (from 4 tiles per CU on; below, the
+    // LDS tile: 2^19 x 4 25 against 28 us), 2048 rows of 16 columns 0.540 ->
+    // 0.48-0.49 (8 columns are as much as the LDS holds: 64-byte runs).  Whole
+    // column transforms, by width (Builder::col_variant), us, LDS -> register
+    // tile: 512 x 999 8.0 -> 5.7, 1024 x 513 12.6 -> 7.2, 1024 x 4999 32 -> 20
+    // (the pipelined 16-column tile left 2 rounds of 256 workgroups, the second
+    // 22% full), 1024^2 x 16 images' columns 55 -> 42, 2048 x 2048 19.8 -> 17.1,
+    // 4096 x 2049 58 -> 40, 4096 x 6000 154 -> 110.  4096 rows past 96 MiB
+    // want 8 columns: two 4-column tiles per CU keep 8 MB of quarter lines in
+    // flight per XCD, twice its L2 (4096 x 4096: 135 us, LDS tile 105) ---
+    make_reg_many<T, 512, 16, 512, C_, C_, 16, 2, 16>(4),
+    make_reg_entry<T, 2048, 16, 1024, C_, C_, 16, 8, 16>(),
+    make_reg_cols<T, 64, 16, 128, 8, 8>(),
+    make_reg_cols<T, 128, 8, 128, 8, 2, 8>(),
+    make_reg_cols<T, 256, 8, 256, 8, 4, 8>(),
+    make_reg_cols<T, 512, 8, 512, 8, 8, 8>(),
+    make_reg_cols<T, 1024, 4, 256, 16, 4, 16>(),
+    make_reg_cols<T, 1024, 8, 512, 16, 4, 16>(),
+    make_reg_cols<T, 1024, 16, 512, 32, 32>(),
+    make_reg_cols<T, 2048, 4, 512, 16, 8, 16>(),
+    make_reg_cols<T, 2048, 8, 1024, 16, 8, 16>(),
+    make_reg_cols<T, 4096, 4, 512, 16, 16, 16>((int64_t)96 << 20),
+    make_reg_cols_big<T, 4096, 8, 1024, 16, 16, 16>((int64_t)96 << 20),
+    // --- transposing rows held in registers: 2048 points, 2^22 x 32 0.505 ->
+    // 0.456 ms (128-byte runs instead of 64) ---
+    make_reg_entry<T, 2048, 16, 1024, R_, C_, 16, 16, 8>(),
+    make_reg_entry<T, 4096, 8, 1024, R_, C_, 16, 16, 16>(),
 };
 // The 2^20 four-step's two pipelined passes paired in one launch (column pass
 // of chunk k, transposing row pass of chunk k - 1).

@@ -89,6 +89,23 @@ const KernelEntry kTable[] = {
     make_reg_wide<T, 8192, 1, 512, 8, 16, 8, 8>(),
     make_reg_long<T, 16384, 1024, HINT_ST, 16, 16, 8, 8>(),
     make_reg_long<T, 16384, 1024, HINT_LD | HINT_ST, 16, 16, 8, 8>(),
+    // --- column tiles held in registers: 2^22 x 16 four-step columns of 2048
+    // 0.612 -> 0.529 ms, transposing rows 0.563 -> 0.427; whole columns: 512 x
+    // 999 8.6 -> 6.8 us, 1024 x 4999 61 -> 48, 2048 x 2048 35 -> 28 (the
+    // pipelined 1024-row tile stays the four-step's: 0.469 against 0.496) ---
+    make_reg_entry<T, 2048, 8, 1024, C_, C_, 16, 8, 16>(),
+    make_reg_cols<T, 128, 8, 128, 8, 2, 8>(),
+    make_reg_cols<T, 128, 16, 256, 8, 2, 8>(),
+    make_reg_cols<T, 256, 4, 128, 8, 4, 8>(),
+    make_reg_cols<T, 256, 8, 256, 8, 4, 8>(),
+    make_reg_cols<T, 512, 4, 256, 8, 8, 8>(),
+    make_reg_cols<T, 512, 8, 512, 8, 8, 8>(),
+    make_reg_cols<T, 1024, 4, 256, 16, 4, 16>(),
+    make_reg_cols<T, 1024, 8, 512, 16, 4, 16>(),
+    make_reg_cols<T, 2048, 4, 512, 16, 8, 16>(),
+    make_reg_cols<T, 2048, 8, 1024, 16, 8, 16>(),
+    // --- transposing rows held in registers ---
+    make_reg_entry<T, 2048, 8, 1024, R_, C_, 16, 16, 8>(),
 };
 // The 2^20 four-step's two pipelined passes paired in one launch (column pass
 // of chunk k, transposing row pass of chunk k - 1).

@@ -413,7 +413,8 @@ int max_fourstep_col(int prec, int store = 0)
     const KernelEntry *tab = tile_table(prec, store, &cnt);
     const int cs = store ? 4 : (prec ? 16 : 8);
     for (int i = 0; i < cnt; i++)
-        if (tab[i].inp == PAT_COL && tab[i].outp == PAT_COL && tab[i].M * cs >= 64) best = std::max(best, tab[i].L);
+        if (tab[i].inp == PAT_COL && tab[i].outp == PAT_COL && tab[i].M * cs >= 64 && !tab[i].cols)
+            best = std::max(best, tab[i].L);
     return best;
 }
 
@@ -445,6 +446,26 @@ void four_step_split(int prec, int lg, int *l1, int *l2, int n1_override = 0)
     }
     *l1 = a;
     *l2 = b;
+}
+
+// The split of a batch of `bytes` a side that a plan of complex rows takes.
+// Its lengths just past the single-pass rows do better with columns of 256 (128
+// for c128 2^14), whose two passes are more alike and split a small batch over
+// more workgroups; MI355X, us per call against the row length of 1024 above:
+// c64 2^15 x 1 12.8 -> 10.7, 2^16 x 1 13.3 -> 10.9, x 256 97 -> 93 (x 1024 375
+// -> 384: not past the Infinity Cache), 2^17 x 16 18.8 -> 16.1, x 512 393 -> 380;
+// c128 2^14 x 1 15.4 -> 11.8, 2^15 x 1 16.2 -> 12.0, x 1024 403 -> 394, 2^16 x 1
+// 16.5 -> 12.4, 2^17 x 256 440 -> 399.
+void rows_split(int prec, int store, int lg, int64_t bytes, int *l1, int *l2, int n1_override)
+{
+    int n1 = n1_override;
+    const bool cached = bytes <= ((int64_t)128 << 20);
+    if (n1 <= 0 && !store) {
+        if (!prec && (lg == 17 || ((lg == 15 || lg == 16) && cached))) n1 = 8;
+        if (prec && lg >= 15 && lg <= 17) n1 = 8;
+        if (prec && lg == 14 && cached) n1 = 7;
+    }
+    four_step_split(prec, lg, l1, l2, n1);
 }
 
 // ---------------------------------------------------------------------------
@@ -506,6 +527,9 @@ struct Launch {
     C2rArgs cr{};
     RealRowsArgs rr{};
     RepackArgs rp{};
+    // register-held tiles: stores not streamed (KernelEntry::fn_plain), and the
+    // column-side runs cover whole 128-byte lines that no other tile touches
+    bool plain = false, own_lines = false;
     int rr_mode = RR_R2C;
     const RowsEntry *rre = nullptr;
     int in_buf = B_IN, out_buf = B_OUT;
@@ -644,6 +668,9 @@ bool tile_offsets_fit(int pat, int64_t L, int64_t M, int64_t inner, int64_t elem
 // Batches of at least this many bytes a side stream through HBM: row tiles
 // with the `wide` flag.
 constexpr int64_t kStreamBytes = (int64_t)512 << 20;
+// What a pass of up to this many bytes leaves for the next one is stored plain,
+// to be found in the Infinity Cache.
+constexpr int64_t kKeptBytes = (int64_t)256 << 20;
 // Row batches of at most this many bytes a side take the `cached` row tiles
 // (c64 2048 points on MI355X: 64 MiB 59.8 -> 55.8 us, 128 MiB 101.3 -> 101.4).
 constexpr int64_t kCachedBytes = (int64_t)128 << 20;
@@ -685,6 +712,8 @@ struct Builder {
              int tw_mode, int64_t tw_n, bool first, bool last, int variant = -1)
     {
         const KernelEntry *k = find_tile(prec, L, inp, outp, prefer_m, opts.pipe_mask, variant, store);
+        if (k && k->many && (n_inner + k->M - 1) / k->M * n_outer1 * n_outer2 < (int64_t)k->many * p->num_cus)
+            k = find_tile(prec, L, inp, outp, k->M, opts.pipe_mask, -1, store, true);
         if (k && k->reg && !(tile_offsets_fit(inp, k->L, k->M, in_inner, in_elem, csize) &&
                              tile_offsets_fit(outp, k->L, k->M, out_inner, out_elem, csize)))
             k = find_tile(prec, L, inp, outp, prefer_m, opts.pipe_mask, -1, store, true);
@@ -754,6 +783,24 @@ struct Builder {
         l.first = first;
         l.last = last;
         l.grid = ntiles;
+        if (k->reg && !store) {
+            // Whole lines (bases are checked per call): the hardware's block
+            // order was faster there (c64 2048 x 16, 2^22 x 32: columns 0.528 ->
+            // 0.497 ms, transposing rows 0.473 -> 0.456), and only there stores
+            // along a column side are streamed: runs that share lines with
+            // other tiles want the L2 to merge them (FFTVert 1024 x 4999, odd
+            // pitch: 41 us streamed, 21 plain).  What the next pass of
+            // the plan reads back within the Infinity Cache is stored plain
+            // too (c128 1024^2 x 16 images: 225 -> 188 us, one c64 4096^2: 164 -> 146).
+            auto lines = [&](int64_t v) { return v * (int64_t)csize % 128 == 0; };
+            const bool in_lines = inp == PAT_ROW || (k->M * (int64_t)csize >= 128 && lines(in_elem) && lines(in_outer) &&
+                                                     lines(in_outer2) && lines(in_off_el));
+            const bool out_lines = outp == PAT_ROW || (k->M * (int64_t)csize >= 128 && lines(out_elem) &&
+                                                       lines(out_outer) && lines(out_outer2) && lines(out_off_el));
+            const int64_t bytes = (int64_t)k->L * n_inner * n_outer1 * n_outer2 * (int64_t)csize;
+            l.own_lines = (inp == PAT_COL || outp == PAT_COL) && in_lines && out_lines;
+            l.plain = k->fn_plain && (!out_lines || (!last && bytes <= kKeptBytes));
+        }
         if (k->persistent) {
             // one resident wave of workgroups looping over the tiles
             int per_cu = 1;
@@ -853,7 +900,7 @@ struct Builder {
         // four-step: n = N1 (column length) * N2 (row length)
         const int lg = ilog2(n);
         int l1, l2;
-        four_step_split(prec, lg, &l1, &l2, opts.n1_log2);
+        rows_split(prec, store, lg, n * batch * (int64_t)csize, &l1, &l2, opts.n1_log2);
         const int64_t N1 = (int64_t)1 << l1, N2 = (int64_t)1 << l2;
         if (N1 > max_len(prec, PAT_COL, PAT_COL, store) || N2 > max_len(prec, PAT_ROW, PAT_COL, store))
             return fail(GFFT_ERR_UNSUPPORTED, "length %lld exceeds the two-pass limit", (long long)n);
@@ -970,6 +1017,32 @@ struct Builder {
         return GFFT_OK;
     }
 
+    // Register-held tile for whole column transforms of length L: the widest
+    // registered one (KernelEntry::cols) whose tiles still number at least the
+    // CUs, else the narrowest; where the default tile is wider than all of
+    // them, that one while it does.  -1: the default.  `plane`: the columns of a
+    // complex 2D transform, which keep tiles of 4 columns at 4096 rows (8 columns
+    // ran one 4096 x 4096 plane in 126 us instead of 145, FFTVert of 6000 such
+    // columns in 110 instead of 156).
+    int col_variant(int L, int64_t cols, int64_t batch, bool plane) const
+    {
+        if (store) return -1;
+        int cnt = 0, best = -1;
+        const KernelEntry *tab = tile_table(prec, 0, &cnt);
+        auto tiles = [&](int m) { return (cols + m - 1) / m * batch; };
+        auto better = [&](int m, int than) {
+            const bool a = tiles(m) >= p->num_cus, b = tiles(than) >= p->num_cus;
+            return a != b ? a : a ? m > than : m < than;
+        };
+        const int64_t bytes = cols * L * batch * (int64_t)csize;
+        for (int i = 0; i < cnt; i++)
+            if (tab[i].cols && tab[i].cols <= (plane ? 1 : 2) && tab[i].L == L && bytes > tab[i].least - 1 &&
+                (!tab[i].most || bytes <= tab[i].most) && (best < 0 || better(tab[i].M, tab[best].M))) best = i;
+        if (best < 0) return -1;
+        const KernelEntry *d = find_tile(prec, L, PAT_COL, PAT_COL, 0, opts.pipe_mask);
+        return d && d->M > tab[best].M && better(d->M, tab[best].M) ? -1 : best;
+    }
+
     // Column FFTs of length `rows` down `cols` columns, `batch` matrices.
     // in/out pitch (row stride) and batch distance in complex elements.
     int columns(int64_t rows, int64_t cols, int64_t batch, int in_buf, int64_t in_pitch, int64_t in_dist,
@@ -992,7 +1065,7 @@ struct Builder {
         const int maxcol = max_len(prec, PAT_COL, PAT_COL, store);
         if (rows <= maxcol)
             return tile((int)rows, PAT_COL, PAT_COL, 0, in_buf, 0, out_buf, 0, cols, batch, 1, 0, in_dist, 1,
-                        in_pitch, 0, out_dist, 1, out_pitch, TW_NONE, 0, first, last);
+                        in_pitch, 0, out_dist, 1, out_pitch, TW_NONE, 0, first, last, col_variant((int)rows, cols, batch, p->d.kind == GFFT_C2C_2D));
         // rows = A * B, sub-pass 1 over n2 (length B, rows n1 + A*n2) with
         // twiddle W_rows^(n1*k2) into scratch, sub-pass 2 over n1 (length A)
         // writing row k2 + B*k1.
@@ -1981,7 +2054,9 @@ int run_launches(const std::vector<Launch> &launches, int prec, int xcd_remap, c
             // workgroups that each take one contiguous run of tiles keep the
             // hardware's block order (measured: c64 2^20 column pass 0.441 ->
             // 0.435 ms); interleaved tiles keep neighbours on one XCD
-            a.xcd_remap = p->xcd_remap && a.runs >= 0;
+            const bool own = l.own_lines && ((uintptr_t)ip & 127) == 0 && ((uintptr_t)op & 127) == 0;
+            const bool plain = l.plain || (l.own_lines && !own && l.k->fn_plain);
+            a.xcd_remap = p->xcd_remap && a.runs >= 0 && !own;
             if (l.in_buf == B_IN) {
                 a.scale = scale.given;
                 a.scale_div = scale.div;
@@ -1991,8 +2066,8 @@ int run_launches(const std::vector<Launch> &launches, int prec, int xcd_remap, c
                 a.limit = scale.limit;
             }
             void *args[] = {&a};
-            HIP_TRY(hipExtLaunchKernel((const void *)l.k->fn, dim3((unsigned)l.grid), dim3(l.k->NT), args, 0, s,
-                                       nullptr, tail, 0));
+            HIP_TRY(hipExtLaunchKernel((const void *)(plain ? l.k->fn_plain : l.k->fn), dim3((unsigned)l.grid),
+                                       dim3(l.k->NT), args, 0, s, nullptr, tail, 0));
             if (tail && stopped) *stopped = true;
             break;
         }
@@ -2312,7 +2387,7 @@ int build_batch(gfft_batch_plan_s *p)
             continue;
         }
         int l1, l2;
-        four_step_split(prec, c.lg, &l1, &l2, b.opts.n1_log2);
+        rows_split(prec, 0, c.lg, L * c.count * (int64_t)cs, &l1, &l2, b.opts.n1_log2);
         const int64_t N1 = (int64_t)1 << l1, N2 = (int64_t)1 << l2;
         const int64_t chunk = std::max<int64_t>(1, std::min<int64_t>(c.count, ((int64_t)1 << 30) / (L * (int64_t)cs)));
         b.need_scratch(chunk * L);
@@ -2419,7 +2494,7 @@ std::vector<PlanOpts> tune_candidates(int prec, int64_t n)
         bool cpipe = false, rpipe = false;
         for (int i = 0; i < cnt; i++) {
             const KernelEntry &e = tab[i];
-            if (e.L == N1 && e.inp == PAT_COL && e.outp == PAT_COL) {
+            if (e.L == N1 && e.inp == PAT_COL && e.outp == PAT_COL && !e.tune_only) {
                 if (std::find(cms.begin(), cms.end(), e.M) == cms.end()) cms.push_back(e.M);
                 cpipe = cpipe || e.persistent;
             }

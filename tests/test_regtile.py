@@ -238,3 +238,49 @@ def test_scale_of_small_images(gpu, w, h, pitch):
     ref = torch.fft.fft2(torch.view_as_complex(x[:, :, :w].double().contiguous())) * s.cpu().double().view(-1, 1, 1)
     got = torch.view_as_complex(y.cpu().double())
     assert float((got - ref).norm() / ref.norm()) <= 2 * 2.0 ** -11 + O.tol_c64(max(2, w * h))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("prec,n,cols,pin,pout", [
+    ("c64", 64, 3, 0, 0), ("c64", 64, 17, 1, 0), ("c64", 128, 9, 0, 1), ("c64", 256, 1, 0, 0), ("c64", 256, 15, 2, 1),
+    ("c64", 512, 7, 0, 0), ("c64", 512, 4111, 0, 1), ("c64", 1024, 5, 1, 1), ("c64", 1024, 1030, 0, 0),
+    ("c64", 1024, 4097, 1, 0), ("c64", 2048, 3, 0, 0), ("c64", 2048, 1027, 0, 3), ("c64", 2048, 4112, 0, 0),
+    ("c64", 4096, 2, 1, 0), ("c64", 4096, 1026, 0, 0), ("c64", 4096, 3100, 0, 2),
+    ("c128", 128, 3, 0, 1), ("c128", 128, 4100, 0, 0), ("c128", 256, 5, 1, 0), ("c128", 256, 2050, 0, 0), ("c128", 512, 3, 0, 0),
+    ("c128", 512, 2056, 0, 0), ("c128", 1024, 2, 0, 1), ("c128", 1024, 2049, 0, 0), ("c128", 2048, 1, 0, 0),
+    ("c128", 2048, 2049, 1, 1)])
+def test_columns_vs_float64(gpu, prec, n, cols, pin, pout):
+    """Column tiles with missing columns, at aligned and odd pitches, on
+    aligned and shifted buffers, against numpy's float64 transform."""
+    import genfft_amd as G
+    p, ndt, tdt, tol = PREC[prec]
+    x = _rand((n, cols + pin), ndt, n + cols)
+    for inv, shift in ((False, 0), (True, 1)):
+        src = torch.zeros(n * (cols + pin) + shift, dtype=tdt, device=gpu)[shift:]
+        src.copy_(torch.from_numpy(x.reshape(-1)))
+        out = torch.full((n * (cols + pout) + shift,), 7 + 5j, dtype=tdt, device=gpu)[shift:]
+        G.FFTVert(n, tdt).transform(out, cols + pout, src, cols + pin, cols, inv)
+        h = out.cpu().numpy().reshape(n, cols + pout)
+        v = x[:, :cols].astype(np.complex128)
+        ref = np.fft.ifft(v, axis=0) * n if inv else np.fft.fft(v, axis=0)
+        assert O.rel_l2_rows(np.ascontiguousarray(h[:, :cols].T), np.ascontiguousarray(ref.T)).max() <= tol(n)
+        if pout:
+            assert np.all(h[:, cols:] == 7 + 5j)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("prec,n,batch", [
+    ("c64", 1 << 15, 3), ("c64", 1 << 16, 2), ("c64", 1 << 17, 3), ("c64", 1 << 19, 16), ("c64", 1 << 21, 9),
+    ("c64", 1 << 22, 3), ("c64", 1 << 23, 2), ("c128", 1 << 14, 3), ("c128", 1 << 15, 2), ("c128", 1 << 17, 2),
+    ("c128", 1 << 21, 3), ("c128", 1 << 22, 2)])
+def test_four_step_vs_float64(gpu, prec, n, batch):
+    """The splits and register-held passes of long transforms, both directions."""
+    import genfft_amd as G
+    p, ndt, tdt, tol = PREC[prec]
+    x = _rand((batch, n), ndt, 11)
+    tx = torch.from_numpy(x).to(gpu)
+    for inv in (False, True):
+        h = G.fft(tx, inverse=inv).cpu().numpy()
+        v = x.astype(np.complex128)
+        ref = np.fft.ifft(v) * n if inv else np.fft.fft(v)
+        assert O.rel_l2_rows(h, ref).max() <= tol(n)
