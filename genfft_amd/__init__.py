@@ -20,6 +20,7 @@ in the reference API.  Tensors must live on a GPU; there is no CPU fallback.
 """
 from __future__ import annotations
 
+import collections
 import ctypes
 import threading
 
@@ -94,7 +95,7 @@ def _check_gpu(*ts: torch.Tensor) -> torch.device:
     for t in ts:
         if not t.is_cuda:
             raise ValueError("genfft_amd works on GPU tensors only (got a CPU tensor)")
-        if not _row_major(t):
+        if not (t.is_contiguous() or _row_major(t)):  # a contiguous tensor is row-major
             raise ValueError(f"tensor with strides {tuple(t.stride())} is not row-major (innermost stride 1, "
                              "outer strides covering the inner ones); call .contiguous()")
         if dev is None:
@@ -139,6 +140,16 @@ class Plan:
         every byte the call reads or writes (no launch ever sees a short
         buffer)."""
         dev = _check_gpu(inp, out)
+        self._check_buffers(inp, out)
+        return dev
+
+    def _check_buffers(self, inp: torch.Tensor, out: torch.Tensor) -> None:
+        """Types and extents.  The bytes of a tensor's own elements are at most
+        those to the end of its storage, so those are looked up only when the
+        former are too few (a row-major view may be padded past its last row)."""
+        if inp.dtype in self._in_dt and inp.nbytes >= self.in_bytes and \
+                out.dtype in self._out_dt and out.nbytes >= self.out_bytes:
+            return
         for t, want, need, what in ((inp, self._in_dt, self.in_bytes, "input"),
                                     (out, self._out_dt, self.out_bytes, "output")):
             if t.dtype not in want:
@@ -146,10 +157,14 @@ class Plan:
             if _extent(t) < need:
                 raise ValueError(f"{what} holds {_extent(t)} bytes but the plan {'reads' if what == 'input' else 'writes'} "
                                  f"{need}")
-        return dev
 
     def execute(self, inp: torch.Tensor, out: torch.Tensor, inverse: bool = False, stream=None) -> None:
-        dev = self._check(inp, out)
+        self._execute_on(_check_gpu(inp, out), inp, out, inverse, stream)
+
+    def _execute_on(self, dev: torch.device, inp: torch.Tensor, out: torch.Tensor, inverse: bool = False,
+                    stream=None) -> None:
+        """execute() on tensors that _check_gpu has passed, on `dev`."""
+        self._check_buffers(inp, out)
         _call_on(_dev_idx(dev), stream, self._lib.gfft_execute, self._h, inp.data_ptr(), out.data_ptr(),
                  C.GFFT_INVERSE if inverse else C.GFFT_FORWARD)
 
@@ -303,9 +318,9 @@ _CACHE_BYTES = 4 << 30
 
 def _plan(kind, n, precision, device, **kw) -> Plan:
     global _cache
-    import collections
-    key = (kind, n, precision, device.index if device.index is not None else torch.cuda.current_device(),
-           tuple(sorted(kw.items())))
+    idx = device.index
+    key = (kind, n, precision, idx if idx is not None else torch.cuda.current_device(),
+           tuple(kw.items()) if len(kw) < 2 else tuple(sorted(kw.items())))
     with _cache_lock:
         if _cache is None:
             _cache = collections.OrderedDict()
@@ -361,7 +376,7 @@ class FFT:
         dev = _check_gpu(out, inp)
         _need_contig(out, inp)
         b = _batch_of(inp, self.n)
-        _plan(C.GFFT_C2C, self.n, self._prec, dev, batch=b).execute(inp, out, inverse=inv)
+        _plan(C.GFFT_C2C, self.n, self._prec, dev, batch=b)._execute_on(dev, inp, out, inv)
 
     def transform_no_scramble(self, inout: torch.Tensor, inv: bool = False) -> None:
         """fft.h:69-73: in place, input already in bit-reversed order."""
@@ -381,7 +396,7 @@ class FFT:
         dev = _check_gpu(out, inp)
         _need_contig(out, inp)
         b = _batch_of(inp, self.n)
-        _plan(C.GFFT_R2C, self.n, self._prec, dev, batch=b).execute(inp, out)
+        _plan(C.GFFT_R2C, self.n, self._prec, dev, batch=b)._execute_on(dev, inp, out)
 
     def transform_interleave(self, out: torch.Tensor, in1: torch.Tensor, in2: torch.Tensor) -> None:
         """fft.h:100-105: FFT of in1 + i*in2 (split later with separate_2x_real_FFT)."""
@@ -416,7 +431,7 @@ class RealFFT:
         if out.numel() < b * nout:
             raise ValueError("output too small")
         od = out.numel() // b
-        _plan(C.GFFT_R2C, self.n, self._prec, dev, batch=b, half=half, out_dist=od).execute(inp, out)
+        _plan(C.GFFT_R2C, self.n, self._prec, dev, batch=b, half=half, out_dist=od)._execute_on(dev, inp, out)
 
     def inverse(self, out: torch.Tensor, inp: torch.Tensor) -> None:
         """Half spectrum (n/2+1 bins) -> n reals, unscaled (the reference's
@@ -424,7 +439,7 @@ class RealFFT:
         dev = _check_gpu(out, inp)
         _need_contig(out, inp)
         b = _batch_of(out, self.n)
-        _plan(C.GFFT_C2R, self.n, self._prec, dev, batch=b).execute(inp, out, inverse=True)
+        _plan(C.GFFT_C2R, self.n, self._prec, dev, batch=b)._execute_on(dev, inp, out, True)
 
 
 class DIT:
@@ -462,7 +477,7 @@ class FFTVert:
             out_stride = in_stride = cols
         dev = _check_gpu(out, inp)
         _plan(C.GFFT_COLS, self.n, self._prec, dev, n2=int(cols), in_stride=int(in_stride),
-              out_stride=int(out_stride)).execute(inp, out, inverse=inv)
+              out_stride=int(out_stride))._execute_on(dev, inp, out, inv)
 
     def transform_no_scramble(self, data, stride, cols, inv: bool = False) -> None:
         """fft.h:132-136: in place, rows already in bit-reversed order."""
@@ -490,7 +505,7 @@ class FFT2D:
     def transform(self, out, out_stride, inp, in_stride, inv: bool = False, batch: int = 1) -> None:
         dev = _check_gpu(out, inp)
         _plan(C.GFFT_C2C_2D, self.width, self._prec, dev, n2=self.height, in_stride=int(in_stride),
-              out_stride=int(out_stride), batch=batch).execute(inp, out, inverse=inv)
+              out_stride=int(out_stride), batch=batch)._execute_on(dev, inp, out, inv)
 
 
 class RealFFT2D:
@@ -513,7 +528,7 @@ class RealFFT2D:
         odd included); ``out`` the full complex spectrum, pitch ``out_stride``."""
         dev = _check_gpu(out, inp)
         _plan(C.GFFT_R2C_2D, self.width, self._prec, dev, n2=self.height, in_stride=int(in_stride),
-              out_stride=int(out_stride)).execute(inp, out)
+              out_stride=int(out_stride))._execute_on(dev, inp, out)
 
     def forward_2x(self, out, out_stride, in1, in_stride1, in2, in_stride2) -> None:
         """FFTReal.h:106-118: the 2D FFT of in1 + i*in2 (two real images, pitches
@@ -540,7 +555,7 @@ class RealFFT2D:
         ``in_stride`` complex; ``out``: real, pitch ``out_stride`` scalars."""
         dev = _check_gpu(out, inp)
         _plan(C.GFFT_C2R_2D, self.width, self._prec, dev, n2=self.height, in_stride=int(in_stride),
-              out_stride=int(out_stride)).execute(inp, out, inverse=True)
+              out_stride=int(out_stride))._execute_on(dev, inp, out, True)
 
 
 def separate_2x_real_FFT(out1: torch.Tensor, out2: torch.Tensor, inp: torch.Tensor, n: int) -> None:

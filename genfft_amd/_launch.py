@@ -12,13 +12,16 @@ import torch
 
 from . import _capi as C
 
-# torch's raw current-stream query (an int handle, no Stream object); the
-# public query is the fallback where this build lacks it
+# torch's raw current-stream and current-device queries (int handles, no
+# objects); the public queries are the fallback where this build lacks them.
+# Every caller holds a GPU tensor, so the device runtime is up.
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_current_device = getattr(torch._C, "_cuda_getDevice", None) or torch.cuda.current_device
 
 
 def device_index(dev: torch.device) -> int:
-    return dev.index if dev.index is not None else torch.cuda.current_device()
+    idx = dev.index
+    return idx if idx is not None else torch.cuda.current_device()
 
 
 def stream_handle(idx: int, stream=None) -> int:
@@ -32,7 +35,9 @@ def stream_handle(idx: int, stream=None) -> int:
 
 def call_on(idx: int, stream, fn, *args) -> None:
     """C.check(fn(*args, stream_handle)) with device idx current."""
-    if torch.cuda.current_device() != idx:
+    if _current_device() != idx:
         with torch.cuda.device(idx):
             return call_on(idx, stream, fn, *args)
-    C.check(fn(*args, stream_handle(idx, stream)))
+    st = fn(*args, stream_handle(idx, stream))
+    if st:
+        C.check(st)
