@@ -668,9 +668,25 @@ bool tile_offsets_fit(int pat, int64_t L, int64_t M, int64_t inner, int64_t elem
 // Batches of at least this many bytes a side stream through HBM: row tiles
 // with the `wide` flag.
 constexpr int64_t kStreamBytes = (int64_t)512 << 20;
-// What a pass of up to this many bytes leaves for the next one is stored plain,
-// to be found in the Infinity Cache.
-constexpr int64_t kKeptBytes = (int64_t)256 << 20;
+// What a column pass of up to this many bytes leaves for the next pass is
+// stored plain, to be found in the Infinity Cache (MI355X, us streamed / plain:
+// c64 2^21 x 8, 128 MiB, 122 / 114, x 16 231 / 242, x 32 441 / 481).
+constexpr int64_t kKeptBytes = (int64_t)192 << 20;
+// The row pass of a 2D plan, whose columns run in place, stores plain up to
+// here (c64 1024^2 x 36, 288 MiB: 234 / 210 us, x 96 602 / 581, x 256, 2 GiB,
+// 1613 / 1621) ...
+constexpr int64_t kKeptRowBytes = (int64_t)1 << 30;
+// ... except where all of it is dirty in the L2s at the end, between the two
+// sizes, and its columns of up to kShortColumn points leave little time to
+// write it out (us streamed / plain: c64 1024 x 128, 8 MiB, 12.7 / 13.2, 16 MiB
+// 19.3 / 20.4, 24 MiB 22.4 / 23.8, 28 MiB 25.6 / 25.8, 4 MiB 11.4 / 11.3;
+// 1024^2, 24 MiB, 27.6 / 26.9).
+constexpr int64_t kDirtyLeast = (int64_t)4 << 20, kDirtyMost = (int64_t)24 << 20, kShortColumn = 512;
+// In-place columns of up to this many bytes keep the tile order of the row pass
+// before them, so that an XCD finds the images it left in its own L2 (c128 64 x
+// 128 images, 8 MiB: 16.2 -> 13.5 us, 10 MiB 17.3 / 17.4), from 8 images on
+// (256 x 128 x 4: 9.4 us in the hardware's order, 10.0 in the rows').
+constexpr int64_t kOneL2Bytes = (int64_t)8 << 20;
 // Row batches of at most this many bytes a side take the `cached` row tiles
 // (c64 2048 points on MI355X: 64 MiB 59.8 -> 55.8 us, 128 MiB 101.3 -> 101.4).
 constexpr int64_t kCachedBytes = (int64_t)128 << 20;
@@ -791,15 +807,20 @@ struct Builder {
             // other tiles want the L2 to merge them (FFTVert 1024 x 4999, odd
             // pitch: 41 us streamed, 21 plain).  What the next pass of
             // the plan reads back within the Infinity Cache is stored plain
-            // too (c128 1024^2 x 16 images: 225 -> 188 us, one c64 4096^2: 164 -> 146).
+            // too (c128 1024^2 x 16 images: 225 -> 188 us, one c64 4096^2: 164 -> 146;
+            // kKeptBytes and what follows it).
             auto lines = [&](int64_t v) { return v * (int64_t)csize % 128 == 0; };
             const bool in_lines = inp == PAT_ROW || (k->M * (int64_t)csize >= 128 && lines(in_elem) && lines(in_outer) &&
                                                      lines(in_outer2) && lines(in_off_el));
             const bool out_lines = outp == PAT_ROW || (k->M * (int64_t)csize >= 128 && lines(out_elem) &&
                                                        lines(out_outer) && lines(out_outer2) && lines(out_off_el));
             const int64_t bytes = (int64_t)k->L * n_inner * n_outer1 * n_outer2 * (int64_t)csize;
-            l.own_lines = (inp == PAT_COL || outp == PAT_COL) && in_lines && out_lines;
-            l.plain = k->fn_plain && (!out_lines || (!last && bytes <= kKeptBytes));
+            const bool row_pass = inp == PAT_ROW && outp == PAT_ROW && first && !last && p->d.kind == GFFT_C2C_2D;
+            const bool dirty = row_pass && p->d.n2 <= kShortColumn && bytes > kDirtyLeast && bytes <= kDirtyMost;
+            const bool near_rows = !first && in_buf == out_buf && bytes <= kOneL2Bytes && n_outer1 >= 8;
+            l.own_lines = (inp == PAT_COL || outp == PAT_COL) && in_lines && out_lines && !near_rows;
+            l.plain = k->fn_plain &&
+                      (!out_lines || near_rows || (!last && !dirty && bytes <= (row_pass ? kKeptRowBytes : kKeptBytes)));
         }
         if (k->persistent) {
             // one resident wave of workgroups looping over the tiles

@@ -284,3 +284,27 @@ def test_four_step_vs_float64(gpu, prec, n, batch):
         v = x.astype(np.complex128)
         ref = np.fft.ifft(v) * n if inv else np.fft.fft(v)
         assert O.rel_l2_rows(h, ref).max() <= tol(n)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("prec,w,h,batch,pad", [
+    ("c64", 256, 128, 16, 0), ("c64", 1024, 128, 24, 0), ("c64", 1024, 128, 25, 0), ("c64", 512, 512, 2, 1),
+    ("c128", 64, 128, 7, 0), ("c128", 64, 128, 64, 0), ("c128", 64, 128, 65, 0), ("c128", 128, 256, 9, 3)])
+def test_batches_of_images(gpu, prec, w, h, batch, pad):
+    """2D batches at the edges of where the row pass streams its stores and
+    the columns run in its tile order, on aligned and shifted buffers."""
+    import genfft_amd as G
+    p, ndt, tdt, tol = PREC[prec]
+    x = _rand((batch, h, w + pad), ndt, w + batch)
+    plan = G.Plan(C.GFFT_C2C_2D, w, precision=p, n2=h, batch=batch, in_stride=w + pad, out_stride=w + pad)
+    for inv, shift in ((False, 0), (True, 1)):
+        src = torch.zeros(x.size + shift, dtype=tdt, device=gpu)[shift:]
+        src.copy_(torch.from_numpy(x.reshape(-1)))
+        out = torch.full((x.size + shift,), 7 + 5j, dtype=tdt, device=gpu)[shift:]
+        plan.execute(src, out, inverse=inv)
+        got = out.cpu().numpy().reshape(x.shape)
+        v = x[:, :, :w].astype(np.complex128)
+        ref = np.fft.ifft2(v) * (w * h) if inv else np.fft.fft2(v)
+        assert O.rel_l2_rows(np.ascontiguousarray(got[:, :, :w]).reshape(batch, -1), ref.reshape(batch, -1)).max() <= tol(w * h)
+        if pad:
+            assert np.all(got[:, :, w:] == 7 + 5j)
