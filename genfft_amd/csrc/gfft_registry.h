@@ -31,7 +31,8 @@ struct KernelEntry {
     int wave;        // 1: one wavefront per row, lanes exchanged without LDS (wave_rows1024_kernel)
     int reg;         // 1: tile held in registers (reg_tile_kernel); its own pass twiddle table layout
     int many;        // tiles per CU from which this one is taken instead of the LDS tile of its width
-    int64_t most;    // cols: bytes a side up to which it is taken (0: any)
+    int64_t most;    // cols, cached: bytes a side up to which it is taken (0: any)
+    int64_t most_odd;  // cols: the same where rows of the matrix share lines
     int64_t least;   // cols: bytes a side from which it is taken
     int cols;        // 1: column tile for whole column transforms only; 2: but not those of complex 2D planes
     int cached;      // 1: row tile the planner takes for batches within the Infinity Cache
@@ -202,10 +203,11 @@ constexpr KernelEntry make_reg_many(int many)
 // A column tile of a whole column transform (not of a four-step pass), which
 // the planner picks by width (Builder::col_variant).
 template <typename T, int L, int M, int NT, int... RS>
-constexpr KernelEntry make_reg_cols(int64_t most = 0)
+constexpr KernelEntry make_reg_cols(int64_t most = 0, int64_t most_odd = 0)
 {
     KernelEntry e = make_reg_entry<T, L, M, NT, PAT_COL, PAT_COL, RS...>();
     e.most = most;
+    e.most_odd = most_odd;
     e.tune_only = 1;
     e.cols = 1;
     return e;
@@ -232,9 +234,10 @@ constexpr KernelEntry make_reg_narrow()
 
 // A row tile for batches that stay within the Infinity Cache.
 template <typename T, int L, int M, int NT, int... RS>
-constexpr KernelEntry make_reg_cached()
+constexpr KernelEntry make_reg_cached(int64_t most = 0)
 {
     KernelEntry e = make_reg_narrow<T, L, M, NT, RS...>();
+    e.most = most;
     e.cached = 1;
     return e;
 }

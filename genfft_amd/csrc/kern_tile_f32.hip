@@ -159,6 +159,22 @@ const KernelEntry kTable[] = {
     // 0.456 ms (128-byte runs instead of 64) ---
     make_reg_entry<T, 2048, 16, 1024, R_, C_, 16, 16, 8>(),
     make_reg_entry<T, 4096, 8, 1024, R_, C_, 16, 16, 16>(),
+    // --- more column tiles of whole column transforms.  Few rows, us, LDS ->
+    // register tile: 32 x 16 4.5 -> 3.3, x 32768 5.3 -> 4.5, 64 x 300 5.1 ->
+    // 3.8, x 32768 7.5 -> 6.5, 128 x 32768 12.2 -> 11.1, 256 x 4096 5.8 -> 5.2,
+    // x 131072 112 -> 104, 512 x 8192 14.3 -> 12.8, x 131072 243 -> 219.  The
+    // columns of images, read from the Infinity Cache, want the LDS tiles'
+    // fewer threads past 64 MiB (256 rows: 46.2 against 46.5 us there, 134.9
+    // against 130.8 at 160 MiB) and 32 MiB (512 rows: 26.9 against 29.3, 47.5
+    // against 45.5 at 64 MiB) ---
+    make_reg_cols<T, 32, 16, 64, 8, 4>(),
+    make_reg_cols<T, 32, 64, 256, 8, 4>(),
+    make_reg_cols<T, 64, 64, 512, 8, 8>(),
+    make_reg_cols<T, 128, 32, 512, 8, 2, 8>(),
+    make_reg_cols<T, 256, 16, 512, 8, 4, 8>((int64_t)64 << 20),
+    make_reg_cols_big<T, 256, 16, 512, 8, 4, 8>(0),
+    make_reg_cols<T, 512, 16, 1024, 8, 8, 8>((int64_t)32 << 20),
+    make_reg_cols_big<T, 512, 16, 1024, 8, 8, 8>(0),
 };
 // The 2^20 four-step's two pipelined passes paired in one launch (column pass
 // of chunk k, transposing row pass of chunk k - 1).

@@ -92,20 +92,39 @@ const KernelEntry kTable[] = {
     // --- column tiles held in registers: 2^22 x 16 four-step columns of 2048
     // 0.612 -> 0.529 ms, transposing rows 0.563 -> 0.427; whole columns: 512 x
     // 999 8.6 -> 6.8 us, 1024 x 4999 61 -> 48, 2048 x 2048 35 -> 28 (the
-    // pipelined 1024-row tile stays the four-step's: 0.469 against 0.496) ---
+    // pipelined 1024-row tile stays the four-step's: 0.469 against 0.496).  512
+    // rows whose pitch is no multiple of a line stay on the LDS tile past 128
+    // MiB: 16387 columns 66 against 70, 65539 249 against 290 ---
     make_reg_entry<T, 2048, 8, 1024, C_, C_, 16, 8, 16>(),
     make_reg_cols<T, 128, 8, 128, 8, 2, 8>(),
     make_reg_cols<T, 128, 16, 256, 8, 2, 8>(),
     make_reg_cols<T, 256, 4, 128, 8, 4, 8>(),
     make_reg_cols<T, 256, 8, 256, 8, 4, 8>(),
-    make_reg_cols<T, 512, 4, 256, 8, 8, 8>(),
-    make_reg_cols<T, 512, 8, 512, 8, 8, 8>(),
+    make_reg_cols<T, 512, 4, 256, 8, 8, 8>(0, (int64_t)128 << 20),
+    make_reg_cols<T, 512, 8, 512, 8, 8, 8>(0, (int64_t)128 << 20),
     make_reg_cols<T, 1024, 4, 256, 16, 4, 16>(),
     make_reg_cols<T, 1024, 8, 512, 16, 4, 16>(),
     make_reg_cols<T, 2048, 4, 512, 16, 8, 16>(),
     make_reg_cols<T, 2048, 8, 1024, 16, 8, 16>(),
     // --- transposing rows held in registers ---
     make_reg_entry<T, 2048, 8, 1024, R_, C_, 16, 16, 8>(),
+    // --- short rows and columns held in registers.  Rows, us, one row / 1 MiB /
+    // 32 MiB / 128 MiB, LDS -> register tile: 16 points 3.9 -> 3.0 / 5.5 -> 3.2 /
+    // 14.5 -> 14.6 / LDS, 32 4.7 -> 3.4 / 6.3 -> 3.6 / 16.1 -> 12.8 / 60 -> 57,
+    // 64 4.8 -> 3.5 / 6.4 -> 3.6 / 16.3 -> 12.6 / 61 -> 55, 128 4.6 -> 3.9 /
+    // 6.1 -> 4.1 / 16.0 -> 13.3 / 59 -> 56; 512 MiB (streaming loads) 64 points
+    // 195 -> 188, 128 193 -> 184, 32 195 -> 206 (LDS).  Columns: 32 rows x 1000
+    // 4.9 -> 3.4, x 262144 54 -> 41, 64 x 300 5.2 -> 3.6, x 131072 57 -> 41 ---
+    make_reg_cached<T, 16, 16, 64, 4, 4>((int64_t)64 << 20),
+    make_reg_cached<T, 32, 16, 64, 8, 4>(),
+    make_reg_cached<T, 64, 8, 64, 8, 8>(),
+    make_reg_wide<T, 64, 8, 64, 8, 8>(),
+    make_reg_cached<T, 128, 8, 128, 8, 2, 8>(),
+    make_reg_wide<T, 128, 8, 128, 8, 2, 8>(),
+    make_reg_cols<T, 32, 16, 64, 8, 4>(),
+    make_reg_cols<T, 32, 32, 128, 8, 4>(),
+    make_reg_cols<T, 64, 8, 64, 8, 8>(),
+    make_reg_cols<T, 64, 32, 256, 8, 8>(),
 };
 // The 2^20 four-step's two pipelined passes paired in one launch (column pass
 // of chunk k, transposing row pass of chunk k - 1).

@@ -529,7 +529,7 @@ struct Launch {
     RepackArgs rp{};
     // register-held tiles: stores not streamed (KernelEntry::fn_plain), and the
     // column-side runs cover whole 128-byte lines that no other tile touches
-    bool plain = false, own_lines = false;
+    bool plain = false, own_lines = false, row_order = false;
     int rr_mode = RR_R2C;
     const RowsEntry *rre = nullptr;
     int in_buf = B_IN, out_buf = B_OUT;
@@ -687,6 +687,12 @@ constexpr int64_t kDirtyLeast = (int64_t)4 << 20, kDirtyMost = (int64_t)24 << 20
 // 128 images, 8 MiB: 16.2 -> 13.5 us, 10 MiB 17.3 / 17.4), from 8 images on
 // (256 x 128 x 4: 9.4 us in the hardware's order, 10.0 in the rows').
 constexpr int64_t kOneL2Bytes = (int64_t)8 << 20;
+// Columns of up to kFewRows points keep that order too from kFewRowsLeast on (us,
+// hardware's order / neighbours on one XCD: c64 64 rows x 65536, pitch 512 KB,
+// 16.8 / 11.9, x 32768 6.4 / 6.5; 32 rows x 65536 7.6 / 6.6, x 32768 4.5 / 4.7,
+// x 1048576 108 / 101; 128 rows x 32768 11.1 / 12.7).
+constexpr int kFewRows = 64;
+constexpr int64_t kFewRowsLeast = (int64_t)16 << 20;
 // Row batches of at most this many bytes a side take the `cached` row tiles
 // (c64 2048 points on MI355X: 64 MiB 59.8 -> 55.8 us, 128 MiB 101.3 -> 101.4).
 constexpr int64_t kCachedBytes = (int64_t)128 << 20;
@@ -818,7 +824,9 @@ struct Builder {
             const bool row_pass = inp == PAT_ROW && outp == PAT_ROW && first && !last && p->d.kind == GFFT_C2C_2D;
             const bool dirty = row_pass && p->d.n2 <= kShortColumn && bytes > kDirtyLeast && bytes <= kDirtyMost;
             const bool near_rows = !first && in_buf == out_buf && bytes <= kOneL2Bytes && n_outer1 >= 8;
-            l.own_lines = (inp == PAT_COL || outp == PAT_COL) && in_lines && out_lines && !near_rows;
+            const bool short_cols = inp == PAT_COL && outp == PAT_COL && k->L <= kFewRows && bytes >= kFewRowsLeast;
+            l.own_lines = (inp == PAT_COL || outp == PAT_COL) && in_lines && out_lines;
+            l.row_order = near_rows || short_cols;
             l.plain = k->fn_plain &&
                       (!out_lines || near_rows || (!last && !dirty && bytes <= (row_pass ? kKeptRowBytes : kKeptBytes)));
         }
@@ -848,7 +856,13 @@ struct Builder {
     // default tiles would leave CUs idle; -1: the default.
     int cached_row_variant(int n, int64_t rows) const
     {
-        const int v = n * rows * (int64_t)csize <= kCachedBytes ? row_variant_of(prec, n, &KernelEntry::cached, store) : -1;
+        const int64_t bytes = n * rows * (int64_t)csize;
+        int v = bytes <= kCachedBytes ? row_variant_of(prec, n, &KernelEntry::cached, store) : -1;
+        if (v >= 0) {
+            int cnt = 0;
+            const int64_t most = tile_table(prec, store, &cnt)[v].most;
+            if (most && bytes > most) v = -1;
+        }
         return v >= 0 || store ? v : narrow_row_variant(prec, n, rows, p->num_cus);
     }
 
@@ -1045,7 +1059,7 @@ struct Builder {
     // complex 2D transform, which keep tiles of 4 columns at 4096 rows (8 columns
     // ran one 4096 x 4096 plane in 126 us instead of 145, FFTVert of 6000 such
     // columns in 110 instead of 156).
-    int col_variant(int L, int64_t cols, int64_t batch, bool plane) const
+    int col_variant(int L, int64_t cols, int64_t batch, bool plane, bool lines) const
     {
         if (store) return -1;
         int cnt = 0, best = -1;
@@ -1058,7 +1072,8 @@ struct Builder {
         const int64_t bytes = cols * L * batch * (int64_t)csize;
         for (int i = 0; i < cnt; i++)
             if (tab[i].cols && tab[i].cols <= (plane ? 1 : 2) && tab[i].L == L && bytes > tab[i].least - 1 &&
-                (!tab[i].most || bytes <= tab[i].most) && (best < 0 || better(tab[i].M, tab[best].M))) best = i;
+                (!tab[i].most || bytes <= tab[i].most) && (lines || !tab[i].most_odd || bytes <= tab[i].most_odd) &&
+                (best < 0 || better(tab[i].M, tab[best].M))) best = i;
         if (best < 0) return -1;
         const KernelEntry *d = find_tile(prec, L, PAT_COL, PAT_COL, 0, opts.pipe_mask);
         return d && d->M > tab[best].M && better(d->M, tab[best].M) ? -1 : best;
@@ -1086,7 +1101,9 @@ struct Builder {
         const int maxcol = max_len(prec, PAT_COL, PAT_COL, store);
         if (rows <= maxcol)
             return tile((int)rows, PAT_COL, PAT_COL, 0, in_buf, 0, out_buf, 0, cols, batch, 1, 0, in_dist, 1,
-                        in_pitch, 0, out_dist, 1, out_pitch, TW_NONE, 0, first, last, col_variant((int)rows, cols, batch, p->d.kind == GFFT_C2C_2D));
+                        in_pitch, 0, out_dist, 1, out_pitch, TW_NONE, 0, first, last, 
+                        col_variant((int)rows, cols, batch, p->d.kind == GFFT_C2C_2D,
+                                    (in_pitch | out_pitch) * (int64_t)csize % 128 == 0));
         // rows = A * B, sub-pass 1 over n2 (length B, rows n1 + A*n2) with
         // twiddle W_rows^(n1*k2) into scratch, sub-pass 2 over n1 (length A)
         // writing row k2 + B*k1.
@@ -2077,7 +2094,7 @@ int run_launches(const std::vector<Launch> &launches, int prec, int xcd_remap, c
             // 0.435 ms); interleaved tiles keep neighbours on one XCD
             const bool own = l.own_lines && ((uintptr_t)ip & 127) == 0 && ((uintptr_t)op & 127) == 0;
             const bool plain = l.plain || (l.own_lines && !own && l.k->fn_plain);
-            a.xcd_remap = p->xcd_remap && a.runs >= 0 && !own;
+            a.xcd_remap = p->xcd_remap && a.runs >= 0 && (!own || l.row_order);
             if (l.in_buf == B_IN) {
                 a.scale = scale.given;
                 a.scale_div = scale.div;

@@ -28,7 +28,8 @@ def _rand(shape, dt, seed):
     ("c64", 512, 5, 0, 1), ("c64", 1024, 3, 0, 0), ("c64", 1024, 1025, 1, 0), ("c64", 2048, 3, 5, 0),
     ("c64", 4096, 2, 0, 1), ("c64", 8192, 1, 0, 0), ("c64", 8192, 5, 3, 1), ("c64", 16384, 3, 0, 7), ("c64", 32768, 96, 0, 0),
     ("c64", 32768, 97, 5, 3),
-    ("c128", 256, 1, 0, 0), ("c128", 256, 13, 1, 0), ("c128", 512, 7, 0, 3), ("c128", 1024, 3, 1, 1),
+    ("c128", 16, 17, 0, 1), ("c128", 16, 4099, 0, 0), ("c128", 32, 15, 1, 0), ("c128", 64, 1, 0, 0), ("c128", 64, 4100, 3, 0),
+    ("c128", 128, 9, 0, 3), ("c128", 128, 4097, 0, 0), ("c128", 256, 1, 0, 0), ("c128", 256, 13, 1, 0), ("c128", 512, 7, 0, 3), ("c128", 1024, 3, 1, 1),
     ("c128", 2048, 2, 0, 0), ("c128", 4096, 3, 3, 0), ("c128", 8192, 2, 0, 1), ("c128", 16384, 96, 0, 0),
     ("c128", 16384, 97, 1, 5)])
 def test_rows_vs_oracle(gpu, prec, n, batch, pin, pout):
@@ -242,10 +243,13 @@ def test_scale_of_small_images(gpu, w, h, pitch):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("prec,n,cols,pin,pout", [
+    ("c64", 32, 1, 0, 0), ("c64", 32, 17, 0, 1), ("c64", 32, 16390, 0, 0), ("c64", 64, 16385, 1, 0), ("c64", 64, 32768, 0, 0),
+    ("c64", 128, 8200, 0, 0), ("c64", 256, 4112, 0, 1), ("c64", 512, 4100, 0, 0),
     ("c64", 64, 3, 0, 0), ("c64", 64, 17, 1, 0), ("c64", 128, 9, 0, 1), ("c64", 256, 1, 0, 0), ("c64", 256, 15, 2, 1),
     ("c64", 512, 7, 0, 0), ("c64", 512, 4111, 0, 1), ("c64", 1024, 5, 1, 1), ("c64", 1024, 1030, 0, 0),
     ("c64", 1024, 4097, 1, 0), ("c64", 2048, 3, 0, 0), ("c64", 2048, 1027, 0, 3), ("c64", 2048, 4112, 0, 0),
     ("c64", 4096, 2, 1, 0), ("c64", 4096, 1026, 0, 0), ("c64", 4096, 3100, 0, 2),
+    ("c128", 32, 1, 0, 0), ("c128", 32, 4098, 1, 0), ("c128", 32, 32768, 0, 0), ("c128", 64, 7, 0, 0), ("c128", 64, 8199, 0, 1),
     ("c128", 128, 3, 0, 1), ("c128", 128, 4100, 0, 0), ("c128", 256, 5, 1, 0), ("c128", 256, 2050, 0, 0), ("c128", 512, 3, 0, 0),
     ("c128", 512, 2056, 0, 0), ("c128", 1024, 2, 0, 1), ("c128", 1024, 2049, 0, 0), ("c128", 2048, 1, 0, 0),
     ("c128", 2048, 2049, 1, 1)])
