@@ -283,32 +283,25 @@ __device__ __forceinline__ void reg_store(cx<T> *p, const cx<T> *x, int stride)
     }
 }
 
-// INP / OUTP as in tile_fft_kernel.  The first pass walks along the rows when
-// they are read (INP = ROW), the later ones when they are written.
+// One tile: sequences s0 .. s0 + nvalid - 1 of transform o, read from `in` and
+// written to `out` (the transform's first elements).  INP / OUTP as in
+// tile_fft_kernel.  The first pass walks along the rows when they are read
+// (INP = ROW), the later ones when they are written.
 template <typename T, int L, int M, int NT, int INP, int OUTP, int HINT, int... RS>
-__global__ void __launch_bounds__(NT, 4) reg_tile_kernel(TileArgs a)
+__device__ __forceinline__ void reg_tile(T *plane, const TileArgs &a, const cx<T> *in, cx<T> *out, int s0, int o,
+                                         int nvalid, int tid)
 {
     constexpr int E = M * L / NT;
     constexpr int R1 = first_radix<RS...>(), RL = last_radix<RS...>();
     constexpr int CM = col_map<T, L, M, NT, RS...>();
     constexpr int MP = INP == PAT_ROW ? MAP_J : CM, MPL = OUTP == PAT_ROW ? MAP_J : CM;
     using G = PlaneGeom<T, L, M, R1, INP == PAT_ROW>;
-    __shared__ __align__(16) T plane[G::ELEMS];
-    const int tid = threadIdx.x;
-    const int tile = a.xcd_remap ? xcd_tile(blockIdx.x, gridDim.x) : (int)blockIdx.x;
-    const int t2 = tile / a.tiles_inner;
-    const int ti = tile - t2 * a.tiles_inner;
-    const int o2 = t2 / a.n_outer1;
-    const int o = t2 - o2 * a.n_outer1;
-    const int s0 = ti * M;
-    const int nvalid = min(M, a.n_inner - s0);
     cx<T> v[E];
     // HBM accesses: a uniform 64-bit base for each r plus one 32-bit
     // per-thread byte offset (the host admits only layouts it fits)
     {
         using A = Bfly<L, M, NT, MP, R1>;
         const bool sw = swap_in_of(a, o);
-        const cx<T> *in = reinterpret_cast<const cx<T> *>(a.in) + in_base(a, o2, o);
         in += INP == PAT_ROW ? (int64_t)s0 * a.in_inner : (int64_t)s0;
         const int64_t step = (INP == PAT_ROW ? (int64_t)A::LR : (int64_t)A::LR * a.in_elem) * (int64_t)sizeof(cx<T>);
         const char *ib = reinterpret_cast<const char *>(in);
@@ -343,7 +336,6 @@ __global__ void __launch_bounds__(NT, 4) reg_tile_kernel(TileArgs a)
     {
         using A = Bfly<L, M, NT, MPL, RL>;
         const bool sw = swap_out_of(a, o);
-        cx<T> *out = reinterpret_cast<cx<T> *>(a.out) + out_base(a, o2, o);
         out += OUTP == PAT_ROW ? (int64_t)s0 * a.out_inner : (int64_t)s0;
         const int64_t step = (OUTP == PAT_ROW ? (int64_t)A::LR : (int64_t)A::LR * a.out_elem) * (int64_t)sizeof(cx<T>);
         char *ob = reinterpret_cast<char *>(out);
@@ -389,6 +381,22 @@ __global__ void __launch_bounds__(NT, 4) reg_tile_kernel(TileArgs a)
             }
         }
     }
+}
+
+template <typename T, int L, int M, int NT, int INP, int OUTP, int HINT, int... RS>
+__global__ void __launch_bounds__(NT, 4) reg_tile_kernel(TileArgs a)
+{
+    using G = PlaneGeom<T, L, M, first_radix<RS...>(), INP == PAT_ROW>;
+    __shared__ __align__(16) T plane[G::ELEMS];
+    const int tile = a.xcd_remap ? xcd_tile(blockIdx.x, gridDim.x) : (int)blockIdx.x;
+    const int t2 = tile / a.tiles_inner;
+    const int ti = tile - t2 * a.tiles_inner;
+    const int o2 = t2 / a.n_outer1;
+    const int o = t2 - o2 * a.n_outer1;
+    const int s0 = ti * M;
+    reg_tile<T, L, M, NT, INP, OUTP, HINT, RS...>(
+        plane, a, reinterpret_cast<const cx<T> *>(a.in) + in_base(a, o2, o),
+        reinterpret_cast<cx<T> *>(a.out) + out_base(a, o2, o), s0, o, min(M, a.n_inner - s0), threadIdx.x);
 }
 
 // scale of a 16-bit transform from the largest |re| + |im| of its input: the

@@ -1,0 +1,192 @@
+// kern_xcd.hip -- both passes of a four-step in one persistent launch, each
+// transform on one XCD (see gfft_xcd.h).
+//
+// What bounds it: how many tiles are in flight.  Four workgroups of 256 threads
+// (or two of 512) hold 4 MB of tiles per XCD, as much as its L2, so the ring's
+// traffic goes on to the Infinity Cache (counters: reads and writes past the L2
+// are those of two launches), and a row tile must come that many tasks after its
+// column tiles not to wait: with `lag` 2 instead of 10, c64 2^16 x 2048 takes
+// 0.83-2.1 ms instead of 0.63.  MI355X against two launches, ms at 1 GiB / us at
+// 238 MiB: c64 2^16 0.78 -> 0.63 / 198 -> 167, 2^17 0.81 -> 0.73 / 206 -> 186,
+// 2^18 0.80 -> 0.67 / 200 -> 172; c128 2^15 0.81 -> 0.65 / 208 -> 169, 2^16 0.83
+// -> 0.64 / 212 -> 164, 2^17 0.88 -> 0.70 / 221 -> 182 (one pass over HBM at a
+// copy's rate: 0.39 / 91).  At 66 MiB 70 -> 71 us (c64 2^16) to 77 -> 70 (c128
+// 2^17): it is taken wherever its ring fits the two launches' workspace.
+#include "gfft_regtile.h"
+#include "gfft_xcd.h"
+
+namespace gfft {
+namespace {
+
+__device__ __forceinline__ uint32_t xcc_id()
+{
+    // s_getreg_b32 HW_REG_XCC_ID (20), 4 bits from bit 0
+    return (uint32_t)__builtin_amdgcn_s_getreg(20 | (3 << 11)) & (kXcds - 1);
+}
+
+// The counters of an XCD are only touched from it, so they live in its L2:
+// atomics of workgroup scope run there (the same at agent scope go past the L2,
+// and one at a time: 45 ns each).  The count of claimed transforms is everybody's.
+__device__ __forceinline__ uint32_t bump(uint32_t *p, uint32_t by = 1u)
+{
+    return __hip_atomic_fetch_add(p, by, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+// Waits until *p >= v.  An atomic of its own, for a load might find the CU's cache.
+__device__ __forceinline__ uint32_t await(uint32_t *p, uint32_t v)
+{
+    uint32_t zero = 0, x;
+    asm volatile("" : "+v"(zero));
+    while ((x = bump(p, zero)) < v) __builtin_amdgcn_s_sleep(1);
+    return x;
+}
+
+// Takes the next task of an XCD's queue.  Whoever takes a block's first task
+// claims the next transform of the batch for the block at once, after the block
+// before has its own, so an XCD's blocks run out of transforms in order.
+__device__ __forceinline__ uint32_t take(uint32_t *pop, uint32_t *blk, uint32_t *state, uint32_t per_block,
+                                         uint32_t blocks)
+{
+    const uint32_t j = bump(pop), b = j / per_block;
+    if (j % per_block == 0 && b < blocks) {
+        uint32_t *const w = blk + (int64_t)b * 4;
+        if (b) await(w - 4, 1u);
+        bump(w, __hip_atomic_fetch_add(state, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u);
+    }
+    return j;
+}
+
+template <int... RS>
+struct Radices {};
+
+template <typename T, int L, int M, int NT, int INP, int HINT, int... RS>
+__device__ __forceinline__ void tile_of(T *plane, const TileArgs &a, const cx<T> *in, cx<T> *out, int s0, int o,
+                                        int tid, Radices<RS...>)
+{
+    reg_tile<T, L, M, NT, INP, PAT_COL, HINT, RS...>(plane, a, in, out, s0, o, M, tid);
+}
+
+// Transform length N1 * N2: T1 column tiles (N1 points, M of the N2 columns),
+// then T2 row tiles (N2 points, M of the N1 rows, stored transposed).
+//
+// Each XCD has a queue: task j of block b = j / (T1 + T2) is a column tile of
+// its b-th transform or a row tile of its (b - lag)-th, handed out by one
+// counter.  The blocks claim transforms from the whole batch (take), so any
+// spread of workgroups over XCDs finishes it.  A task waits only for tasks
+// handed out before it (a row tile for its transform's column tiles, a column
+// tile for the row tiles that read the ring slot before), which their workgroups
+// run in order, and a claim only for the claim before it, so the earliest
+// unfinished task never waits and the grid always drains; a workgroup ends at
+// the first row task of a block past the batch, which no later task can be
+// inside, and holds no other task then.
+//
+// What one CU hands to another stays on one XCD, so no cache is written back:
+// stores are in the L2 once vmcnt is 0, and the readers drop their CU's own
+// cache (buffer_inv sc0) after they saw the count.
+template <typename T, int N1, int N2, int M, int NT, class RA, class RB>
+__global__ void __launch_bounds__(NT, 4) xcd_fft_kernel(XcdArgs x)
+{
+    constexpr int T1 = N2 / M, T2 = N1 / M;
+    constexpr int64_t N = (int64_t)N1 * N2;
+    constexpr int PLANE = N1 > N2 ? (N1 + N1 / 2) * M : (N2 + N2 / 2) * M;
+    __shared__ __align__(16) T plane[PLANE];
+    __shared__ int task[4];
+    const int tid = threadIdx.x;
+    const uint32_t q = xcc_id();
+    uint32_t *const pop = x.state + 32 * (1 + q);
+    uint32_t *const blk = x.state + 32 * (1 + kXcds) + (int64_t)q * x.blocks * 4;  // {claim, columns done, rows done, -}
+    cx<T> *const ring = reinterpret_cast<cx<T> *>(x.col.out) + (int64_t)q * x.ring * N;
+    uint32_t next = 0;  // thread 0: taken one task ahead
+    if (tid == 0) next = take(pop, blk, x.state, T1 + T2, x.blocks);
+    for (;;) {
+        if (tid == 0) {
+            const int b = (int)(next / (T1 + T2)), r = (int)(next % (T1 + T2));
+            const bool rows = r >= T1;
+            const int c = rows ? b - x.lag : b;
+            int g = -1;  // nothing to do
+            if (b >= x.blocks) {
+                g = -2;  // end
+            } else if (c >= 0) {
+                uint32_t *const w = blk + (int64_t)c * 4;
+                g = (int)await(w, 1u) - 1;
+                if (g >= x.batch) g = rows ? -2 : -1;
+                else if (rows) await(w + 1, T1);
+                else if (c >= x.ring) await(w - (int64_t)x.ring * 4 + 2, T2);
+            }
+            task[0] = g;
+            task[1] = r;
+            task[2] = c;
+            if (g != -2) next = take(pop, blk, x.state, T1 + T2, x.blocks);
+        }
+        __syncthreads();
+        const int g = task[0], r = task[1], c = task[2];
+        if (g == -2) break;
+        if (g >= 0) {
+            cx<T> *const slot = ring + (int64_t)(c % x.ring) * N;
+            if (r < T1) {
+                tile_of<T, N1, M, NT, PAT_COL, HINT_LD>(
+                    plane, x.col, reinterpret_cast<const cx<T> *>(x.col.in) + in_base(x.col, 0, g), slot, r * M, g, tid,
+                    RA{});
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            } else {
+                asm volatile("buffer_inv sc0" ::: "memory");
+                tile_of<T, N2, M, NT, PAT_ROW, HINT_ST>(
+                    plane, x.row, slot, reinterpret_cast<cx<T> *>(x.row.out) + out_base(x.row, 0, g), (r - T1) * M, g,
+                    tid, RB{});
+            }
+        }
+        __syncthreads();
+        if (tid == 0 && g >= 0) bump(blk + (int64_t)c * 4 + (r < T1 ? 1 : 2));
+    }
+}
+
+__global__ void __launch_bounds__(256) xcd_reset_kernel(uint32_t *state, int64_t words)
+{
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i < words) state[i] = 0u;
+}
+
+template <typename T, int N1, int N2, int M, int NT, int... RA, int... RB>
+constexpr XcdEntry make_xcd(int lag, int ring, int per_cu, Radices<RA...>, Radices<RB...>)
+{
+    constexpr int PLANE = N1 > N2 ? (N1 + N1 / 2) * M : (N2 + N2 / 2) * M;
+    static_assert(PlaneGeom<T, N1, M, first_radix<RA...>(), false>::ELEMS <= PLANE, "column plane");
+    static_assert(PlaneGeom<T, N2, M, first_radix<RB...>(), true>::ELEMS <= PLANE, "row plane");
+    XcdEntry e{};
+    e.prec = sizeof(T) == 8 ? 1 : 0;
+    for (int n = N1 * N2; n > 1; n >>= 1) e.lg++;
+    e.col = reg_shape<T, N1, M, NT, PAT_COL, PAT_COL, RA...>();
+    e.row = reg_shape<T, N2, M, NT, PAT_ROW, PAT_COL, RB...>();
+    e.NT = NT;
+    e.lds_bytes = PLANE * (int)sizeof(T);
+    e.lag = lag;
+    e.ring = ring;
+    e.per_cu = per_cu;
+    e.fn = &xcd_fft_kernel<T, N1, N2, M, NT, Radices<RA...>, Radices<RB...>>;
+    return e;
+}
+
+const XcdEntry kXcd[] = {
+    make_xcd<float, 256, 256, 16, 256>(10, 16, 4, Radices<16, 16>{}, Radices<16, 16>{}),
+    make_xcd<float, 256, 512, 16, 512>(5, 10, 2, Radices<8, 4, 8>{}, Radices<16, 2, 16>{}),
+    make_xcd<float, 512, 512, 16, 512>(5, 10, 2, Radices<16, 2, 16>{}, Radices<16, 2, 16>{}),
+    make_xcd<double, 128, 256, 8, 128>(6, 12, 4, Radices<8, 2, 8>{}, Radices<16, 16>{}),
+    make_xcd<double, 256, 256, 8, 128>(10, 16, 4, Radices<16, 16>{}, Radices<16, 16>{}),
+    make_xcd<double, 256, 512, 8, 256>(4, 8, 2, Radices<8, 4, 8>{}, Radices<16, 2, 16>{}),
+};
+
+}  // namespace
+
+const XcdEntry *xcd_entries(int *count)
+{
+    *count = (int)(sizeof(kXcd) / sizeof(kXcd[0]));
+    return kXcd;
+}
+
+hipError_t launch_xcd_reset(uint32_t *state, int64_t words, hipStream_t s)
+{
+    hipLaunchKernelGGL(xcd_reset_kernel, dim3((unsigned)((words + 255) / 256)), dim3(256), 0, s, state, words);
+    return hipGetLastError();
+}
+
+}  // namespace gfft

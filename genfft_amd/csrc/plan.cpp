@@ -44,6 +44,7 @@
 #include "gfft_misc.h"
 #include "gfft_r2c.h"
 #include "gfft_registry.h"
+#include "gfft_xcd.h"
 
 // Workspace of gfft_execute_noalloc: one static device array, instantiated
 // on every GPU the library's code object is loaded on and held until the
@@ -510,7 +511,7 @@ PlanOpts resolve_opts(int prec, int64_t n, const PlanOpts *forced)
 // ---------------------------------------------------------------------------
 enum BufId { B_IN = 0, B_OUT = 1, B_SCR = 2 };
 enum LaunchType { LT_TILE, LT_UNPACK, LT_PACK, LT_HFILL, LT_COPY, LT_MIX, LT_MIX_RESET, LT_R2C, LT_C2R, LT_RROWS,
-                  LT_REPACK, LT_DUAL };
+                  LT_REPACK, LT_DUAL, LT_XCD };
 
 // bytes of one complex element in memory
 size_t csize_of(int prec, int store) { return store ? 4 : (prec ? 16 : 8); }
@@ -547,7 +548,12 @@ struct Launch {
     int64_t in_off_b = 0, out_off_b = 0;
     bool vin_ok_b = false, vout_ok_b = false, first_b = false, last_b = false;
     int64_t split = 0;
-    bool reads(int buf) const { return in_buf == buf || (type == LT_DUAL && in_buf_b == buf); }
+    // LT_XCD: both passes of a four-step (k / ta the columns, kb / tb the
+    // transposing rows) with its ring and counters in the workspace
+    const XcdEntry *xe = nullptr;
+    XcdArgs xa{};
+    int64_t state_off = 0;  // bytes
+    bool reads(int buf) const { return in_buf == buf || (type == LT_DUAL && in_buf_b == buf) || (type == LT_XCD && buf == B_SCR); }
     bool writes(int buf) const { return out_buf == buf || (type == LT_DUAL && out_buf_b == buf); }
 };
 
@@ -634,8 +640,8 @@ struct gfft_plan_s {
     // place: in == out with equal byte distances in_step / out_step (batch
     // members, or rows) and in_step2 / out_step2 (2D images).
     bool overlap_hazard = false;
-    // The launches of the same plan without register-held long rows (none: it
-    // has none).  They read every input before they write an output wherever
+    // The launches of the same plan without register-held long rows and
+    // one-launch four-steps (none: it has none).  They read every input before they write an output wherever
     // the four-step does, so a call on overlapping buffers runs these, through
     // the workspace they were sized for, and no staging copy is needed.
     std::vector<gfft::Launch> alt;
@@ -712,7 +718,7 @@ struct Builder {
     int64_t scratch_elems = 0;  // complex elements of scratch needed
     int store = 0;              // 16-bit storage format (tile_kernels_f16 / _bf16), default shapes only
     bool no_long_rows = false;  // rows past the LDS tiles run as a four-step (gfft_plan_s::alt)
-    bool long_rows = false;     // set when some took the register-held tile
+    bool long_rows = false;     // set when some took the register-held tile, or a one-launch four-step (LT_XCD)
 
     void need_scratch(int64_t elems) { scratch_elems = std::max(scratch_elems, elems); }
 
@@ -939,6 +945,10 @@ struct Builder {
         const int64_t N1 = (int64_t)1 << l1, N2 = (int64_t)1 << l2;
         if (N1 > max_len(prec, PAT_COL, PAT_COL, store) || N2 > max_len(prec, PAT_ROW, PAT_COL, store))
             return fail(GFFT_ERR_UNSUPPORTED, "length %lld exceeds the two-pass limit", (long long)n);
+        if (const XcdEntry *e = xcd_entry(n, batch); e && in_buf != B_SCR && out_buf != B_SCR) {
+            long_rows = true;
+            return xcd_four_step(*e, batch, in_buf, in_off, in_dist, out_buf, out_off, out_dist, first, last);
+        }
         if (opts.dual && !store) {
             const int st = four_step_dual(n, N1, N2, batch, in_buf, in_off, in_dist, out_buf, out_off, out_dist, first,
                                           last);
@@ -971,6 +981,100 @@ struct Builder {
                       n, N2, 1, 0, out_dist, 1, N1, TW_NONE, 0, false, last);
             if (st) return st;
         }
+        return GFFT_OK;
+    }
+
+    // Workgroups of an XcdEntry's launch, and the scratch it keeps: a ring of
+    // transforms per XCD, then the counters.
+    int64_t xcd_grid(const XcdEntry &e, int64_t batch) const
+    {
+        int per_cu = e.per_cu;
+        int most = 0;
+        if (!dry && hipOccupancyMaxActiveBlocksPerMultiprocessor(&most, (const void *)e.fn, e.NT, 0) == hipSuccess)
+            per_cu = std::min(per_cu, std::max(1, most));
+        const int64_t tasks = batch * (e.col.L / e.col.M + e.row.L / e.row.M);
+        return std::min<int64_t>((int64_t)per_cu * std::max(1, p->num_cus), tasks);
+    }
+    int64_t xcd_scratch(const XcdEntry &e, int64_t batch, int64_t *state_off) const
+    {
+        *state_off = ((int64_t)kXcds * e.ring << e.lg) * (int64_t)csize;
+        return *state_off + 4 * xcd_state_words(xcd_blocks(batch, e.lag, (int64_t)e.per_cu * p->num_cus));
+    }
+
+    // Both passes of a four-step of length n in one launch, or null.
+    const XcdEntry *xcd_entry(int64_t n, int64_t batch) const
+    {
+        if (store || no_long_rows || opts.dual || opts.n1_log2 || opts.col_m || opts.row_m || opts.pipe_mask != 3 ||
+            opts.row_variant >= 0)
+            return nullptr;
+        int cnt = 0;
+        const XcdEntry *tab = xcd_entries(&cnt);
+        for (int i = 0; i < cnt; i++) {
+            if (tab[i].prec != prec || ((int64_t)1 << tab[i].lg) != n) continue;
+            int64_t off;
+            // within the workspace the two launches would have had
+            return xcd_scratch(tab[i], batch, &off) <= std::min(batch * n * (int64_t)csize, chunk_bytes()) ? &tab[i]
+                                                                                                           : nullptr;
+        }
+        return nullptr;
+    }
+
+    int xcd_four_step(const XcdEntry &e, int64_t batch, int in_buf, int64_t in_off, int64_t in_dist, int out_buf,
+                      int64_t out_off, int64_t out_dist, bool first, bool last)
+    {
+        const int64_t N1 = e.col.L, N2 = e.row.L, n = N1 * N2;
+        Launch l;
+        l.type = LT_XCD;
+        l.xe = &e;
+        l.k = &e.col;
+        l.kb = &e.row;
+        const int64_t bytes = xcd_scratch(e, batch, &l.state_off);
+        need_scratch((bytes + (int64_t)csize - 1) / (int64_t)csize);
+        l.grid = xcd_grid(e, batch);
+        if (batch * std::max(N1, N2) / e.col.M > INT32_MAX)
+            return fail(GFFT_ERR_UNSUPPORTED, "too many tiles (%lld)", (long long)batch);
+        auto fill = [&](TileArgs &a, const KernelEntry &k, int64_t seqs) {
+            a.n_inner = (int32_t)seqs;
+            a.tiles_inner = (int32_t)(seqs / k.M);
+            a.n_outer1 = (int32_t)batch;
+            a.n_tiles = (int32_t)(a.tiles_inner * batch);
+            TwTable t;
+            int st = get_pass_twiddles(p->device, k, &a.pass_tw, dry);
+            if (!st && k.gen_tw && !(st = get_two_level(p->device, k.L, &t, dry))) {
+                a.gen_lo = t.lo;
+                a.gen_hi = t.hi;
+            }
+            return st;
+        };
+        TileArgs &c = l.ta, &r = l.tb;
+        int st;
+        if ((st = fill(c, e.col, N2)) || (st = fill(r, e.row, N1))) return st;
+        TwTable t;
+        if ((st = get_two_level(p->device, n, &t, dry))) return st;
+        c.tw_mode = TW_INNER;
+        c.tw_lo = t.lo;
+        c.tw_hi = t.hi;
+        c.tw_mask = (uint32_t)t.mask;
+        c.tw_lo_bits = t.lo_bits;
+        c.in_outer = in_dist;
+        c.in_inner = c.out_inner = 1;
+        c.in_elem = c.out_elem = N2;
+        r.in_inner = N2;
+        r.in_elem = 1;
+        r.out_outer = out_dist;
+        r.out_inner = 1;
+        r.out_elem = N1;
+        l.xa.batch = (int32_t)batch;
+        l.xa.lag = e.lag;
+        l.xa.ring = e.ring;
+        l.xa.blocks = (int32_t)xcd_blocks(batch, e.lag, (int64_t)e.per_cu * p->num_cus);
+        l.in_buf = in_buf;
+        l.out_buf = out_buf;
+        l.in_off = in_off * (int64_t)csize;
+        l.out_off = out_off * (int64_t)csize;
+        l.first = first;
+        l.last = last;
+        p->launches.push_back(l);
         return GFFT_OK;
     }
 
@@ -1765,6 +1869,22 @@ int validate_list(const gfft_plan_s *p, const std::vector<Launch> &launches)
         case LT_TILE:
             if ((st = tile_inside(l.k, l.ta, l.in_buf, l.in_off, l.out_buf, l.out_off))) return st;
             break;
+        case LT_XCD: {
+            // the caller's sides, then the ring and the counters
+            const XcdEntry &e = *l.xe;
+            const TileArgs &c = l.ta, &r = l.tb;
+            const int64_t n = (int64_t)1 << e.lg;
+            if ((int64_t)e.col.L * e.row.L != n || c.n_inner != e.row.L || r.n_inner != e.col.L || e.ring <= e.lag ||
+                e.lds_bytes > 160 * 1024)
+                return fail(GFFT_ERR_UNSUPPORTED, "internal: launch %d shape", idx);
+            if ((st = inside(l.in_buf, l.in_off, ((l.xa.batch - 1) * c.in_outer + n) * cs, "column load"))) return st;
+            if ((st = inside(l.out_buf, l.out_off, ((l.xa.batch - 1) * r.out_outer + n) * cs, "row store"))) return st;
+            if ((st = inside(B_SCR, 0, (int64_t)kXcds * e.ring * n * cs, "ring"))) return st;
+            if (l.state_off < (int64_t)kXcds * e.ring * n * cs)
+                return fail(GFFT_ERR_UNSUPPORTED, "internal: launch %d counters", idx);
+            if ((st = inside(B_SCR, l.state_off, 4 * xcd_state_words(l.xa.blocks), "counters"))) return st;
+            break;
+        }
         case LT_DUAL: {
             if ((st = tile_inside(l.k, l.ta, l.in_buf, l.in_off, l.out_buf, l.out_off))) return st;
             if ((st = tile_inside(l.kb, l.tb, l.in_buf_b, l.in_off_b, l.out_buf_b, l.out_off_b))) return st;
@@ -1926,6 +2046,13 @@ int describe_launches(const std::vector<Launch> &launches, const std::string &he
                      role(l.kb, l.tb, l.in_buf_b, l.in_off_b, l.out_buf_b, l.out_off_b).c_str());
             break;
         }
+        case LT_XCD:
+            snprintf(line, sizeof(line), "xcd_four_step L=%d,%d M=%d NT=%d lds=%d grid=%lld batch=%d ring=%d lag=%d "
+                     "in=%s+%lld out=%s+%lld in_dist=%lld out_dist=%lld first=%d last=%d\n", l.k->L, l.kb->L, l.k->M,
+                     l.xe->NT, l.xe->lds_bytes, (long long)l.grid, l.xa.batch, l.xa.ring, l.xa.lag, bn[l.in_buf],
+                     (long long)l.in_off, bn[l.out_buf], (long long)l.out_off, (long long)l.ta.in_outer,
+                     (long long)l.tb.out_outer, (int)l.first, (int)l.last);
+            break;
         case LT_UNPACK:
         case LT_PACK:
             snprintf(line, sizeof(line), "%s n=%lld batch=%lld in=%s+%lld out=%s+%lld in_dist=%lld out_dist=%lld "
@@ -2106,6 +2233,24 @@ int run_launches(const std::vector<Launch> &launches, int prec, int xcd_remap, c
             void *args[] = {&a};
             HIP_TRY(hipExtLaunchKernel((const void *)(plain ? l.k->fn_plain : l.k->fn), dim3((unsigned)l.grid),
                                        dim3(l.k->NT), args, 0, s, nullptr, tail, 0));
+            if (tail && stopped) *stopped = true;
+            break;
+        }
+        case LT_XCD: {
+            XcdArgs a = l.xa;
+            a.col = l.ta;
+            a.row = l.tb;
+            a.col.in = ip;
+            a.col.out = scratch;
+            a.row.in = scratch;
+            a.row.out = op;
+            a.col.swap_in = inv && l.first;
+            a.row.swap_out = inv && l.last;
+            a.state = (uint32_t *)((char *)scratch + l.state_off);
+            HIP_TRY(launch_xcd_reset(a.state, xcd_state_words(a.blocks), s));
+            void *args[] = {&a};
+            HIP_TRY(hipExtLaunchKernel((const void *)l.xe->fn, dim3((unsigned)l.grid), dim3(l.xe->NT), args, 0, s,
+                                       nullptr, tail, 0));
             if (tail && stopped) *stopped = true;
             break;
         }
@@ -2424,6 +2569,16 @@ int build_batch(gfft_batch_plan_s *p)
             set_jobs(c.first, true, true);
             continue;
         }
+        if (const XcdEntry *e = b.xcd_entry(L, c.count)) {
+            if ((st = b.xcd_four_step(*e, c.count, B_IN, 0, 0, B_OUT, 0, 0, false, false))) return st;
+            Launch &l = tmp.launches.back();
+            l.ta.job_in = p->d_job_in;
+            l.tb.job_out = p->d_job_out;
+            l.ta.job_inv = l.tb.job_inv = p->d_job_inv;
+            l.ta.job_first = l.tb.job_first = (int32_t)c.first;
+            l.ta.job_swap_in = l.tb.job_swap_out = 1;
+            continue;
+        }
         int l1, l2;
         rows_split(prec, 0, c.lg, L * c.count * (int64_t)cs, &l1, &l2, b.opts.n1_log2);
         const int64_t N1 = (int64_t)1 << l1, N2 = (int64_t)1 << l2;
@@ -2445,6 +2600,11 @@ int build_batch(gfft_batch_plan_s *p)
     const int64_t scratch_bytes = b.scratch_elems * (int64_t)cs;
     for (const Launch &l : tmp.launches) {
         const TileArgs &a = l.ta;
+        if (l.type == LT_XCD) {
+            if (l.state_off + 4 * xcd_state_words(l.xa.blocks) > scratch_bytes)
+                return fail(GFFT_ERR_UNSUPPORTED, "internal: batch launch leaves the scratch buffer");
+            continue;
+        }
         const int64_t n_outer2 = a.n_tiles / ((int64_t)a.tiles_inner * a.n_outer1);
         for (int side = 0; side < 2; side++) {
             if ((side ? l.out_buf : l.in_buf) != B_SCR) continue;
@@ -2524,6 +2684,10 @@ std::vector<PlanOpts> tune_candidates(int prec, int64_t n)
             o.row_variant = i;
             out.push_back(o);
         }
+    int nx = 0;
+    const XcdEntry *xcd = xcd_entries(&nx);
+    for (int i = 0; i < nx; i++)  // untuned: both passes in one launch, batch permitting
+        if (xcd[i].prec == prec && ((int64_t)1 << xcd[i].lg) == n) out.push_back(PlanOpts{});
     const int lg = ilog2(n), maxcol = max_len(prec, PAT_COL, PAT_COL), maxtr = max_len(prec, PAT_ROW, PAT_COL);
     for (int l1 = 1; l1 < lg; l1++) {
         const int64_t N1 = (int64_t)1 << l1, N2 = (int64_t)1 << (lg - l1);

@@ -1,0 +1,123 @@
+"""Four-steps that run both passes in one launch, a transform per XCD
+(genfft_amd/csrc/kern_xcd.hip), against numpy's float64 transform at the
+library's bounds (rel-L2 2e-7*log2 N complex64, 1e-15*log2 N complex128)."""
+import numpy as np
+import pytest
+import torch
+
+import oracle_lib as O
+from genfft_amd import _capi as C
+from test_capi_cpu import desc, explain
+
+PREC = {"c64": (C.GFFT_F32, np.complex64, torch.complex64, O.tol_c64),
+        "c128": (C.GFFT_F64, np.complex128, torch.complex128, O.tol_c128)}
+SHAPES = [("c64", 1 << 16, 131, 5, 3), ("c64", 1 << 16, 150, 0, 0), ("c64", 1 << 17, 82, 0, 1), ("c64", 1 << 18, 81, 1, 0),
+          ("c128", 1 << 15, 98, 0, 0), ("c128", 1 << 15, 203, 1, 3), ("c128", 1 << 16, 130, 0, 0), ("c128", 1 << 17, 66, 0, 1)]
+
+
+def test_route(monkeypatch):
+    """Taken from where the ring fits the two launches' workspace, which stays
+    what it was; by untuned complex batches only."""
+    for prec, n, least in ((0, 1 << 16, 129), (0, 1 << 17, 81), (0, 1 << 18, 81), (1, 1 << 15, 97), (1, 1 << 16, 129),
+                           (1, 1 << 17, 65)):
+        for batch in (least - 1, least + 1):
+            st, text = explain(desc(C.GFFT_C2C, prec, n, 0, batch))
+            head = text.split("on overlapping buffers:")
+            assert st == 0 and ("xcd_four_step" in head[0]) == (batch > least)
+            assert f"scratch_bytes={batch * n * (8 << prec)}\n" in head[0]
+            if batch > least:
+                assert "xcd" not in head[1] and head[1].count("tile L=") == 2
+    for d in (desc(C.GFFT_C2C, C.GFFT_F16, 1 << 16, 0, 600), desc(C.GFFT_C2C, 0, 1 << 19, 0, 200),
+              desc(C.GFFT_C2C, 0, 1 << 16, 0, 600, flags=C.GFFT_FLAG_NO_WORKSPACE)):
+        assert "xcd" not in explain(d)[1]
+    monkeypatch.setenv("GFFT_N1_LOG2", "7")
+    assert "xcd" not in explain(desc(C.GFFT_C2C, 0, 1 << 16, 0, 600))[1]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("prec,n,batch,pin,pout", SHAPES)
+def test_vs_float64(gpu, prec, n, batch, pin, pout):
+    import genfft_amd as G
+    p, ndt, tdt, tol = PREC[prec]
+    rng = np.random.default_rng(n + batch)
+    x = (rng.uniform(-1, 1, (batch, n + pin)) + 1j * rng.uniform(-1, 1, (batch, n + pin))).astype(ndt)
+    tx = torch.from_numpy(x).to(gpu)
+    plan = G.Plan(C.GFFT_C2C, n, precision=p, batch=batch, in_dist=n + pin, out_dist=n + pout)
+    assert "xcd_four_step" in plan.describe()
+    v = x[:, :n].astype(np.complex128)
+    for inv in (False, True):
+        ref = np.fft.ifft(v) * n if inv else np.fft.fft(v)
+        for _ in range(2):  # the counters start over
+            y = torch.full((batch, n + pout), 7 + 5j, dtype=tdt, device=gpu)
+            plan.execute(tx, y, inverse=inv)
+            h = y.cpu().numpy()
+            assert O.rel_l2_rows(np.ascontiguousarray(h[:, :n]), ref).max() <= tol(n)
+            if pout:
+                assert np.all(h[:-1, n:] == 7 + 5j)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shift", [0, 1, 3 << 16])
+def test_overlapping_buffers(gpu, shift):
+    """In place, and with the output shifted against the input (two launches)."""
+    import genfft_amd as G
+    n, batch = 1 << 16, 131
+    buf = torch.zeros(batch * n + shift, dtype=torch.complex64, device=gpu)
+    rng = np.random.default_rng(shift)
+    x = (rng.uniform(-1, 1, (batch, n)) + 1j * rng.uniform(-1, 1, (batch, n))).astype(np.complex64)
+    buf[:batch * n].copy_(torch.from_numpy(x.reshape(-1)))
+    out = buf[shift:shift + batch * n]
+    G.Plan(C.GFFT_C2C, n, batch=batch).execute(buf[:batch * n], out)
+    h = out.cpu().numpy().reshape(batch, n)
+    assert O.rel_l2_rows(h, np.fft.fft(x.astype(np.complex128))).max() <= O.tol_c64(n)
+
+
+@pytest.mark.gpu
+def test_two_streams_and_a_graph(gpu):
+    """One plan from two streams, whose calls share its ring, and replays."""
+    import genfft_amd as G
+    n, batch = 1 << 15, 100
+    g = torch.Generator().manual_seed(3)
+    x = [torch.randn(batch, n, dtype=torch.complex128, generator=g).to(gpu) for _ in range(2)]
+    y = [torch.empty_like(t) for t in x]
+    ref = [torch.fft.fft(t.cpu()) for t in x]
+    plan = G.Plan(C.GFFT_C2C, n, precision=C.GFFT_F64, batch=batch)
+    side = [torch.cuda.Stream(), torch.cuda.Stream()]
+    torch.cuda.synchronize()
+    for k in range(4):
+        with torch.cuda.stream(side[k % 2]):
+            plan.execute(x[k % 2], y[k % 2])
+    torch.cuda.synchronize()
+    for a, b in zip(y, ref):
+        assert float(((a.cpu() - b).norm(dim=1) / b.norm(dim=1)).max()) <= O.tol_c128(n)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        plan.execute(x[0], y[0])
+    for k in range(3):
+        y[0].zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert float(((y[0].cpu() - ref[0]).norm(dim=1) / ref[0].norm(dim=1)).max()) <= O.tol_c128(n)
+
+
+@pytest.mark.gpu
+def test_in_an_uneven_batch(gpu):
+    import genfft_amd as G
+    rng = np.random.default_rng(9)
+    sizes = np.concatenate([np.full(140, 1 << 16), np.full(20, 1 << 12), np.full(3, 1 << 17)])
+    rng.shuffle(sizes)
+    offs = np.concatenate([[1], 1 + np.cumsum(sizes + rng.integers(0, 3, len(sizes)))[:-1]])
+    dirs = rng.integers(0, 2, len(sizes))
+    total = int(offs[-1] + sizes[-1])
+    x = torch.from_numpy((rng.uniform(-1, 1, total) + 1j * rng.uniform(-1, 1, total)).astype(np.complex64))
+    plan = G.UnevenBatch(sizes.tolist(), offs.tolist(), offs.tolist(), [bool(d) for d in dirs], torch.complex64)
+    assert "xcd_four_step" in plan.describe()
+    tx = x.to(gpu)
+    for _ in range(2):
+        y = torch.zeros_like(tx)
+        plan.execute(tx, y)
+        h = y.cpu().numpy()
+        for n, o, d in zip(sizes, offs, dirs):
+            v = x.numpy()[o:o + n].astype(np.complex128)
+            ref = np.fft.ifft(v) * n if d else np.fft.fft(v)
+            assert O.rel_l2_rows(h[o:o + n][None], ref[None]).max() <= O.tol_c64(n)
