@@ -105,12 +105,15 @@ def parse():
 
 def tile_launches(text):
     """The launch lines of a plan description, each with its launch index
-    (every line after the `plan` header is one launch, in execution order)."""
+    (every line after the `plan` header is one launch, in execution order, up
+    to those a call on overlapping buffers would run)."""
     out = []
     idx = -1
     for ln in text.splitlines():
         if not ln.strip() or ln.startswith("plan "):
             continue
+        if ln.startswith("on overlapping buffers"):
+            break  # the launches of another route
         idx += 1
         if ln.startswith("dual"):
             # two tile passes in one launch: "dual ... | <role A fields> | <role B fields>"
@@ -121,7 +124,7 @@ def tile_launches(text):
             f["index"] = idx
             out.append(f)
             continue
-        if not ln.startswith(("tile", "r2c_rows_unpack", "c2r_pack_cols", "real_rows", "unpack", "pack", "hfill",
+        if not ln.startswith(("tile", "xcd_four_step", "r2c_rows_unpack", "c2r_pack_cols", "real_rows", "unpack", "pack", "hfill",
                               "copy", "repack")):
             continue
         f = dict(kv.split("=", 1) for kv in ln.split()[1:] if "=" in kv)
@@ -762,6 +765,11 @@ def main():
             # each role reads and writes its own elements
             key = "dual " + " + ".join(_tile_key(r) for r in l["roles"])
             elems = sum(_tile_elems(r) for r in l["roles"])
+        elif l["kind"] == "xcd_four_step":
+            # both passes of a transform: its input read and its output written once
+            n1, n2_ = (int(v) for v in l["L"].split(","))
+            key = f"xcd four-step L={n1},{n2_} M={l['M']}"
+            elems = int(l["batch"]) * n1 * n2_
         elif l["kind"] == "real_rows":
             # rows of n = 2L reals <-> bins in one pass (unpack / pack fused)
             key = f"real rows {l['mode']} L={l['L']} M={l['M']}"

@@ -7,11 +7,15 @@
 // are those of two launches), and a row tile must come that many tasks after its
 // column tiles not to wait: with `lag` 2 instead of 10, c64 2^16 x 2048 takes
 // 0.83-2.1 ms instead of 0.63.  MI355X against two launches, ms at 1 GiB / us at
-// 238 MiB: c64 2^16 0.78 -> 0.63 / 198 -> 167, 2^17 0.81 -> 0.73 / 206 -> 186,
-// 2^18 0.80 -> 0.67 / 200 -> 172; c128 2^15 0.81 -> 0.65 / 208 -> 169, 2^16 0.83
-// -> 0.64 / 212 -> 164, 2^17 0.88 -> 0.70 / 221 -> 182 (one pass over HBM at a
-// copy's rate: 0.39 / 91).  At 66 MiB 70 -> 71 us (c64 2^16) to 77 -> 70 (c128
-// 2^17): it is taken wherever its ring fits the two launches' workspace.
+// 238 MiB: c64 2^16 0.75 -> 0.63 / 198 -> 170, 2^17 0.80 -> 0.64 / 205 -> 168,
+// 2^18 0.78 -> 0.64 / 201 -> 174, 2^19 0.86 -> 0.66 / 211 -> 178, 2^20 0.81 -> 0.64 /
+// 215 -> 187; c128 2^15 0.80 -> 0.65 / 208 -> 180, 2^16 0.81 -> 0.64 / 210 -> 165,
+// 2^17 0.85 -> 0.70 / 219 -> 181, 2^18 0.84 -> 0.68 / 213 -> 191 (one pass over HBM
+// at a copy's rate: 0.39 / 91).  Near the smallest batches: c64 2^16 x 130 68 -> 69
+// us, 2^17 x 81 84 -> 73, 2^20 x 25 191 -> 175, c128 2^18 x 41 156 -> 143: it is
+// taken wherever its ring fits the workspace the two launches would have.  Longer
+// transforms' rings leave the Infinity Cache; c128 2^19 gained 4% at 1 GiB and
+// nothing at 238 MiB and stays on two launches.
 #include "gfft_regtile.h"
 #include "gfft_xcd.h"
 
@@ -59,6 +63,15 @@ __device__ __forceinline__ uint32_t take(uint32_t *pop, uint32_t *blk, uint32_t 
 template <int... RS>
 struct Radices {};
 
+// Scalars of the exchange plane, for either pass.
+template <typename T, int N1, int N2, int M, int... RA, int... RB>
+constexpr int plane_of(Radices<RA...>, Radices<RB...>)
+{
+    constexpr int a = PlaneGeom<T, N1, M, first_radix<RA...>(), false>::ELEMS;
+    constexpr int b = PlaneGeom<T, N2, M, first_radix<RB...>(), true>::ELEMS;
+    return a > b ? a : b;
+}
+
 template <typename T, int L, int M, int NT, int INP, int HINT, int... RS>
 __device__ __forceinline__ void tile_of(T *plane, const TileArgs &a, const cx<T> *in, cx<T> *out, int s0, int o,
                                         int tid, Radices<RS...>)
@@ -83,13 +96,12 @@ __device__ __forceinline__ void tile_of(T *plane, const TileArgs &a, const cx<T>
 // What one CU hands to another stays on one XCD, so no cache is written back:
 // stores are in the L2 once vmcnt is 0, and the readers drop their CU's own
 // cache (buffer_inv sc0) after they saw the count.
-template <typename T, int N1, int N2, int M, int NT, class RA, class RB>
-__global__ void __launch_bounds__(NT, 4) xcd_fft_kernel(XcdArgs x)
+template <typename T, int N1, int N2, int M, int NT, int WPE, class RA, class RB>
+__global__ void __launch_bounds__(NT, WPE) xcd_fft_kernel(XcdArgs x)
 {
     constexpr int T1 = N2 / M, T2 = N1 / M;
     constexpr int64_t N = (int64_t)N1 * N2;
-    constexpr int PLANE = N1 > N2 ? (N1 + N1 / 2) * M : (N2 + N2 / 2) * M;
-    __shared__ __align__(16) T plane[PLANE];
+    __shared__ __align__(16) T plane[plane_of<T, N1, N2, M>(RA{}, RB{})];
     __shared__ int task[4];
     const int tid = threadIdx.x;
     const uint32_t q = xcc_id();
@@ -146,33 +158,39 @@ __global__ void __launch_bounds__(256) xcd_reset_kernel(uint32_t *state, int64_t
     if (i < words) state[i] = 0u;
 }
 
-template <typename T, int N1, int N2, int M, int NT, int... RA, int... RB>
+// WPE: waves per SIMD the registers are budgeted for
+template <typename T, int N1, int N2, int M, int NT, int WPE, int... RA, int... RB>
 constexpr XcdEntry make_xcd(int lag, int ring, int per_cu, Radices<RA...>, Radices<RB...>)
 {
-    constexpr int PLANE = N1 > N2 ? (N1 + N1 / 2) * M : (N2 + N2 / 2) * M;
-    static_assert(PlaneGeom<T, N1, M, first_radix<RA...>(), false>::ELEMS <= PLANE, "column plane");
-    static_assert(PlaneGeom<T, N2, M, first_radix<RB...>(), true>::ELEMS <= PLANE, "row plane");
     XcdEntry e{};
     e.prec = sizeof(T) == 8 ? 1 : 0;
     for (int n = N1 * N2; n > 1; n >>= 1) e.lg++;
     e.col = reg_shape<T, N1, M, NT, PAT_COL, PAT_COL, RA...>();
     e.row = reg_shape<T, N2, M, NT, PAT_ROW, PAT_COL, RB...>();
     e.NT = NT;
-    e.lds_bytes = PLANE * (int)sizeof(T);
+    e.lds_bytes = plane_of<T, N1, N2, M>(Radices<RA...>{}, Radices<RB...>{}) * (int)sizeof(T);
     e.lag = lag;
     e.ring = ring;
     e.per_cu = per_cu;
-    e.fn = &xcd_fft_kernel<T, N1, N2, M, NT, Radices<RA...>, Radices<RB...>>;
+    e.fn = &xcd_fft_kernel<T, N1, N2, M, NT, WPE, Radices<RA...>, Radices<RB...>>;
     return e;
 }
 
+// Where a length is listed twice, the first whose ring fits the workspace.
+// Radix 32 * 16 and 32 * 32 with 16 or 32 elements per thread against more
+// threads of fewer, ms at 1 GiB: 2^17 0.63 / 0.73, 2^18 0.64 / 0.67, 2^19 0.66 /
+// 0.91, 2^20 0.64 / 0.84 (16 * 4 * 16).
 const XcdEntry kXcd[] = {
-    make_xcd<float, 256, 256, 16, 256>(10, 16, 4, Radices<16, 16>{}, Radices<16, 16>{}),
-    make_xcd<float, 256, 512, 16, 512>(5, 10, 2, Radices<8, 4, 8>{}, Radices<16, 2, 16>{}),
-    make_xcd<float, 512, 512, 16, 512>(5, 10, 2, Radices<16, 2, 16>{}, Radices<16, 2, 16>{}),
-    make_xcd<double, 128, 256, 8, 128>(6, 12, 4, Radices<8, 2, 8>{}, Radices<16, 16>{}),
-    make_xcd<double, 256, 256, 8, 128>(10, 16, 4, Radices<16, 16>{}, Radices<16, 16>{}),
-    make_xcd<double, 256, 512, 8, 256>(4, 8, 2, Radices<8, 4, 8>{}, Radices<16, 2, 16>{}),
+    make_xcd<float, 256, 256, 16, 256, 4>(10, 16, 4, Radices<16, 16>{}, Radices<16, 16>{}),
+    make_xcd<float, 256, 512, 16, 256, 4>(5, 10, 4, Radices<16, 16>{}, Radices<32, 16>{}),
+    make_xcd<float, 512, 512, 16, 256, 4>(6, 10, 4, Radices<32, 16>{}, Radices<32, 16>{}),
+    make_xcd<float, 1024, 512, 16, 512, 4>(3, 6, 2, Radices<32, 32>{}, Radices<16, 2, 16>{}),
+    make_xcd<float, 1024, 1024, 16, 512, 4>(2, 4, 2, Radices<32, 32>{}, Radices<32, 32>{}),
+    make_xcd<float, 1024, 1024, 16, 512, 4>(1, 3, 2, Radices<32, 32>{}, Radices<32, 32>{}),
+    make_xcd<double, 128, 256, 8, 128, 3>(6, 12, 4, Radices<8, 2, 8>{}, Radices<16, 16>{}),
+    make_xcd<double, 256, 256, 8, 128, 3>(10, 16, 4, Radices<16, 16>{}, Radices<16, 16>{}),
+    make_xcd<double, 256, 512, 8, 256, 2>(4, 8, 2, Radices<8, 4, 8>{}, Radices<16, 2, 16>{}),
+    make_xcd<double, 512, 512, 8, 256, 2>(2, 5, 2, Radices<16, 2, 16>{}, Radices<16, 2, 16>{}),
 };
 
 }  // namespace

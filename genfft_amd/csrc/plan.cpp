@@ -289,6 +289,7 @@ struct PlanOpts {
     int col_runs = -2;     // persistent column passes' tile order (TileArgs::runs; -2: by element size)
     int row_runs = 0;      // persistent transposing-row and single passes' tile order
     int dual = 0;          // four-step batches in chunks, column pass of chunk k beside row pass of k - 1
+    int two_launches = 0;  // no one-launch four-step
 };
 
 // Picks the tile kernel for (precision, L, patterns): the registry entry
@@ -502,7 +503,10 @@ PlanOpts resolve_opts(int prec, int64_t n, const PlanOpts *forced)
     if (getenv("GFFT_R2C_FUSE")) o.r2c_fuse = (int)env_int("GFFT_R2C_FUSE", 1);
     if (getenv("GFFT_COL_RUNS")) o.col_runs = (int)env_int("GFFT_COL_RUNS", -2);
     if (getenv("GFFT_ROW_RUNS")) o.row_runs = (int)env_int("GFFT_ROW_RUNS", 0);
-    if (getenv("GFFT_DUAL")) o.dual = (int)env_int("GFFT_DUAL", 0);
+    if (getenv("GFFT_DUAL")) {  // 0: the two passes one after the other
+        o.dual = (int)env_int("GFFT_DUAL", 0);
+        o.two_launches = 1;
+    }
     return o;
 }
 
@@ -1004,7 +1008,7 @@ struct Builder {
     // Both passes of a four-step of length n in one launch, or null.
     const XcdEntry *xcd_entry(int64_t n, int64_t batch) const
     {
-        if (store || no_long_rows || opts.dual || opts.n1_log2 || opts.col_m || opts.row_m || opts.pipe_mask != 3 ||
+        if (store || no_long_rows || opts.dual || opts.two_launches || opts.n1_log2 || opts.col_m || opts.row_m || opts.pipe_mask != 3 ||
             opts.row_variant >= 0)
             return nullptr;
         int cnt = 0;
@@ -1013,8 +1017,7 @@ struct Builder {
             if (tab[i].prec != prec || ((int64_t)1 << tab[i].lg) != n) continue;
             int64_t off;
             // within the workspace the two launches would have had
-            return xcd_scratch(tab[i], batch, &off) <= std::min(batch * n * (int64_t)csize, chunk_bytes()) ? &tab[i]
-                                                                                                           : nullptr;
+            if (xcd_scratch(tab[i], batch, &off) <= std::min(batch * n * (int64_t)csize, chunk_bytes())) return &tab[i];
         }
         return nullptr;
     }
@@ -2767,6 +2770,10 @@ int gfft_autotune(int precision, int64_t n, int64_t batch, int reps, char *repor
         if (hipDeviceGetAttribute(&p->num_cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
             p->num_cus = 256;
         if (build_plan(p.get(), false, &o) || validate(p.get())) continue;  // candidate not plannable
+        // the untuned plan counts where it is none of the other candidates
+        if (n > max_len(precision, PAT_ROW, PAT_ROW) && !o.n1_log2 && o.row_variant < 0 &&
+            p->launches[0].type != LT_XCD)
+            continue;
         if (p->scratch_bytes && hipMalloc(&p->scratch, p->scratch_bytes) != hipSuccess) continue;
         float ms = 0;
         int r = run(p.get(), in, out, GFFT_FORWARD, s);  // warm-up

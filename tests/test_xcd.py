@@ -12,14 +12,16 @@ from test_capi_cpu import desc, explain
 PREC = {"c64": (C.GFFT_F32, np.complex64, torch.complex64, O.tol_c64),
         "c128": (C.GFFT_F64, np.complex128, torch.complex128, O.tol_c128)}
 SHAPES = [("c64", 1 << 16, 131, 5, 3), ("c64", 1 << 16, 150, 0, 0), ("c64", 1 << 17, 82, 0, 1), ("c64", 1 << 18, 81, 1, 0),
-          ("c128", 1 << 15, 98, 0, 0), ("c128", 1 << 15, 203, 1, 3), ("c128", 1 << 16, 130, 0, 0), ("c128", 1 << 17, 66, 0, 1)]
+          ("c128", 1 << 15, 98, 0, 0), ("c128", 1 << 15, 203, 1, 3), ("c128", 1 << 16, 130, 0, 0), ("c128", 1 << 17, 66, 0, 1),
+          ("c64", 1 << 19, 50, 1, 0), ("c64", 1 << 20, 25, 0, 0), ("c64", 1 << 20, 33, 0, 1),
+          ("c128", 1 << 18, 42, 0, 1)]
 
 
 def test_route(monkeypatch):
     """Taken from where the ring fits the two launches' workspace, which stays
     what it was; by untuned complex batches only."""
     for prec, n, least in ((0, 1 << 16, 129), (0, 1 << 17, 81), (0, 1 << 18, 81), (1, 1 << 15, 97), (1, 1 << 16, 129),
-                           (1, 1 << 17, 65)):
+                           (1, 1 << 17, 65), (0, 1 << 19, 49), (0, 1 << 20, 25), (1, 1 << 18, 41)):
         for batch in (least - 1, least + 1):
             st, text = explain(desc(C.GFFT_C2C, prec, n, 0, batch))
             head = text.split("on overlapping buffers:")
@@ -27,7 +29,7 @@ def test_route(monkeypatch):
             assert f"scratch_bytes={batch * n * (8 << prec)}\n" in head[0]
             if batch > least:
                 assert "xcd" not in head[1] and head[1].count("tile L=") == 2
-    for d in (desc(C.GFFT_C2C, C.GFFT_F16, 1 << 16, 0, 600), desc(C.GFFT_C2C, 0, 1 << 19, 0, 200),
+    for d in (desc(C.GFFT_C2C, C.GFFT_F16, 1 << 16, 0, 600), desc(C.GFFT_C2C, 0, 1 << 21, 0, 100),
               desc(C.GFFT_C2C, 0, 1 << 16, 0, 600, flags=C.GFFT_FLAG_NO_WORKSPACE)):
         assert "xcd" not in explain(d)[1]
     monkeypatch.setenv("GFFT_N1_LOG2", "7")
@@ -121,3 +123,22 @@ def test_in_an_uneven_batch(gpu):
             v = x.numpy()[o:o + n].astype(np.complex128)
             ref = np.fft.ifft(v) * n if d else np.fft.fft(v)
             assert O.rel_l2_rows(h[o:o + n][None], ref[None]).max() <= O.tol_c64(n)
+
+
+@pytest.mark.gpu
+def test_tuned_and_saved(gpu, tmp_path):
+    """The autotuner times the one-launch form beside the others, and a saved
+    choice of it loads as one."""
+    import genfft_amd as G
+    n, batch = 1 << 17, 82
+    try:
+        rep = G.autotune(n, batch, torch.complex64, reps=3)
+        assert sum(c["n1_log2"] == 0 and c["row_variant"] < 0 for c in rep["candidates"]) == 1
+        path = str(tmp_path / "t.json")
+        G.save_tuning(path)
+        C.check(C.lib().gfft_tuning_clear())
+        G.load_tuning(path)
+        text = G.Plan(C.GFFT_C2C, n, batch=batch).describe()
+        assert ("xcd_four_step" in text) == (rep["best"]["n1_log2"] == 0)
+    finally:
+        C.check(C.lib().gfft_tuning_clear())
