@@ -11,7 +11,7 @@
 // 2^18 0.78 -> 0.64 / 201 -> 174, 2^19 0.86 -> 0.66 / 211 -> 178, 2^20 0.81 -> 0.64 /
 // 215 -> 187; c128 2^15 0.80 -> 0.65 / 208 -> 180, 2^16 0.81 -> 0.64 / 210 -> 165,
 // 2^17 0.85 -> 0.70 / 219 -> 181, 2^18 0.84 -> 0.68 / 213 -> 191 (one pass over HBM
-// at a copy's rate: 0.39 / 91).  Near the smallest batches: c64 2^16 x 130 68 -> 69
+// at a copy's rate: 0.39 / 91).  Near the smallest batches: c64 2^16 x 145 76 -> 70
 // us, 2^17 x 81 84 -> 73, 2^20 x 25 191 -> 175, c128 2^18 x 41 156 -> 143: it is
 // taken wherever its ring fits the workspace the two launches would have.  Longer
 // transforms' rings leave the Infinity Cache; c128 2^19 gained 4% at 1 GiB and
@@ -181,7 +181,7 @@ constexpr XcdEntry make_xcd(int lag, int ring, int per_cu, Radices<RA...>, Radic
 // threads of fewer, ms at 1 GiB: 2^17 0.63 / 0.73, 2^18 0.64 / 0.67, 2^19 0.66 /
 // 0.91, 2^20 0.64 / 0.84 (16 * 4 * 16).
 const XcdEntry kXcd[] = {
-    make_xcd<float, 256, 256, 16, 256, 4>(10, 16, 4, Radices<16, 16>{}, Radices<16, 16>{}),
+    make_xcd<float, 256, 256, 16, 256, 4>(10, 18, 4, Radices<16, 16>{}, Radices<16, 16>{}),
     make_xcd<float, 256, 512, 16, 256, 4>(5, 10, 4, Radices<16, 16>{}, Radices<32, 16>{}),
     make_xcd<float, 512, 512, 16, 256, 4>(6, 10, 4, Radices<32, 16>{}, Radices<32, 16>{}),
     make_xcd<float, 1024, 512, 16, 512, 4>(3, 6, 2, Radices<32, 32>{}, Radices<16, 2, 16>{}),
