@@ -126,15 +126,18 @@ __global__ void __launch_bounds__(256) mix_fft_kernel(MixArgs a)
     __shared__ int64_t jin[C::MAXM], jout[C::MAXM];
     __shared__ uint8_t jinv[C::MAXM];
     __shared__ int task_id;
+    // A block's first task is its own index, the rest come from the queue, whose
+    // one counter takes ~25 ns a turn: with two turns per block and task 1759
+    // transforms of 2^9..2^12 spent most of their 42 us on it (24 now).  Every
+    // block takes one number past the end, so the launch takes n_tasks numbers
+    // in all, and whoever gets the last one clears the counter for the next
+    // launch (a launch of its own for that cost 4.3 us and a gap).
+    int ti = blockIdx.x;
     for (;;) {
         // thread index re-materialised per task: otherwise every tid-derived
         // LDS offset of all twelve tile shapes is hoisted and kept live
         int tid = threadIdx.x;
         asm volatile("" : "+v"(tid));
-        if (tid == 0) task_id = (int)atomicAdd(a.counter, 1u);
-        __syncthreads();
-        const int ti = task_id;
-        if (ti >= a.n_tasks) break;  // every wave of the block takes this exit once the queue is drained
         const MixTask t = a.tasks[ti];
         if (tid < t.count) {
             jin[tid] = a.job_in[t.first + tid];
@@ -162,11 +165,17 @@ __global__ void __launch_bounds__(256) mix_fft_kernel(MixArgs a)
             break;
         default: break;
         }
+        if (a.n_tasks <= (int)gridDim.x) break;
+        if (tid == 0) {
+            const uint32_t v = atomicAdd(a.counter, 1u);
+            if (v == (uint32_t)a.n_tasks - 1u) *a.counter = 0u;
+            task_id = (int)(gridDim.x + v);
+        }
         __syncthreads();  // LDS and job slots are reused by the next task
+        ti = task_id;
+        if (ti >= a.n_tasks) break;  // every wave of the block takes this exit once the queue is drained
     }
 }
-
-__global__ void mix_reset_kernel(uint32_t *counter) { *counter = 0u; }
 
 }  // namespace
 
@@ -174,12 +183,6 @@ hipError_t launch_mix(int prec, const MixArgs &a, int grid, hipStream_t s)
 {
     if (prec) hipLaunchKernelGGL(mix_fft_kernel<double>, dim3(grid), dim3(256), 0, s, a);
     else hipLaunchKernelGGL(mix_fft_kernel<float>, dim3(grid), dim3(256), 0, s, a);
-    return hipGetLastError();
-}
-
-hipError_t launch_mix_reset(uint32_t *counter, hipStream_t s)
-{
-    hipLaunchKernelGGL(mix_reset_kernel, dim3(1), dim3(1), 0, s, counter);
     return hipGetLastError();
 }
 

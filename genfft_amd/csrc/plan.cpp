@@ -514,7 +514,7 @@ PlanOpts resolve_opts(int prec, int64_t n, const PlanOpts *forced)
 // Plan representation
 // ---------------------------------------------------------------------------
 enum BufId { B_IN = 0, B_OUT = 1, B_SCR = 2 };
-enum LaunchType { LT_TILE, LT_UNPACK, LT_PACK, LT_HFILL, LT_COPY, LT_MIX, LT_MIX_RESET, LT_R2C, LT_C2R, LT_RROWS,
+enum LaunchType { LT_TILE, LT_UNPACK, LT_PACK, LT_HFILL, LT_COPY, LT_MIX, LT_R2C, LT_C2R, LT_RROWS,
                   LT_REPACK, LT_DUAL, LT_XCD };
 
 // bytes of one complex element in memory
@@ -1989,7 +1989,6 @@ int validate_list(const gfft_plan_s *p, const std::vector<Launch> &launches)
             break;
         }
         case LT_MIX:
-        case LT_MIX_RESET:
             return fail(GFFT_ERR_UNSUPPORTED, "internal: launch %d belongs to batch plans", idx);
         }
     }
@@ -2099,9 +2098,6 @@ int describe_launches(const std::vector<Launch> &launches, const std::string &he
             break;
         case LT_MIX:
             snprintf(line, sizeof(line), "mix tasks=%d grid=%lld\n", l.mix.n_tasks, (long long)l.grid);
-            break;
-        case LT_MIX_RESET:
-            snprintf(line, sizeof(line), "mix_reset\n");
             break;
         }
         s += line;
@@ -2339,9 +2335,6 @@ int run_launches(const std::vector<Launch> &launches, int prec, int xcd_remap, c
             HIP_TRY(launch_repack(a, s));
             break;
         }
-        case LT_MIX_RESET:
-            HIP_TRY(launch_mix_reset(l.mix.counter, s));
-            break;
         case LT_MIX: {
             MixArgs a = l.mix;
             a.in = ip;
@@ -2504,10 +2497,6 @@ int build_batch(gfft_batch_plan_s *p)
 
     if (!tasks.empty()) {
         if ((st = upload((void **)&p->d_tasks, tasks.data(), tasks.size() * sizeof(MixTask)))) return st;
-        Launch r;
-        r.type = LT_MIX_RESET;
-        r.mix.counter = p->d_counter;
-        p->launches.push_back(r);
         Launch l;
         l.type = LT_MIX;
         l.mix.job_in = p->d_job_in;
@@ -3234,7 +3223,7 @@ int gfft_plan_profile_launch(gfft_plan plan, const void *in, void *out, int dire
     if ((direction != GFFT_FORWARD && direction != GFFT_INVERSE) || !(plan->dir_mask & (1 << direction)))
         return fail(GFFT_ERR_INVALID_ARG, "direction %d is not one this plan runs", direction);
     const Launch &l = plan->launches[launch];
-    if (l.type == LT_MIX || l.type == LT_MIX_RESET)
+    if (l.type == LT_MIX)
         return fail(GFFT_ERR_UNSUPPORTED, "a work-queue launch runs once per reset");
     if (plan->scratch_bytes && !plan->scratch)
         return fail(GFFT_ERR_INVALID_ARG, "plan created with GFFT_FLAG_NO_WORKSPACE holds no workspace");
