@@ -675,6 +675,11 @@ bool tile_offsets_fit(int pat, int64_t L, int64_t M, int64_t inner, int64_t elem
     return last * (int64_t)csize < ((int64_t)1 << 31);
 }
 
+// Uneven batches of up to this many launches are enqueued, not replayed as a
+// graph, in graph mode too: a replay starts ~8 us later than a launch (MI355X,
+// us a call, replay / enqueued: 1 launch 16.6 / 8.4, 3 launches 34.1 / 26.3, 8
+// launches 70.3 / 62.7).
+constexpr size_t kFewLaunches = 8;
 // Batches of at least this many bytes a side stream through HBM: row tiles
 // with the `wide` flag.
 constexpr int64_t kStreamBytes = (int64_t)512 << 20;
@@ -3224,7 +3229,7 @@ int gfft_plan_profile_launch(gfft_plan plan, const void *in, void *out, int dire
         return fail(GFFT_ERR_INVALID_ARG, "direction %d is not one this plan runs", direction);
     const Launch &l = plan->launches[launch];
     if (l.type == LT_MIX)
-        return fail(GFFT_ERR_UNSUPPORTED, "a work-queue launch runs once per reset");
+        return fail(GFFT_ERR_UNSUPPORTED, "a work-queue launch belongs to batch plans");
     if (plan->scratch_bytes && !plan->scratch)
         return fail(GFFT_ERR_INVALID_ARG, "plan created with GFFT_FLAG_NO_WORKSPACE holds no workspace");
     if (int st = on_plan_device(plan->device)) return st;
@@ -3372,7 +3377,7 @@ int gfft_batch_execute(gfft_batch_plan plan, const void *in, void *out, int mode
     if (int st = on_plan_device(plan->device)) return st;
     const hipStream_t s = (hipStream_t)stream;
     std::lock_guard<std::mutex> lk(plan->mu);
-    if (mode == GFFT_BATCH_EAGER) {
+    if (mode == GFFT_BATCH_EAGER || (mode == GFFT_BATCH_GRAPH && plan->launches.size() <= kFewLaunches)) {
         std::lock_guard<std::mutex> lo(plan->order.mu);
         HIP_TRY(plan->order.before(s));
         int st = enqueue_batch(plan, in, out, s);

@@ -261,7 +261,7 @@ GFFT_API int gfft_interleave_real_2d(int precision, void *out, int64_t out_strid
  * write where another job reads or writes (a job may be in place). */
 typedef struct gfft_batch_plan_s *gfft_batch_plan;
 
-#define GFFT_BATCH_GRAPH 0    /* capture the launches once into a HIP graph and replay it */
+#define GFFT_BATCH_GRAPH 0    /* more than 8 launches: capture them once into a HIP graph and replay it */
 #define GFFT_BATCH_EAGER 1    /* enqueue the launches directly */
 #define GFFT_BATCH_PER_JOB 2  /* the plain path: one single-transform plan launch per job */
 

@@ -126,3 +126,22 @@ def test_uneven_full_configuration_sample(gpu):
     pick = np.random.default_rng(1).choice(count, 500, replace=False)
     assert len(set(int(sizes[j]) for j in pick)) == 11
     check_jobs(xs, ys, sizes, offs, offs, inv, "f32", pick)
+
+
+def test_many_launches_replay_as_a_graph(gpu):
+    """A list long enough to be replayed (two launches per length past the
+    rows' limit), bit-identical to the same list enqueued."""
+    import genfft_amd as G
+    sizes = [1 << k for k in range(11, 21) for _ in range(2)]
+    offs = np.concatenate([[0], np.cumsum(sizes)[:-1]])
+    b = G.UnevenBatch(sizes, offs, offs, [k % 2 == 1 for k in range(len(sizes))])
+    assert len(b.describe().splitlines()) > 9
+    g = torch.Generator().manual_seed(5)
+    ref = torch.empty(sum(sizes), dtype=torch.complex64, device=gpu)
+    x = torch.randn(sum(sizes), dtype=torch.complex64, generator=g).to(gpu)
+    b.execute(x, ref, mode="eager")
+    for rep in range(3):
+        y = torch.zeros_like(ref)
+        b.execute(x, y, mode="graph")
+        torch.cuda.synchronize()
+        assert torch.equal(y, ref), rep
