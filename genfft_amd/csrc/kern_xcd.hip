@@ -43,6 +43,12 @@ __device__ __forceinline__ uint32_t await(uint32_t *p, uint32_t v)
     return x;
 }
 
+// Acquire at agent scope of what an await() has seen, as the compiler writes it
+// (buffer_inv sc1; sc0 is the scope of a workgroup), without the wait of its
+// fence for this wave's own output stores.  The wave's next atomic, whose result
+// it waits for, follows it through the cache.
+__device__ __forceinline__ void acquire_agent() { asm volatile("buffer_inv sc1" ::: "memory"); }
+
 // Takes the next task of an XCD's queue.  Whoever takes a block's first task
 // claims the next transform of the batch for the block at once, after the block
 // before has its own, so an XCD's blocks run out of transforms in order.
@@ -92,8 +98,13 @@ __device__ __forceinline__ void tile_of(T *plane, const TileArgs &a, const cx<T>
 // inside, and holds no other task then.
 //
 // What one CU hands to another stays on one XCD, so no cache is written back:
-// stores are in the L2 once vmcnt is 0, and the readers drop their CU's own
-// cache (buffer_inv sc0) after they saw the count.
+// stores are in the L2 once vmcnt is 0.  The readers are on other CUs, whose own
+// caches may hold lines of the ring from the slot's last transform: the thread
+// that saw the count acquires at agent scope (acquire_agent) and the workgroup
+// barrier hands that on to the other waves, which share its CU's cache.  MI355X,
+// c64 2^20 x 128 / uneven batch of 5000 transforms of 2^6..2^16: 640 / 319 us so,
+// 794 / 425 with every wave invalidating, 653 / 313 with agent-scope loads of
+// the ring instead.
 template <typename T, int N1, int N2, int M, int NT, int WPE, class RA, class RB>
 __global__ void __launch_bounds__(NT, WPE) xcd_fft_kernel(XcdArgs x)
 {
@@ -120,8 +131,10 @@ __global__ void __launch_bounds__(NT, WPE) xcd_fft_kernel(XcdArgs x)
                 uint32_t *const w = blk + (int64_t)c * 4;
                 g = (int)await(w, 1u) - 1;
                 if (g >= x.batch) g = rows ? -2 : -1;
-                else if (rows) await(w + 1, T1);
-                else if (c >= x.ring) await(w - (int64_t)x.ring * 4 + 2, T2);
+                else if (rows) {
+                    await(w + 1, T1);
+                    acquire_agent();
+                } else if (c >= x.ring) await(w - (int64_t)x.ring * 4 + 2, T2);
             }
             task[0] = g;
             task[1] = r;
@@ -139,7 +152,6 @@ __global__ void __launch_bounds__(NT, WPE) xcd_fft_kernel(XcdArgs x)
                     RA{});
                 asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             } else {
-                asm volatile("buffer_inv sc0" ::: "memory");
                 tile_of<T, N2, M, NT, PAT_ROW, HINT_ST>(
                     plane, x.row, slot, reinterpret_cast<cx<T> *>(x.row.out) + out_base(x.row, 0, g), (r - T1) * M, g,
                     tid, RB{});

@@ -1,6 +1,11 @@
 """Four-steps that run both passes in one launch, a transform per XCD
 (genfft_amd/csrc/kern_xcd.hip), against numpy's float64 transform at the
 library's bounds (rel-L2 2e-7*log2 N complex64, 1e-15*log2 N complex128)."""
+import os
+import re
+import shutil
+import subprocess
+
 import numpy as np
 import pytest
 import torch
@@ -34,6 +39,31 @@ def test_route(monkeypatch):
         assert "xcd" not in explain(d)[1]
     monkeypatch.setenv("GFFT_N1_LOG2", "7")
     assert "xcd" not in explain(desc(C.GFFT_C2C, 0, 1 << 16, 0, 600))[1]
+
+
+HIPCC = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+
+
+@pytest.mark.skipif(not os.path.exists(HIPCC), reason="needs the compiler")
+def test_hand_over_is_acquired_at_agent_scope(tmp_path):
+    """Row tiles read what other CUs' workgroups stored: every one-launch kernel
+    invalidates at the scope of an agent (sc1), as the compiler does for an
+    agent-scope acquire, before the barrier that hands the task out."""
+    csrc = os.path.join(os.path.dirname(C.LIB_PATH), "csrc")
+    asm = str(tmp_path / "xcd.s")
+    subprocess.run([HIPCC, "--offload-arch=gfx950", "-O3", "-std=c++17", "-Xclang", "-target-feature", "-Xclang",
+                    "-packed-fp32-ops", "--offload-device-only", "-S", os.path.join(csrc, "kern_xcd.hip"), "-o", asm],
+                   check=True, capture_output=True)
+    kernels = re.split(r"^(?=\S*xcd_fft_kernel\S*:)", open(asm).read(), flags=re.M)[1:]
+    assert len(kernels) >= 9
+    for text in kernels:
+        body = text.split(".end_amdhsa_kernel")[0]
+        # a batch that reads the ring: the acquire, then loads
+        inv = re.findall(r"^\s*buffer_inv\s*(.*?)\s*$", body, flags=re.M)
+        assert inv and all(v.split() == ["sc1"] for v in inv), (text.split(":")[0], inv)
+        for after in re.split(r"^\s*buffer_inv.*$", body, flags=re.M)[1:]:
+            ops = re.findall(r"^\s*(s_barrier|global_load\w*|flat_load\w*)", after, flags=re.M)
+            assert ops[0] == "s_barrier", (text.split(":")[0], ops[0])
 
 
 @pytest.mark.gpu
