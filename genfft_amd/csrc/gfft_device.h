@@ -185,6 +185,11 @@ enum : int { PAT_ROW = 0, PAT_COL = 1 };
 enum : int { LAY_SEQ = 0, LAY_ELEM = 1 };
 enum : int { TW_NONE = 0, TW_INNER = 1, TW_OUTER = 2 };
 
+// Gain and limit of an automatic scale (scale_from_max).
+struct ScaleBound {
+    float gain, limit;
+};
+
 struct TileArgs {
     const void *in;
     void *out;
@@ -216,8 +221,18 @@ struct TileArgs {
     int32_t job_first;
     int32_t job_swap_in, job_swap_out;
     const void *pass_tw;  // Stockham pass twiddles, complex T
-    const double *tw_lo;  // complex double [1 << tw_lo_bits]: W_Ntw^m
-    const double *tw_hi;  // complex double [Ntw >> tw_lo_bits]: W_Ntw^(m << tw_lo_bits)
+    // Automatic scale (kernels that hold a whole transform, reg_rows_kernel_h,
+    // which have no four-step twiddle): the kernel computes the scale of
+    // transform s (scale_from_max with `bound`), applies it and writes it to
+    // auto_scale[s].  Null: off.
+    union {
+        const double *tw_lo;  // complex double [1 << tw_lo_bits]: W_Ntw^m
+        float *auto_scale;
+    };
+    union {
+        const double *tw_hi;  // complex double [Ntw >> tw_lo_bits]: W_Ntw^(m << tw_lo_bits)
+        ScaleBound bound;
+    };
     // Two-level FP64 table of W_L, b = (log2 L + 1) / 2: gen_lo[m] = W_L^m
     // (m < 2^b), gen_hi[h] = W_L^(h << b), for pipelined kernels whose last
     // pass builds its twiddles instead of reading pass_tw (PassTw::GEN)
@@ -229,12 +244,10 @@ struct TileArgs {
     // scale[] of that transform.  Null: no scaling.
     const float *scale;
     int64_t scale_div, scale_off;
-    // Automatic scale (kernels that hold a whole transform, reg_rows_kernel_h):
-    // the kernel computes the scale of transform s (scale_from_max with gain
-    // and limit), applies it and writes it to auto_scale[s].  Null: off.
-    float *auto_scale;
-    float gain, limit;
 };
+// The smallest launches feel the size of their arguments: at 256 bytes 8-point
+// rows and columns took 4.3-4.7 us, at 240 3.9-4.6 (MI355X; 2-8% a call).
+static_assert(sizeof(TileArgs) <= 240, "TileArgs outgrew its launch cost");
 
 // FP64 twiddle W_Ntw^m from the two-level table.
 __device__ __forceinline__ cx<double> tw_fp64(const TileArgs &a, uint32_t m)

@@ -470,7 +470,7 @@ __global__ void __launch_bounds__(NT, 4) reg_rows_kernel_h(TileArgs a)
 #pragma unroll
             for (int i = 0; i < TPS / 64; i++) m = fmaxf(m, red[i]);
         }
-        scl = scale_from_max(m, a.gain, a.limit);
+        scl = scale_from_max(m, a.bound.gain, a.bound.limit);
         if (tid % TPS == 0 && s < nvalid) a.auto_scale[s0 + s] = scl;
     } else if (a.scale && s < nvalid) {
         scl = a.scale[(a.scale_off + ibase + (int64_t)s * a.in_inner) / a.scale_div];

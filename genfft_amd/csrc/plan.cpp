@@ -2230,9 +2230,10 @@ int run_launches(const std::vector<Launch> &launches, int prec, int xcd_remap, c
                 a.scale = scale.given;
                 a.scale_div = scale.div;
                 a.scale_off = l.in_off / (int64_t)csize_of(l.k->prec, l.k->store);
-                a.auto_scale = scale.automatic;
-                a.gain = scale.gain;
-                a.limit = scale.limit;
+                if (scale.automatic) {  // row tiles only: they have no twiddle table there
+                    a.auto_scale = scale.automatic;
+                    a.bound = {scale.gain, scale.limit};
+                }
             }
             void *args[] = {&a};
             HIP_TRY(hipExtLaunchKernel((const void *)(plain ? l.k->fn_plain : l.k->fn), dim3((unsigned)l.grid),
