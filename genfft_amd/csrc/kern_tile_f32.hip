@@ -134,7 +134,9 @@ const KernelEntry kTable[] = {
     // --- column tiles held in registers.  Four-step passes (MI355X, 1 GiB a
     // pass): 512 rows 0.476 -> 0.421 ms (from 4 tiles per CU on; below, the
     // LDS tile: 2^19 x 4 25 against 28 us), 2048 rows of 16 columns 0.540 ->
-    // 0.48-0.49 (8 columns are as much as the LDS holds: 64-byte runs).  Whole
+    // 0.48-0.49 (8 columns are as much as the LDS holds: 64-byte runs), from one
+    // tile per CU on (real 2^21 x 2, 64 of them against 128 of 8 columns: 67.7 /
+    // 62.9 us; 2^21 x 8, 256 of them: 134 / 146).  Whole
     // column transforms, by width (Builder::col_variant), us, LDS -> register
     // tile: 512 x 999 8.0 -> 5.7, 1024 x 513 12.6 -> 7.2, 1024 x 4999 32 -> 20
     // (the pipelined 16-column tile left 2 rounds of 256 workgroups, the second
@@ -143,7 +145,7 @@ const KernelEntry kTable[] = {
     // want 8 columns: two 4-column tiles per CU keep 8 MB of quarter lines in
     // flight per XCD, twice its L2 (4096 x 4096: 135 us, LDS tile 105) ---
     make_reg_many<T, 512, 16, 512, C_, C_, 16, 2, 16>(4),
-    make_reg_entry<T, 2048, 16, 1024, C_, C_, 16, 8, 16>(),
+    make_reg_many<T, 2048, 16, 1024, C_, C_, 16, 8, 16>(1),
     make_reg_cols<T, 64, 16, 128, 8, 8>(),
     make_reg_cols<T, 128, 8, 128, 8, 2, 8>(),
     make_reg_cols<T, 256, 8, 256, 8, 4, 8>(),
@@ -157,8 +159,8 @@ const KernelEntry kTable[] = {
     make_reg_cols_big<T, 4096, 8, 1024, 16, 16, 16>((int64_t)96 << 20),
     // --- transposing rows held in registers: 2048 points, 2^22 x 32 0.505 ->
     // 0.456 ms (128-byte runs instead of 64) ---
-    make_reg_entry<T, 2048, 16, 1024, R_, C_, 16, 16, 8>(),
-    make_reg_entry<T, 4096, 8, 1024, R_, C_, 16, 16, 16>(),
+    make_reg_many<T, 2048, 16, 1024, R_, C_, 16, 16, 8>(1),
+    make_reg_many<T, 4096, 8, 1024, R_, C_, 16, 16, 16>(1),
     // --- more column tiles of whole column transforms.  Few rows, us, LDS ->
     // register tile: 32 x 16 4.5 -> 3.3, x 32768 5.3 -> 4.5, 64 x 300 5.1 ->
     // 3.8, x 32768 7.5 -> 6.5, 128 x 32768 12.2 -> 11.1, 256 x 4096 5.8 -> 5.2,

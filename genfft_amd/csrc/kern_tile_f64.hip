@@ -95,7 +95,7 @@ const KernelEntry kTable[] = {
     // pipelined 1024-row tile stays the four-step's: 0.469 against 0.496).  512
     // rows whose pitch is no multiple of a line stay on the LDS tile past 128
     // MiB: 16387 columns 66 against 70, 65539 249 against 290 ---
-    make_reg_entry<T, 2048, 8, 1024, C_, C_, 16, 8, 16>(),
+    make_reg_many<T, 2048, 8, 1024, C_, C_, 16, 8, 16>(1),
     make_reg_cols<T, 128, 8, 128, 8, 2, 8>(),
     make_reg_cols<T, 128, 16, 256, 8, 2, 8>(),
     make_reg_cols<T, 256, 4, 128, 8, 4, 8>(),
@@ -107,7 +107,7 @@ const KernelEntry kTable[] = {
     make_reg_cols<T, 2048, 4, 512, 16, 8, 16>(),
     make_reg_cols<T, 2048, 8, 1024, 16, 8, 16>(),
     // --- transposing rows held in registers ---
-    make_reg_entry<T, 2048, 8, 1024, R_, C_, 16, 16, 8>(),
+    make_reg_many<T, 2048, 8, 1024, R_, C_, 16, 16, 8>(1),
     // --- short rows and columns held in registers.  Rows, us, one row / 1 MiB /
     // 32 MiB / 128 MiB, LDS -> register tile: 16 points 3.9 -> 3.0 / 5.5 -> 3.2 /
     // 14.5 -> 14.6 / LDS, 32 4.7 -> 3.4 / 6.3 -> 3.6 / 16.1 -> 12.8 / 60 -> 57,

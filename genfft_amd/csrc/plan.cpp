@@ -749,8 +749,10 @@ struct Builder {
              int tw_mode, int64_t tw_n, bool first, bool last, int variant = -1)
     {
         const KernelEntry *k = find_tile(prec, L, inp, outp, prefer_m, opts.pipe_mask, variant, store);
-        if (k && k->many && (n_inner + k->M - 1) / k->M * n_outer1 * n_outer2 < (int64_t)k->many * p->num_cus)
-            k = find_tile(prec, L, inp, outp, k->M, opts.pipe_mask, -1, store, true);
+        if (k && k->many && (n_inner + k->M - 1) / k->M * n_outer1 * n_outer2 < (int64_t)k->many * p->num_cus) {
+            const KernelEntry *d = find_tile(prec, L, inp, outp, k->M, opts.pipe_mask, -1, store, true);
+            if (d && (d->M == k->M || !prefer_m)) k = d;  // a tuned width stays
+        }
         if (k && k->reg && !(tile_offsets_fit(inp, k->L, k->M, in_inner, in_elem, csize) &&
                              tile_offsets_fit(outp, k->L, k->M, out_inner, out_elem, csize)))
             k = find_tile(prec, L, inp, outp, prefer_m, opts.pipe_mask, -1, store, true);

@@ -312,3 +312,17 @@ def test_batches_of_images(gpu, prec, w, h, batch, pad):
         assert O.rel_l2_rows(np.ascontiguousarray(got[:, :, :w]).reshape(batch, -1), ref.reshape(batch, -1)).max() <= tol(w * h)
         if pad:
             assert np.all(got[:, :, w:] == 7 + 5j)
+
+
+@pytest.mark.parametrize("kind,prec,n,few,many,narrow,wide", [
+    (C.GFFT_R2C, 0, 1 << 21, 2, 8, "8", "16"), (C.GFFT_R2C, 0, 1 << 22, 1, 4, "8", "16"),
+    (C.GFFT_R2C, 1, 1 << 21, 1, 4, "4", "8"), (C.GFFT_C2C, 0, 1 << 21, 1, 4, "8", "16"),
+    (C.GFFT_C2C, 1, 1 << 21, 1, 4, "4", "8")])
+def test_small_batches_of_long_transforms_keep_the_narrow_columns(kind, prec, n, few, many, narrow, wide):
+    """The wide 2048-row column tiles held in registers are taken once they
+    number the 256 CUs (complex64 real 2^21 x 2: 67.7 us with 64 of them, 62.9
+    with 128 narrow ones)."""
+    for batch, m in ((few, narrow), (many, wide)):
+        st, text = explain(desc(kind, prec, n, 0, batch, flags=C.GFFT_FLAG_HALF if kind == C.GFFT_R2C else 0))
+        cols = [t for t in tiles(text) if field(t, "L") == "2048" and field(t, "inp") == "1"]
+        assert st == 0 and [field(t, "M") for t in cols] == [m], text
