@@ -239,8 +239,9 @@ constexpr int col_map()
 }
 
 // Cache hints of a launch's HBM accesses: HINT_LD / HINT_ST mark its loads /
-// stores nontemporal (streaming).
-enum : int { HINT_NONE = 0, HINT_LD = 1, HINT_ST = 2 };
+// stores nontemporal (streaming); HINT_AGENT its loads as of agent scope, for
+// what another CU wrote earlier in the same launch (whole tiles of rows only).
+enum : int { HINT_NONE = 0, HINT_LD = 1, HINT_ST = 2, HINT_AGENT = 4 };
 
 // W adjacent elements, read or written together (complex64 pairs as 16 bytes
 // at the 8-byte alignment of an element, which global accesses allow).
@@ -283,6 +284,18 @@ __device__ __forceinline__ void reg_store(cx<T> *p, const cx<T> *x, int stride)
     }
 }
 
+// One element, `own` + `step` bytes from a uniform base, read at agent scope
+// (sc1): past the CU's own cache.  `buffer` ends with the tile.
+template <typename T>
+__device__ __forceinline__ cx<T> agent_load(__amdgpu_buffer_rsrc_t buffer, uint32_t own, int step)
+{
+    constexpr int SC1 = 16;
+    if constexpr (sizeof(T) == 4)
+        return __builtin_bit_cast(cx<T>, __builtin_amdgcn_raw_buffer_load_b64(buffer, (int)own, step, SC1));
+    else
+        return __builtin_bit_cast(cx<T>, __builtin_amdgcn_raw_buffer_load_b128(buffer, (int)own, step, SC1));
+}
+
 // One tile: sequences s0 .. s0 + nvalid - 1 of transform o, read from `in` and
 // written to `out` (the transform's first elements).  INP / OUTP as in
 // tile_fft_kernel.  The first pass walks along the rows when they are read
@@ -311,6 +324,14 @@ __device__ __forceinline__ void reg_tile(T *plane, const TileArgs &a, const cx<T
             const uint32_t to = (INP == PAT_ROW ? (uint32_t)s * (uint32_t)a.in_inner + (uint32_t)j
                                                 : (uint32_t)j * (uint32_t)a.in_elem + (uint32_t)s) * (uint32_t)sizeof(cx<T>);
             cx<T> *x = &v[q * A::W * R1];
+            if constexpr ((HINT & HINT_AGENT) != 0) {
+                static_assert(INP == PAT_ROW && A::W == 1, "tiles of rows");
+                const __amdgpu_buffer_rsrc_t buffer = __builtin_amdgcn_make_buffer_rsrc(
+                    const_cast<char *>(ib), 0, (int)(M * a.in_inner * (int64_t)sizeof(cx<T>)), 0x00027000);
+#pragma unroll
+                for (int r = 0; r < R1; r++) x[r] = agent_load<T>(buffer, to, (int)(r * step));
+                continue;
+            }
 #pragma unroll
             for (int r = 0; r < R1; r++) {
                 const cx<T> *p = reinterpret_cast<const cx<T> *>(ib + r * step + to);

@@ -43,12 +43,6 @@ __device__ __forceinline__ uint32_t await(uint32_t *p, uint32_t v)
     return x;
 }
 
-// Acquire at agent scope of what an await() has seen, as the compiler writes it
-// (buffer_inv sc1; sc0 is the scope of a workgroup), without the wait of its
-// fence for this wave's own output stores.  The wave's next atomic, whose result
-// it waits for, follows it through the cache.
-__device__ __forceinline__ void acquire_agent() { asm volatile("buffer_inv sc1" ::: "memory"); }
-
 // Takes the next task of an XCD's queue.  Whoever takes a block's first task
 // claims the next transform of the batch for the block at once, after the block
 // before has its own, so an XCD's blocks run out of transforms in order.
@@ -99,12 +93,12 @@ __device__ __forceinline__ void tile_of(T *plane, const TileArgs &a, const cx<T>
 //
 // What one CU hands to another stays on one XCD, so no cache is written back:
 // stores are in the L2 once vmcnt is 0.  The readers are on other CUs, whose own
-// caches may hold lines of the ring from the slot's last transform: the thread
-// that saw the count acquires at agent scope (acquire_agent) and the workgroup
-// barrier hands that on to the other waves, which share its CU's cache.  MI355X,
-// c64 2^20 x 128 / uneven batch of 5000 transforms of 2^6..2^16: 640 / 319 us so,
-// 794 / 425 with every wave invalidating, 653 / 313 with agent-scope loads of
-// the ring instead.
+// caches may hold lines of the ring from the slot's last transform, so they load
+// it at agent scope (HINT_AGENT), from the L2.  MI355X, us, start of a batch's
+// range / 1 GiB: c64 2^16 69.9 / 617, 2^20 182 / 642, c128 2^16 98.9 / 634 so;
+// 73.2 / 632, 186 / 644, 105 / 667 with an agent-scope invalidate (buffer_inv sc1)
+// by the thread that saw the count instead, and c64 2^20 794 with one by every
+// wave.  A workgroup-scope invalidate (sc0) need not drop those lines.
 template <typename T, int N1, int N2, int M, int NT, int WPE, class RA, class RB>
 __global__ void __launch_bounds__(NT, WPE) xcd_fft_kernel(XcdArgs x)
 {
@@ -131,10 +125,8 @@ __global__ void __launch_bounds__(NT, WPE) xcd_fft_kernel(XcdArgs x)
                 uint32_t *const w = blk + (int64_t)c * 4;
                 g = (int)await(w, 1u) - 1;
                 if (g >= x.batch) g = rows ? -2 : -1;
-                else if (rows) {
-                    await(w + 1, T1);
-                    acquire_agent();
-                } else if (c >= x.ring) await(w - (int64_t)x.ring * 4 + 2, T2);
+                else if (rows) await(w + 1, T1);
+                else if (c >= x.ring) await(w - (int64_t)x.ring * 4 + 2, T2);
             }
             task[0] = g;
             task[1] = r;
@@ -142,7 +134,9 @@ __global__ void __launch_bounds__(NT, WPE) xcd_fft_kernel(XcdArgs x)
             if (g != -2) next = take(pop, blk, x.state, T1 + T2, x.blocks);
         }
         __syncthreads();
-        const int g = task[0], r = task[1], c = task[2];
+        // uniform, so that the tiles' bases stay in scalar registers
+        const int g = __builtin_amdgcn_readfirstlane(task[0]), r = __builtin_amdgcn_readfirstlane(task[1]),
+                  c = __builtin_amdgcn_readfirstlane(task[2]);
         if (g == -2) break;
         if (g >= 0) {
             cx<T> *const slot = ring + (int64_t)(c % x.ring) * N;
@@ -152,7 +146,7 @@ __global__ void __launch_bounds__(NT, WPE) xcd_fft_kernel(XcdArgs x)
                     RA{});
                 asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             } else {
-                tile_of<T, N2, M, NT, PAT_ROW, HINT_ST>(
+                tile_of<T, N2, M, NT, PAT_ROW, HINT_ST | HINT_AGENT>(
                     plane, x.row, slot, reinterpret_cast<cx<T> *>(x.row.out) + out_base(x.row, 0, g), (r - T1) * M, g,
                     tid, RB{});
             }
