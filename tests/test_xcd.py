@@ -171,3 +171,99 @@ def test_tuned_and_saved(gpu, tmp_path):
         assert ("xcd_four_step" in text) == (rep["best"]["n1_log2"] == 0)
     finally:
         C.check(C.lib().gfft_tuning_clear())
+
+
+# (prec, n, batch of at least three times the ring's slots, slots, chunk limit)
+WRAPS = [("c64", 1 << 16, 450, 144, 0), ("c64", 1 << 17, 250, 80, 0), ("c64", 1 << 18, 245, 80, 0),
+         ("c64", 1 << 19, 150, 48, 0), ("c64", 1 << 20, 100, 32, 0), ("c64", 1 << 20, 75, 24, 200 << 20),
+         ("c128", 1 << 15, 300, 96, 0), ("c128", 1 << 16, 390, 128, 0), ("c128", 1 << 17, 200, 64, 0),
+         ("c128", 1 << 18, 125, 40, 0)]
+
+
+def _gpu_rand(shape, dtype, seed):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    return torch.randn(shape, dtype=dtype, device="cuda", generator=g)
+
+
+def _worst(y, ref):
+    return float(((y - ref).abs().square().sum(-1) / ref.abs().square().sum(-1)).max().sqrt())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("in_place", [False, True])
+@pytest.mark.parametrize("prec,n,batch,slots,chunk", WRAPS)
+def test_ring_goes_round(gpu, monkeypatch, prec, n, batch, slots, chunk, in_place):
+    """Every ring reused at least three times over: each transform against the
+    two launches (bound: both sides' tolerances), three of them against the
+    long-double oracle."""
+    import genfft_amd as G
+    p, ndt, tdt, tol = PREC[prec]
+    assert batch >= 3 * slots
+    x = _gpu_rand((batch, n), tdt, n)
+    if chunk:
+        monkeypatch.setenv("GFFT_CHUNK_BYTES", str(chunk))
+    one = G.Plan(C.GFFT_C2C, n, precision=p, batch=batch)
+    assert f"batch={batch} ring={slots // 8} " in one.describe()
+    monkeypatch.setenv("GFFT_DUAL", "0")
+    two = G.Plan(C.GFFT_C2C, n, precision=p, batch=batch)
+    assert "xcd" not in two.describe()
+    ref = torch.empty_like(x)
+    two.execute(x, ref)
+    y = x.clone() if in_place else torch.empty_like(x)
+    for k in range(1 if in_place else 2):
+        one.execute(y if in_place else x, y)
+        assert _worst(y, ref) <= 2 * tol(n)
+    rows = [0, batch // 2, batch - 1]
+    want = O.fft_ld(x[rows].cpu().numpy().astype(np.complex128))
+    assert O.rel_l2_rows(y[rows].cpu().numpy(), want).max() <= tol(n)
+
+
+@pytest.mark.gpu
+def test_ring_goes_round_in_an_uneven_batch(gpu):
+    """Two classes of it in one batch, jobs of both directions an odd number of
+    elements apart, one after the other through one workspace."""
+    import genfft_amd as G
+    rng = np.random.default_rng(4)
+    sizes = np.concatenate([np.full(450, 1 << 16), np.full(250, 1 << 17), np.full(40, 1 << 9)])
+    rng.shuffle(sizes)
+    offs = np.concatenate([[0], np.cumsum(sizes + rng.integers(0, 4, len(sizes)))[:-1]])
+    dirs = rng.integers(0, 2, len(sizes)).astype(bool)
+    x = _gpu_rand((int(offs[-1] + sizes[-1]),), torch.complex64, 4)
+    y = torch.zeros_like(x)
+    G.UnevenBatch(sizes.tolist(), offs.tolist(), offs.tolist(), dirs.tolist(), torch.complex64).execute(x, y)
+    for n in (1 << 9, 1 << 16, 1 << 17):
+        for inv in (False, True):
+            at = offs[(sizes == n) & (dirs == inv)]
+            idx = torch.from_numpy(at)[:, None].to(gpu) + torch.arange(n, device=gpu)
+            v, got = x[idx], y[idx]
+            one = G.FFT(n, torch.complex64)
+            for k in range(0, len(at), 60):  # short batches: two launches
+                ref = torch.empty_like(v[k:k + 60])
+                one.transform(ref, v[k:k + 60].contiguous(), inv)
+                assert _worst(got[k:k + 60], ref) <= 2 * O.tol_c64(n)
+
+
+@pytest.mark.gpu
+def test_two_plans_at_once(gpu):
+    """Two plans with rings of their own on two streams at the same time."""
+    import genfft_amd as G
+    cases = [(torch.complex64, C.GFFT_F32, 1 << 17, 200), (torch.complex128, C.GFFT_F64, 1 << 15, 300)]
+    plans = [G.Plan(C.GFFT_C2C, n, precision=p, batch=b) for _, p, n, b in cases]
+    x = [_gpu_rand((b, n), dt, n) for dt, _, n, b in cases]
+    ref = [torch.empty_like(t) for t in x]
+    for pl, a, r in zip(plans, x, ref):
+        pl.execute(a, r)
+    for (dt, _, n, b), a, r in zip(cases, x, ref):
+        assert O.rel_l2_rows(r[[0, b - 1]].cpu().numpy(), np.fft.fft(a[[0, b - 1]].cpu().numpy().astype(np.complex128))
+                             ).max() <= (O.tol_c64(n) if dt == torch.complex64 else O.tol_c128(n))
+    side = [torch.cuda.Stream(), torch.cuda.Stream()]
+    y = [[torch.empty_like(t) for _ in range(3)] for t in x]
+    torch.cuda.synchronize()
+    for k in range(3):
+        for i in (0, 1):
+            with torch.cuda.stream(side[i]):
+                plans[i].execute(x[i], y[i][k])
+    torch.cuda.synchronize()
+    for i in (0, 1):
+        for k in range(3):
+            assert torch.equal(y[i][k], ref[i])  # the same kernel on the same input
