@@ -9,7 +9,7 @@
 // 0.83-2.1 ms instead of 0.63.  MI355X against two launches, ms at 1 GiB / us at
 // 238 MiB: c64 2^16 0.75 -> 0.63 / 198 -> 170, 2^17 0.80 -> 0.64 / 205 -> 168,
 // 2^18 0.78 -> 0.64 / 201 -> 174, 2^19 0.86 -> 0.66 / 211 -> 178, 2^20 0.81 -> 0.64 /
-// 215 -> 187; c128 2^15 0.80 -> 0.65 / 208 -> 180, 2^16 0.81 -> 0.64 / 210 -> 165,
+// 215 -> 187; c128 2^15 0.80 -> 0.65 / 208 -> 166, 2^16 0.81 -> 0.64 / 210 -> 165,
 // 2^17 0.85 -> 0.70 / 219 -> 181, 2^18 0.84 -> 0.68 / 213 -> 191 (one pass over HBM
 // at a copy's rate: 0.39 / 91).  Near the smallest batches: c64 2^16 x 145 76 -> 70
 // us, 2^17 x 81 84 -> 73, 2^20 x 25 191 -> 175, c128 2^18 x 41 156 -> 143: it is
@@ -183,7 +183,9 @@ constexpr XcdEntry make_xcd(int lag, int ring, int per_cu, Radices<RA...>, Radic
 // Where a length is listed twice, the first whose ring fits the workspace.
 // Radix 32 * 16 and 32 * 32 with 16 or 32 elements per thread against more
 // threads of fewer, ms at 1 GiB: 2^17 0.63 / 0.73, 2^18 0.64 / 0.67, 2^19 0.66 /
-// 0.91, 2^20 0.64 / 0.84 (16 * 4 * 16).
+// 0.91, 2^20 0.64 / 0.84 (16 * 4 * 16).  c128 2^15 with 16 sequences a tile
+// instead of 8: half the turns of the XCD's counters, which bound its 16 KB
+// tiles (x 105 61.3 -> 56.0 us, where two launches take 56.2; x 2000 684 -> 627).
 const XcdEntry kXcd[] = {
     make_xcd<float, 256, 256, 16, 256, 4>(10, 18, 4, Radices<16, 16>{}, Radices<16, 16>{}),
     make_xcd<float, 256, 512, 16, 256, 4>(5, 10, 4, Radices<16, 16>{}, Radices<32, 16>{}),
@@ -191,7 +193,7 @@ const XcdEntry kXcd[] = {
     make_xcd<float, 1024, 512, 16, 512, 4>(3, 6, 2, Radices<32, 32>{}, Radices<16, 2, 16>{}),
     make_xcd<float, 1024, 1024, 16, 512, 4>(2, 4, 2, Radices<32, 32>{}, Radices<32, 32>{}),
     make_xcd<float, 1024, 1024, 16, 512, 4>(1, 3, 2, Radices<32, 32>{}, Radices<32, 32>{}),
-    make_xcd<double, 128, 256, 8, 128, 3>(6, 12, 4, Radices<8, 2, 8>{}, Radices<16, 16>{}),
+    make_xcd<double, 128, 256, 16, 256, 3>(7, 12, 3, Radices<8, 2, 8>{}, Radices<16, 16>{}),
     make_xcd<double, 256, 256, 8, 128, 3>(10, 16, 4, Radices<16, 16>{}, Radices<16, 16>{}),
     make_xcd<double, 256, 512, 8, 256, 2>(4, 8, 2, Radices<8, 4, 8>{}, Radices<16, 2, 16>{}),
     make_xcd<double, 512, 512, 8, 256, 2>(2, 5, 2, Radices<16, 2, 16>{}, Radices<16, 2, 16>{}),

@@ -12,7 +12,7 @@ import torch
 
 import oracle_lib as O
 from genfft_amd import _capi as C
-from test_capi_cpu import desc, explain
+from test_capi_cpu import desc, explain, field
 
 PREC = {"c64": (C.GFFT_F32, np.complex64, torch.complex64, O.tol_c64),
         "c128": (C.GFFT_F64, np.complex128, torch.complex128, O.tol_c128)}
@@ -39,6 +39,20 @@ def test_route(monkeypatch):
         assert "xcd" not in explain(d)[1]
     monkeypatch.setenv("GFFT_N1_LOG2", "7")
     assert "xcd" not in explain(desc(C.GFFT_C2C, 0, 1 << 16, 0, 600))[1]
+
+
+@pytest.mark.parametrize("prec,n,batch,lens,m,ring,lag", [
+    (0, 1 << 16, 300, "256,256", 16, 18, 10), (0, 1 << 17, 100, "256,512", 16, 10, 5), (0, 1 << 18, 100, "512,512", 16, 10, 6),
+    (0, 1 << 19, 64, "1024,512", 16, 6, 3), (0, 1 << 20, 128, "1024,1024", 16, 4, 2), (0, 1 << 20, 26, "1024,1024", 16, 3, 1),
+    (1, 1 << 15, 105, "128,256", 16, 12, 7), (1, 1 << 16, 140, "256,256", 8, 16, 10), (1, 1 << 17, 70, "256,512", 8, 8, 4),
+    (1, 1 << 18, 64, "512,512", 8, 5, 2)])
+def test_shape(prec, n, batch, lens, m, ring, lag):
+    """The one launch a batch runs, ahead of the launches for overlapping buffers."""
+    st, text = explain(desc(C.GFFT_C2C, prec, n, 0, batch))
+    lines = text.split("on overlapping buffers:")[0].splitlines()[1:]
+    assert st == 0 and len(lines) == 1 and lines[0].startswith("xcd_four_step ")
+    assert [field(lines[0], k) for k in ("L", "M", "batch", "ring", "lag", "in", "out", "first", "last")] == [
+        lens, str(m), str(batch), str(ring), str(lag), "in+0", "out+0", "1", "1"]
 
 
 HIPCC = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
