@@ -27,8 +27,26 @@ struct XcdEntry {
     KernelEntry col, row;  // shapes (for their twiddle tables and the bounds proof)
     int NT, lds_bytes;
     int lag, ring, per_cu;  // chosen per length, see kern_xcd.hip
-    void (*fn)(XcdArgs);
+    // The kernel by its cache hints: XCD_PLAIN_LD / XCD_PLAIN_ST are the column
+    // tiles' loads / the row tiles' stores not streamed (null: not compiled).
+    void (*fn[4])(XcdArgs);
+    int plain;               // the hints taken where a side's runs share lines (xcd_hints)
+    int64_t out_least, both_least;  // bytes a side from which it is taken there (-1: never)
 };
+
+enum : int { XCD_PLAIN_LD = 1, XCD_PLAIN_ST = 2 };
+
+// The hints of a launch of `bytes` a side whose runs start at multiples of `in`
+// and `out` bytes (or any addresses with their low bits), or -1: two launches.
+// Streamed loads want whole 128-byte lines, streamed stores whole 32-byte
+// sectors; see kern_xcd.hip for the figures.
+inline int xcd_hints(const XcdEntry &e, int64_t bytes, uint64_t in, uint64_t out)
+{
+    const bool in_parts = in % 128 != 0, out_parts = out % 32 != 0;
+    const int64_t least = out_parts ? (in_parts ? e.both_least : e.out_least) : 0;
+    if (least < 0 || bytes < least) return -1;
+    return e.plain & ((in_parts ? XCD_PLAIN_LD : 0) | (out_parts ? XCD_PLAIN_ST : 0));
+}
 
 const XcdEntry *xcd_entries(int *count);
 hipError_t launch_xcd_reset(uint32_t *state, int64_t words, hipStream_t s);

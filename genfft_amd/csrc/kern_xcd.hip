@@ -70,6 +70,12 @@ constexpr int plane_of(Radices<RA...>, Radices<RB...>)
     return a > b ? a : b;
 }
 
+template <typename T, int L, int M, int NT, int INP, int... RS>
+constexpr KernelEntry shape_of(Radices<RS...>)
+{
+    return reg_shape<T, L, M, NT, INP, PAT_COL, RS...>();
+}
+
 template <typename T, int L, int M, int NT, int INP, int HINT, int... RS>
 __device__ __forceinline__ void tile_of(T *plane, const TileArgs &a, const cx<T> *in, cx<T> *out, int s0, int o,
                                         int tid, Radices<RS...>)
@@ -99,7 +105,7 @@ __device__ __forceinline__ void tile_of(T *plane, const TileArgs &a, const cx<T>
 // 73.2 / 632, 186 / 644, 105 / 667 with an agent-scope invalidate (buffer_inv sc1)
 // by the thread that saw the count instead, and c64 2^20 794 with one by every
 // wave.  A workgroup-scope invalidate (sc0) need not drop those lines.
-template <typename T, int N1, int N2, int M, int NT, int WPE, class RA, class RB>
+template <typename T, int N1, int N2, int M, int NT, int WPE, int PLAIN, class RA, class RB>
 __global__ void __launch_bounds__(NT, WPE) xcd_fft_kernel(XcdArgs x)
 {
     constexpr int T1 = N2 / M, T2 = N1 / M;
@@ -141,12 +147,12 @@ __global__ void __launch_bounds__(NT, WPE) xcd_fft_kernel(XcdArgs x)
         if (g >= 0) {
             cx<T> *const slot = ring + (int64_t)(c % x.ring) * N;
             if (r < T1) {
-                tile_of<T, N1, M, NT, PAT_COL, HINT_LD>(
+                tile_of<T, N1, M, NT, PAT_COL, (PLAIN & XCD_PLAIN_LD) ? HINT_NONE : HINT_LD>(
                     plane, x.col, reinterpret_cast<const cx<T> *>(x.col.in) + in_base(x.col, 0, g), slot, r * M, g, tid,
                     RA{});
                 asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             } else {
-                tile_of<T, N2, M, NT, PAT_ROW, HINT_ST | HINT_AGENT>(
+                tile_of<T, N2, M, NT, PAT_ROW, HINT_AGENT | ((PLAIN & XCD_PLAIN_ST) ? HINT_NONE : HINT_ST)>(
                     plane, x.row, slot, reinterpret_cast<cx<T> *>(x.row.out) + out_base(x.row, 0, g), (r - T1) * M, g,
                     tid, RB{});
             }
@@ -163,20 +169,28 @@ __global__ void __launch_bounds__(256) xcd_reset_kernel(uint32_t *state, int64_t
 }
 
 // WPE: waves per SIMD the registers are budgeted for
-template <typename T, int N1, int N2, int M, int NT, int WPE, int... RA, int... RB>
-constexpr XcdEntry make_xcd(int lag, int ring, int per_cu, Radices<RA...>, Radices<RB...>)
+template <typename T, int N1, int N2, int M, int NT, int WPE, int PLAIN, class RA, class RB>
+constexpr XcdEntry make_xcd(int lag, int ring, int per_cu, RA ra, RB rb, int64_t out_least = 0, int64_t both_least = 0)
 {
     XcdEntry e{};
     e.prec = sizeof(T) == 8 ? 1 : 0;
     for (int n = N1 * N2; n > 1; n >>= 1) e.lg++;
-    e.col = reg_shape<T, N1, M, NT, PAT_COL, PAT_COL, RA...>();
-    e.row = reg_shape<T, N2, M, NT, PAT_ROW, PAT_COL, RB...>();
+    e.col = shape_of<T, N1, M, NT, PAT_COL>(ra);
+    e.row = shape_of<T, N2, M, NT, PAT_ROW>(rb);
     e.NT = NT;
-    e.lds_bytes = plane_of<T, N1, N2, M>(Radices<RA...>{}, Radices<RB...>{}) * (int)sizeof(T);
+    e.lds_bytes = plane_of<T, N1, N2, M>(ra, rb) * (int)sizeof(T);
     e.lag = lag;
     e.ring = ring;
     e.per_cu = per_cu;
-    e.fn = &xcd_fft_kernel<T, N1, N2, M, NT, WPE, Radices<RA...>, Radices<RB...>>;
+    e.plain = PLAIN;
+    e.out_least = out_least;
+    e.both_least = both_least;
+    e.fn[0] = &xcd_fft_kernel<T, N1, N2, M, NT, WPE, 0, RA, RB>;
+    e.fn[XCD_PLAIN_ST] = &xcd_fft_kernel<T, N1, N2, M, NT, WPE, XCD_PLAIN_ST, RA, RB>;  // Builder's kXcdKeptBytes too
+    if constexpr ((PLAIN & XCD_PLAIN_LD) != 0) {
+        e.fn[XCD_PLAIN_LD] = &xcd_fft_kernel<T, N1, N2, M, NT, WPE, XCD_PLAIN_LD, RA, RB>;
+        e.fn[XCD_PLAIN_LD | XCD_PLAIN_ST] = &xcd_fft_kernel<T, N1, N2, M, NT, WPE, XCD_PLAIN_LD | XCD_PLAIN_ST, RA, RB>;
+    }
     return e;
 }
 
@@ -186,17 +200,33 @@ constexpr XcdEntry make_xcd(int lag, int ring, int per_cu, Radices<RA...>, Radic
 // 0.91, 2^20 0.64 / 0.84 (16 * 4 * 16).  c128 2^15 with 16 sequences a tile
 // instead of 8: half the turns of the XCD's counters, which bound its 16 KB
 // tiles (x 105 61.3 -> 56.0 us, where two launches take 56.2; x 2000 684 -> 627).
+//
+// Layouts whose runs share lines (xcd_hints): two launches / streamed / plain
+// loads / plain stores / both plain, us, for 1 element between the inputs, the
+// outputs, or 3 and 5 (the sides' alignment decides, not the numbers):
+//   c64 2^16 x 300   130 / 129 / 121 / 129 / 122   147 / 144 / 154 / 134 / 131   148 / 158 / 154 / 152 / 134
+//   c64 2^18 x 200   318 / 335 / 308 / 332 / 323   396 / 439 / 425 / 381 / 426   400 / 487 / 441 / 442 / 443
+//   c64 2^19 x 120   408 / 386 / 376 / 404 / 395   487 / 472 / 512 / 500 / 523   494 / 535 / 548 / 578 / 539
+//   c64 2^20 x 60    447 / 373 / 397 / 443 / 407   518 / 478 / 598 / 542 / 540   547 / 538 / 611 / 614 / 552
+//   c128 2^16 x 140  135 / 123 / 117 / 128 / 127   148 / 158 / 160 / 144 / 141   150 / 172 / 162 / 162 / 147
+//   c128 2^18 x 100  342 / 337 / 327 / 331 / 342   410 / 362 / 348 / 333 / 385   413 / 400 / 364 / 387 / 405
+// 2^18 and 2^19 write an odd output side in two launches below 400 / 480 MiB and
+// where the input's is odd as well; c128 2^18 x 44 (176 MiB) 184 / 198 with both
+// odd.  Outputs in whole 32-byte sectors want streamed stores whatever else
+// (c64 2^17 x 300, 4 elements apart: 332 / 224).
+constexpr int LD = XCD_PLAIN_LD, ST = XCD_PLAIN_ST;
+constexpr int64_t MiB = 1 << 20;
 const XcdEntry kXcd[] = {
-    make_xcd<float, 256, 256, 16, 256, 4>(10, 18, 4, Radices<16, 16>{}, Radices<16, 16>{}),
-    make_xcd<float, 256, 512, 16, 256, 4>(5, 10, 4, Radices<16, 16>{}, Radices<32, 16>{}),
-    make_xcd<float, 512, 512, 16, 256, 4>(6, 10, 4, Radices<32, 16>{}, Radices<32, 16>{}),
-    make_xcd<float, 1024, 512, 16, 512, 4>(3, 6, 2, Radices<32, 32>{}, Radices<16, 2, 16>{}),
-    make_xcd<float, 1024, 1024, 16, 512, 4>(2, 4, 2, Radices<32, 32>{}, Radices<32, 32>{}),
-    make_xcd<float, 1024, 1024, 16, 512, 4>(1, 3, 2, Radices<32, 32>{}, Radices<32, 32>{}),
-    make_xcd<double, 128, 256, 16, 256, 3>(7, 12, 3, Radices<8, 2, 8>{}, Radices<16, 16>{}),
-    make_xcd<double, 256, 256, 8, 128, 3>(10, 16, 4, Radices<16, 16>{}, Radices<16, 16>{}),
-    make_xcd<double, 256, 512, 8, 256, 2>(4, 8, 2, Radices<8, 4, 8>{}, Radices<16, 2, 16>{}),
-    make_xcd<double, 512, 512, 8, 256, 2>(2, 5, 2, Radices<16, 2, 16>{}, Radices<16, 2, 16>{}),
+    make_xcd<float, 256, 256, 16, 256, 4, LD | ST>(10, 18, 4, Radices<16, 16>{}, Radices<16, 16>{}),
+    make_xcd<float, 256, 512, 16, 256, 4, LD | ST>(5, 10, 4, Radices<16, 16>{}, Radices<32, 16>{}),
+    make_xcd<float, 512, 512, 16, 256, 4, LD | ST>(6, 10, 4, Radices<32, 16>{}, Radices<32, 16>{}, 400 * MiB, -1),
+    make_xcd<float, 1024, 512, 16, 512, 4, LD>(3, 6, 2, Radices<32, 32>{}, Radices<16, 2, 16>{}, 480 * MiB, -1),
+    make_xcd<float, 1024, 1024, 16, 512, 4, 0>(2, 4, 2, Radices<32, 32>{}, Radices<32, 32>{}),
+    make_xcd<float, 1024, 1024, 16, 512, 4, LD | ST>(1, 3, 2, Radices<32, 32>{}, Radices<32, 32>{}),
+    make_xcd<double, 128, 256, 16, 256, 3, 0>(7, 12, 3, Radices<8, 2, 8>{}, Radices<16, 16>{}),
+    make_xcd<double, 256, 256, 8, 128, 3, LD | ST>(10, 16, 4, Radices<16, 16>{}, Radices<16, 16>{}),
+    make_xcd<double, 256, 512, 8, 256, 2, LD | ST>(4, 8, 2, Radices<8, 4, 8>{}, Radices<16, 2, 16>{}),
+    make_xcd<double, 512, 512, 8, 256, 2, LD | ST>(2, 5, 2, Radices<16, 2, 16>{}, Radices<16, 2, 16>{}, 0, 256 * MiB),
 };
 
 }  // namespace

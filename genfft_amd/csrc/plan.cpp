@@ -557,6 +557,8 @@ struct Launch {
     const XcdEntry *xe = nullptr;
     XcdArgs xa{};
     int64_t state_off = 0;  // bytes
+    int64_t xcd_bytes = 0;  // a side
+    uint64_t in_steps = 0, out_steps = 0;  // byte distances between the runs, or'ed (xcd_hints)
     bool reads(int buf) const { return in_buf == buf || (type == LT_DUAL && in_buf_b == buf) || (type == LT_XCD && buf == B_SCR); }
     bool writes(int buf) const { return out_buf == buf || (type == LT_DUAL && out_buf_b == buf); }
 };
@@ -687,6 +689,10 @@ constexpr int64_t kStreamBytes = (int64_t)512 << 20;
 // stored plain, to be found in the Infinity Cache (MI355X, us streamed / plain:
 // c64 2^21 x 8, 128 MiB, 122 / 114, x 16 231 / 242, x 32 441 / 481).
 constexpr int64_t kKeptBytes = (int64_t)192 << 20;
+// The same for a one-launch four-step (c64 2^16 x 200, 100 MiB, whose result an
+// unpack reads: 155 / 147 us, c128 2^15 x 200 154 / 140; c128 2^16 x 150, 150
+// MiB, 207 / 217).
+constexpr int64_t kXcdKeptBytes = (int64_t)128 << 20;
 // The row pass of a 2D plan, whose columns run in place, stores plain up to
 // here (c64 1024^2 x 36, 288 MiB: 234 / 210 us, x 96 602 / 581, x 256, 2 GiB,
 // 1613 / 1621) ...
@@ -956,9 +962,17 @@ struct Builder {
         const int64_t N1 = (int64_t)1 << l1, N2 = (int64_t)1 << l2;
         if (N1 > max_len(prec, PAT_COL, PAT_COL, store) || N2 > max_len(prec, PAT_ROW, PAT_COL, store))
             return fail(GFFT_ERR_UNSUPPORTED, "length %lld exceeds the two-pass limit", (long long)n);
-        if (const XcdEntry *e = xcd_entry(n, batch); e && in_buf != B_SCR && out_buf != B_SCR) {
+        const uint64_t in_steps = (uint64_t)((in_off | in_dist) * (int64_t)csize);
+        const uint64_t out_steps = (uint64_t)((out_off | out_dist) * (int64_t)csize);
+        if (const XcdEntry *e = xcd_entry(n, batch, in_steps, out_steps); e && in_buf != B_SCR && out_buf != B_SCR) {
             long_rows = true;
-            return xcd_four_step(*e, batch, in_buf, in_off, in_dist, out_buf, out_off, out_dist, first, last);
+            const int st = xcd_four_step(*e, batch, in_buf, in_off, in_dist, out_buf, out_off, out_dist, first, last);
+            if (st) return st;
+            Launch &l = p->launches.back();
+            l.in_steps = in_steps;
+            l.out_steps = out_steps;
+            l.plain = (!last || p->d.kind == GFFT_R2C) && l.xcd_bytes <= kXcdKeptBytes;  // read again by the plan
+            return GFFT_OK;
         }
         if (opts.dual && !store) {
             const int st = four_step_dual(n, N1, N2, batch, in_buf, in_off, in_dist, out_buf, out_off, out_dist, first,
@@ -1001,7 +1015,7 @@ struct Builder {
     {
         int per_cu = e.per_cu;
         int most = 0;
-        if (!dry && hipOccupancyMaxActiveBlocksPerMultiprocessor(&most, (const void *)e.fn, e.NT, 0) == hipSuccess)
+        if (!dry && hipOccupancyMaxActiveBlocksPerMultiprocessor(&most, (const void *)e.fn[0], e.NT, 0) == hipSuccess)
             per_cu = std::min(per_cu, std::max(1, most));
         const int64_t tasks = batch * (e.col.L / e.col.M + e.row.L / e.row.M);
         return std::min<int64_t>((int64_t)per_cu * std::max(1, p->num_cus), tasks);
@@ -1012,8 +1026,9 @@ struct Builder {
         return *state_off + 4 * xcd_state_words(xcd_blocks(batch, e.lag, (int64_t)e.per_cu * p->num_cus));
     }
 
-    // Both passes of a four-step of length n in one launch, or null.
-    const XcdEntry *xcd_entry(int64_t n, int64_t batch) const
+    // Both passes of a four-step of length n in one launch, or null; in_steps /
+    // out_steps: the byte distances between transforms, or'ed.
+    const XcdEntry *xcd_entry(int64_t n, int64_t batch, uint64_t in_steps, uint64_t out_steps) const
     {
         if (store || no_long_rows || opts.dual || opts.two_launches || opts.n1_log2 || opts.col_m || opts.row_m || opts.pipe_mask != 3 ||
             opts.row_variant >= 0)
@@ -1023,6 +1038,7 @@ struct Builder {
         for (int i = 0; i < cnt; i++) {
             if (tab[i].prec != prec || ((int64_t)1 << tab[i].lg) != n) continue;
             int64_t off;
+            if (xcd_hints(tab[i], batch * n * (int64_t)csize, in_steps, out_steps) < 0) continue;
             // within the workspace the two launches would have had
             if (xcd_scratch(tab[i], batch, &off) <= std::min(batch * n * (int64_t)csize, chunk_bytes())) return &tab[i];
         }
@@ -1074,6 +1090,7 @@ struct Builder {
         r.out_outer = out_dist;
         r.out_inner = 1;
         r.out_elem = N1;
+        l.xcd_bytes = batch * n * (int64_t)csize;
         l.xa.batch = (int32_t)batch;
         l.xa.lag = e.lag;
         l.xa.ring = e.ring;
@@ -2134,13 +2151,17 @@ int run_launches(const std::vector<Launch> &launches, int prec, int xcd_remap, c
 // to be staged.
 const std::vector<Launch> &route(const gfft_plan_s *p, const void *in, const void *out, bool *stage)
 {
-    *stage = false;
-    if (!p->overlap_hazard) return p->launches;
     const uintptr_t i0 = (uintptr_t)in, o0 = (uintptr_t)out;
-    if (!(i0 < o0 + p->out_bytes && o0 < i0 + p->in_bytes)) return p->launches;
-    if (i0 == o0 && p->in_step == p->out_step && p->in_step2 == p->out_step2) return p->launches;
-    *stage = p->alt.empty() || p->alt_hazard;
-    return p->alt.empty() ? p->launches : p->alt;
+    const bool shifted = i0 < o0 + p->out_bytes && o0 < i0 + p->in_bytes &&
+                         !(i0 == o0 && p->in_step == p->out_step && p->in_step2 == p->out_step2);
+    bool alt = p->overlap_hazard && shifted;
+    for (const Launch &l : p->launches)  // buffers whose alignment is the two launches' case
+        if (l.type == LT_XCD)
+            alt = alt || xcd_hints(*l.xe, l.xcd_bytes, l.in_steps | (l.in_buf == B_IN ? i0 : o0),
+                                   l.out_steps | (l.out_buf == B_OUT ? o0 : i0)) < 0;
+    alt = alt && !p->alt.empty();
+    *stage = shifted && (alt ? p->alt_hazard : p->overlap_hazard);
+    return alt ? p->alt : p->launches;
 }
 
 // Whether the plan's one launch holds every transform whole in a workgroup's
@@ -2255,8 +2276,12 @@ int run_launches(const std::vector<Launch> &launches, int prec, int xcd_remap, c
             a.row.swap_out = inv && l.last;
             a.state = (uint32_t *)((char *)scratch + l.state_off);
             HIP_TRY(launch_xcd_reset(a.state, xcd_state_words(a.blocks), s));
+            // (a batch plan, which has no two launches instead, keeps the one)
+            int hints = xcd_hints(*l.xe, l.xcd_bytes, l.in_steps | (uintptr_t)ip, l.out_steps | (uintptr_t)op);
+            if (hints < 0) hints = l.xe->plain;
+            if (l.plain) hints |= XCD_PLAIN_ST;
             void *args[] = {&a};
-            HIP_TRY(hipExtLaunchKernel((const void *)l.xe->fn, dim3((unsigned)l.grid), dim3(l.xe->NT), args, 0, s,
+            HIP_TRY(hipExtLaunchKernel((const void *)l.xe->fn[hints], dim3((unsigned)l.grid), dim3(l.xe->NT), args, 0, s,
                                        nullptr, tail, 0));
             if (tail && stopped) *stopped = true;
             break;
@@ -2569,9 +2594,16 @@ int build_batch(gfft_batch_plan_s *p)
             set_jobs(c.first, true, true);
             continue;
         }
-        if (const XcdEntry *e = b.xcd_entry(L, c.count)) {
+        uint64_t in_steps = 0, out_steps = 0;  // the jobs' offsets, bytes
+        for (int64_t k = c.first; k < c.first + c.count; k++) {
+            in_steps |= (uint64_t)jin[k] * cs;
+            out_steps |= (uint64_t)jout[k] * cs;
+        }
+        if (const XcdEntry *e = b.xcd_entry(L, c.count, in_steps, out_steps)) {
             if ((st = b.xcd_four_step(*e, c.count, B_IN, 0, 0, B_OUT, 0, 0, false, false))) return st;
             Launch &l = tmp.launches.back();
+            l.in_steps = in_steps;
+            l.out_steps = out_steps;
             l.ta.job_in = p->d_job_in;
             l.tb.job_out = p->d_job_out;
             l.ta.job_inv = l.tb.job_inv = p->d_job_inv;

@@ -281,3 +281,50 @@ def test_two_plans_at_once(gpu):
     for i in (0, 1):
         for k in range(3):
             assert torch.equal(y[i][k], ref[i])  # the same kernel on the same input
+
+
+def test_layouts_whose_runs_share_lines():
+    """Distances that leave the runs on parts of lines: taken but where the two
+    launches are faster (complex64 2^18 and 2^19 with odd output distances)."""
+    def one(prec, n, batch, pin, pout):
+        st, text = explain(desc(C.GFFT_C2C, prec, n, 0, batch, ind=n + pin, outd=n + pout))
+        assert st == 0
+        return "xcd_four_step" in text
+    for n, small, large in ((1 << 18, 130, 250), (1 << 19, 80, 130)):
+        assert one(0, n, small, 0, 0) and one(0, n, small, 1, 0) and one(0, n, small, 0, 4)
+        assert not one(0, n, small, 0, 1) and one(0, n, large, 0, 1)
+        assert not one(0, n, small, 3, 5) and not one(0, n, large, 3, 5)
+    for prec, n, batch in ((0, 1 << 16, 146), (0, 1 << 17, 82), (0, 1 << 20, 26), (1, 1 << 15, 98), (1, 1 << 16, 130),
+                           (1, 1 << 17, 66)):
+        assert one(prec, n, batch, 0, 1) and one(prec, n, batch, 3, 5)
+    assert one(1, 1 << 18, 42, 0, 1) and not one(1, 1 << 18, 42, 3, 5) and one(1, 1 << 18, 70, 3, 5)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("pin,pout,shift_in,shift_out", [(1, 0, 0, 0), (0, 1, 0, 0), (3, 5, 0, 0), (4, 4, 0, 0), (0, 0, 1, 0),
+                                                         (0, 0, 0, 1), (0, 0, 3, 2)])
+@pytest.mark.parametrize("prec,n,batch", [("c64", 1 << 16, 150), ("c64", 1 << 17, 90), ("c64", 1 << 18, 90), ("c64", 1 << 19, 52),
+                                          ("c64", 1 << 20, 28), ("c64", 1 << 20, 40), ("c128", 1 << 15, 105),
+                                          ("c128", 1 << 16, 140), ("c128", 1 << 17, 70), ("c128", 1 << 18, 44)])
+def test_alignments(gpu, monkeypatch, prec, n, batch, pin, pout, shift_in, shift_out):
+    """Odd distances and odd base addresses, whichever kernel they take, against
+    the two launches on whole lines."""
+    import genfft_amd as G
+    p, ndt, tdt, tol = PREC[prec]
+    v = _gpu_rand((batch, n), tdt, n)
+    x = torch.zeros(shift_in + batch * (n + pin), dtype=tdt, device=gpu)[shift_in:]
+    x.view(batch, n + pin)[:, :n] = v
+    y = torch.full((shift_out + batch * (n + pout),), 7 + 5j, dtype=tdt, device=gpu)
+    out = y[shift_out:]
+    plan = G.Plan(C.GFFT_C2C, n, precision=p, batch=batch, in_dist=n + pin, out_dist=n + pout)
+    plan.execute(x, out)
+    ref = torch.empty_like(v)
+    monkeypatch.setenv("GFFT_DUAL", "0")
+    G.Plan(C.GFFT_C2C, n, precision=p, batch=batch).execute(v, ref)
+    got = out.view(batch, n + pout)
+    assert _worst(got[:, :n], ref) <= 2 * tol(n)
+    assert bool((y[:shift_out] == 7 + 5j).all()) and bool((got[:-1, n:] == 7 + 5j).all())
+    # an odd output base of 2^18 and 2^19 runs as two launches
+    two = shift_out and prec == "c64" and n in (1 << 18, 1 << 19)
+    if not pin and not pout:
+        assert len(plan.profile(x, out)) == (2 if two else 1)
