@@ -2045,7 +2045,7 @@ int describe_launches(const std::vector<Launch> &launches, const std::string &he
             snprintf(line, sizeof(line),
                      "%s L=%d M=%d NT=%d layout=%d inp=%d outp=%d lds=%d pipe=%d grid=%lld rad=%d,%d,%d,%d tiles=%d "
                      "n_inner=%d tiles_inner=%d n_outer1=%d in=%s+%lld out=%s+%lld "
-                     "in_strides=%lld,%lld,%lld,%lld out_strides=%lld,%lld,%lld,%lld tw=%d first=%d last=%d vin=%d vout=%d runs=%d\n",
+                     "in_strides=%lld,%lld,%lld,%lld out_strides=%lld,%lld,%lld,%lld tw=%d first=%d last=%d vin=%d vout=%d runs=%d lines=%d plain=%d\n",
                      l.k->long_row ? "long_row" : "tile", l.k->L, l.k->M, l.k->NT, l.k->layout, l.k->inp, l.k->outp,
                      l.k->lds_bytes, l.k->persistent, (long long)l.grid, l.k->rad[0],
                      l.k->nrad > 1 ? l.k->rad[1] : 0, l.k->nrad > 2 ? l.k->rad[2] : 0,
@@ -2053,7 +2053,8 @@ int describe_launches(const std::vector<Launch> &launches, const std::string &he
                      bn[l.in_buf], (long long)l.in_off, bn[l.out_buf], (long long)l.out_off,
                      (long long)a.in_outer2, (long long)a.in_outer, (long long)a.in_inner, (long long)a.in_elem,
                      (long long)a.out_outer2, (long long)a.out_outer, (long long)a.out_inner,
-                     (long long)a.out_elem, a.tw_mode, (int)l.first, (int)l.last, (int)l.vin_ok, (int)l.vout_ok, a.runs);
+                     (long long)a.out_elem, a.tw_mode, (int)l.first, (int)l.last, (int)l.vin_ok, (int)l.vout_ok, a.runs, (int)l.own_lines,
+                     (int)l.plain);
             break;
         }
         case LT_DUAL: {
@@ -2574,6 +2575,17 @@ int build_batch(gfft_batch_plan_s *p)
         Launch &l = tmp.launches.back();
         if (in_side) l.vin_ok = l.vin_ok && p->offsets_even;
         if (out_side) l.vout_ok = l.vout_ok && p->offsets_even;
+        // column-side runs start where the jobs do (register-held tiles; own_lines
+        // came from distances of 0)
+        uint64_t in = 0, out = 0;
+        for (int64_t k = first; k < first + a.n_outer1; k++) {
+            in |= (uint64_t)jin[k] * cs;
+            out |= (uint64_t)jout[k] * cs;
+        }
+        const bool in_lines = !in_side || l.k->inp == PAT_ROW || in % 128 == 0;
+        const bool out_lines = !out_side || l.k->outp == PAT_ROW || out % 128 == 0;
+        l.own_lines = l.own_lines && in_lines && out_lines;
+        l.plain = l.plain || (l.k->fn_plain && !out_lines);
     };
     int cnt = 0;
     const KernelEntry *tab = tile_table(prec, 0, &cnt);

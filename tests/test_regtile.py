@@ -326,3 +326,30 @@ def test_small_batches_of_long_transforms_keep_the_narrow_columns(kind, prec, n,
         st, text = explain(desc(kind, prec, n, 0, batch, flags=C.GFFT_FLAG_HALF if kind == C.GFFT_R2C else 0))
         cols = [t for t in tiles(text) if field(t, "L") == "2048" and field(t, "inp") == "1"]
         assert st == 0 and [field(t, "M") for t in cols] == [m], text
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("prec,n,gap,lines", [("c64", 1 << 21, 0, True), ("c64", 1 << 21, 16, True), ("c64", 1 << 21, 1, False),
+                                              ("c64", 1 << 22, 5, False), ("c128", 1 << 20, 8, True), ("c128", 1 << 21, 3, False)])
+def test_uneven_jobs_place_the_runs(gpu, prec, n, gap, lines):
+    """The register-held column sides of a batch's four-steps know from the jobs'
+    offsets whether their runs cover whole lines: odd ones are stored plain."""
+    import genfft_amd as G
+    p, ndt, tdt, tol = PREC[prec]
+    count = 10
+    offs = np.arange(count) * (n + gap)
+    x = torch.randn(count * (n + gap), dtype=tdt, device=gpu)
+    y = torch.zeros_like(x)
+    plan = G.UnevenBatch([n] * count, offs.tolist(), offs.tolist(), [False] * count, tdt)
+    text = plan.describe()
+    for t in tiles(text):
+        reg_side = field(t, "L") == "2048"  # 512- and 1024-point passes keep the LDS tiles here
+        if reg_side and field(t, "outp") == "1" and field(t, "inp") == "0":
+            assert (field(t, "lines"), field(t, "plain")) == (("1", "0") if lines else ("0", "1")), t
+        elif reg_side:
+            assert field(t, "lines") == ("1" if lines else "0"), t
+    assert any(field(t, "L") == "2048" for t in tiles(text)) or n < 1 << 21
+    plan.execute(x, y)
+    idx = torch.from_numpy(offs[[0, count - 1]])[:, None].to(gpu) + torch.arange(n, device=gpu)
+    ref = O.fft_ld(x[idx].cpu().numpy().astype(np.complex128))
+    assert O.rel_l2_rows(y[idx].cpu().numpy(), ref).max() <= tol(n)
