@@ -320,7 +320,10 @@ __device__ __forceinline__ void reg_tile(T *plane, const TileArgs &a, const cx<T
         const char *ib = reinterpret_cast<const char *>(in);
 #pragma unroll
         for (int q = 0; q < A::N; q++) {
-            const int s = A::s(tid, q), j = A::j(tid, q);
+            // a sequence past the last one is computed on that one's elements
+            // and not stored (a branch around each load instead made the one
+            // partly filled tile the slowest: c64 4096 x 107 columns 20.3 us)
+            const int s = min(A::s(tid, q), nvalid - 1), j = A::j(tid, q);
             const uint32_t to = (INP == PAT_ROW ? (uint32_t)s * (uint32_t)a.in_inner + (uint32_t)j
                                                 : (uint32_t)j * (uint32_t)a.in_elem + (uint32_t)s) * (uint32_t)sizeof(cx<T>);
             cx<T> *x = &v[q * A::W * R1];
@@ -335,15 +338,17 @@ __device__ __forceinline__ void reg_tile(T *plane, const TileArgs &a, const cx<T
 #pragma unroll
             for (int r = 0; r < R1; r++) {
                 const cx<T> *p = reinterpret_cast<const cx<T> *>(ib + r * step + to);
-                if (M == 1 || nvalid == M) {
+                if (A::W == 1 || nvalid == M) {
                     reg_load<HINT, A::W>(p, x + r, R1);
                 } else {
-                    // a sequence past the last one is computed on zeros and not stored
-#pragma unroll
-                    for (int e = 0; e < A::W; e++) {
-                        x[e * R1 + r] = {(T)0, (T)0};
-                        if (s + e < nvalid) x[e * R1 + r] = p[e];
-                    }
+                    // pairs stay one access: the last sequence alone is the second
+                    // of the pair before it (its partner's result is not stored)
+                    const bool one = s + 1 >= nvalid;
+                    cx<T> y[2];
+                    if (nvalid > 1) reg_load<HINT, 2>(p - one, y, 1);
+                    else reg_load<HINT, 1>(p, y + 1, 0);
+                    x[r] = one ? y[1] : y[0];
+                    x[R1 + r] = y[1];
                 }
             }
         }
@@ -394,10 +399,10 @@ __device__ __forceinline__ void reg_tile(T *plane, const TileArgs &a, const cx<T
                 cx<T> *p = reinterpret_cast<cx<T> *>(ob + r * step + to);
                 if (M == 1 || nvalid == M) {
                     reg_store<HINT, A::W>(p, x + r, RL);
-                } else {
-#pragma unroll
-                    for (int e = 0; e < A::W; e++)
-                        if (s + e < nvalid) p[e] = x[e * RL + r];
+                } else if (A::W == 2 && s + 1 < nvalid) {
+                    reg_store<HINT_NONE, A::W>(p, x + r, RL);
+                } else if (s < nvalid) {
+                    *p = x[r];
                 }
             }
         }
