@@ -34,6 +34,7 @@ struct KernelEntry {
     int64_t most;    // cols, cached: bytes a side up to which it is taken (0: any)
     int64_t most_odd;  // cols: the same where rows of the matrix share lines
     int64_t least;   // cols: bytes a side from which it is taken
+    int one_round;   // cols: 1: also below, where its tiles are one full round of the CUs
     int cols;        // 1: column tile for whole column transforms only; 2: but not those of complex 2D planes
     int cached;      // 1: row tile the planner takes for batches within the Infinity Cache
     int long_row;    // 1: a row longer than the LDS row tiles (the planner takes it by its own rule)
@@ -218,6 +219,7 @@ constexpr KernelEntry make_reg_cols_big(int64_t least)
 {
     KernelEntry e = make_reg_cols<T, L, M, NT, RS...>();
     e.least = least;
+    e.one_round = least > 0;
     e.cols = 2;
     return e;
 }

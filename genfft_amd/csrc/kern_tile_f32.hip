@@ -143,7 +143,9 @@ const KernelEntry kTable[] = {
     // 22% full), 1024^2 x 16 images' columns 55 -> 42, 2048 x 2048 19.8 -> 17.1,
     // 4096 x 2049 58 -> 40, 4096 x 6000 154 -> 110.  4096 rows past 96 MiB
     // want 8 columns: two 4-column tiles per CU keep 8 MB of quarter lines in
-    // flight per XCD, twice its L2 (4096 x 4096: 135 us, LDS tile 105) ---
+    // flight per XCD, twice its L2 (4096 x 4096: 135 us, LDS tile 105); so do
+    // widths whose 8-column tiles are one round (x 2048 55 / 37.5, x 1400 31.1 /
+    // 26.8; x 2100, a second round of 7 tiles, 55.4 / 59.4) ---
     make_reg_many<T, 512, 16, 512, C_, C_, 16, 2, 16>(4),
     make_reg_many<T, 2048, 16, 1024, C_, C_, 16, 8, 16>(1),
     make_reg_cols<T, 64, 16, 128, 8, 8>(),

@@ -717,6 +717,14 @@ constexpr int64_t kFewRowsLeast = (int64_t)16 << 20;
 // Row batches of at most this many bytes a side take the `cached` row tiles
 // (c64 2048 points on MI355X: 64 MiB 59.8 -> 55.8 us, 128 MiB 101.3 -> 101.4).
 constexpr int64_t kCachedBytes = (int64_t)128 << 20;
+// Runs that start at half lines are streamed like whole ones, in tiles of at
+// least a line (us plain / streamed: c64 2048 rows x 5000 columns 59.7 / 47.9, 512 x
+// 12808 30.3 / 22.7, 256 x 5000 7.95 / 6.95, 128 x 9208 7.50 / 6.58; not 1024 x 5000,
+// 19.2 / 20.6, but x 5608, 43.8 MiB, 24.1 / 21.0), and between these sizes those at
+// quarter lines (128 x 9204 7.50 / 6.97, 256 x 5004 7.98 / 7.40; 64 x 12804, 6.3 MiB,
+// 4.89 / 4.94, 256 x 12804, 25 MiB, 13.2 / 15.3).
+constexpr int64_t kHalfLines1024 = (int64_t)40 << 20;
+constexpr int64_t kSectorsLeast = (int64_t)8 << 20, kSectorsMost = (int64_t)16 << 20;
 // Rows from which a register-held tile per row beats the four-step (MI355X, us
 // per call at 64 / 96 / 128 / 256 rows: c64 32768 points 18.1 / 18.3 / 19.5 /
 // 32 against 16.0 / 23.3 / 28 / 54, c128 16384 points 17.4 / 18.2 / 20.9 / 33
@@ -844,6 +852,11 @@ struct Builder {
             const bool out_lines = outp == PAT_ROW || (k->M * (int64_t)csize >= 128 && lines(out_elem) &&
                                                        lines(out_outer) && lines(out_outer2) && lines(out_off_el));
             const int64_t bytes = (int64_t)k->L * n_inner * n_outer1 * n_outer2 * (int64_t)csize;
+            // runs on parts of lines that are streamed all the same (kHalfLines1024)
+            const int64_t piece = bytes > kSectorsLeast && bytes <= kSectorsMost ? 32 : k->L == 1024 && bytes <= kHalfLines1024 ? 128 : 64;
+            auto pieces = [&](int64_t v) { return v * (int64_t)csize % piece == 0; };
+            const bool out_pieces = outp == PAT_ROW || (k->M * (int64_t)csize >= 128 && pieces(out_elem) && pieces(out_outer) &&
+                                                        pieces(out_outer2) && pieces(out_off_el));
             const bool row_pass = inp == PAT_ROW && outp == PAT_ROW && first && !last && p->d.kind == GFFT_C2C_2D;
             const bool dirty = row_pass && p->d.n2 <= kShortColumn && bytes > kDirtyLeast && bytes <= kDirtyMost;
             const bool near_rows = !first && in_buf == out_buf && bytes <= kOneL2Bytes && n_outer1 >= 8;
@@ -851,7 +864,7 @@ struct Builder {
             l.own_lines = (inp == PAT_COL || outp == PAT_COL) && in_lines && out_lines;
             l.row_order = near_rows || short_cols;
             l.plain = k->fn_plain &&
-                      (!out_lines || near_rows || (!last && !dirty && bytes <= (row_pass ? kKeptRowBytes : kKeptBytes)));
+                      (!out_pieces || near_rows || (!last && !dirty && bytes <= (row_pass ? kKeptRowBytes : kKeptBytes)));
         }
         if (k->persistent) {
             // one resident wave of workgroups looping over the tiles
@@ -1196,18 +1209,27 @@ struct Builder {
         int cnt = 0, best = -1;
         const KernelEntry *tab = tile_table(prec, 0, &cnt);
         auto tiles = [&](int m) { return (cols + m - 1) / m * batch; };
+        // A round of tiles that leaves up to a third of the CUs idle is the better
+        // one still where its runs cover whole lines (us narrower / wider: c64 256
+        // x 3968 columns, 248 of 16, 5.9 / 5.0, 512 x 2816, 176 of them, 8.8 / 7.2, 2048 x
+        // 1408 17.7 / 15.3; c128 1024 x 1408 14.0 / 12.7), but not of short columns
+        // (c128 128 x 2816 4.7 / 5.1, c64 64 x 11264 3.9 / 4.3) or planes (c64 2048
+        // x 256 x 13 44.8 / 52.9).
+        const bool idle = !plane && lines && (L >= 256 || (L == 128 && !prec));
+        const int64_t enough = idle || L == 4096 ? p->num_cus * 2 / 3 : p->num_cus;
         auto better = [&](int m, int than) {
-            const bool a = tiles(m) >= p->num_cus, b = tiles(than) >= p->num_cus;
+            const bool a = tiles(m) >= enough, b = tiles(than) >= enough;
             return a != b ? a : a ? m > than : m < than;
         };
         const int64_t bytes = cols * L * batch * (int64_t)csize;
         for (int i = 0; i < cnt; i++)
-            if (tab[i].cols && tab[i].cols <= (plane ? 1 : 2) && tab[i].L == L && bytes > tab[i].least - 1 &&
+            if (tab[i].cols && tab[i].cols <= (plane ? 1 : 2) && tab[i].L == L &&
+                (bytes >= tab[i].least || (tab[i].one_round && tiles(tab[i].M) >= enough && tiles(tab[i].M) <= p->num_cus)) &&
                 (!tab[i].most || bytes <= tab[i].most) && (lines || !tab[i].most_odd || bytes <= tab[i].most_odd) &&
                 (best < 0 || better(tab[i].M, tab[best].M))) best = i;
         if (best < 0) return -1;
         const KernelEntry *d = find_tile(prec, L, PAT_COL, PAT_COL, 0, opts.pipe_mask);
-        return d && d->M > tab[best].M && better(d->M, tab[best].M) ? -1 : best;
+        return d && d->M > tab[best].M && tiles(d->M) >= p->num_cus ? -1 : best;
     }
 
     // Column FFTs of length `rows` down `cols` columns, `batch` matrices.

@@ -353,3 +353,47 @@ def test_uneven_jobs_place_the_runs(gpu, prec, n, gap, lines):
     idx = torch.from_numpy(offs[[0, count - 1]])[:, None].to(gpu) + torch.arange(n, device=gpu)
     ref = O.fft_ld(x[idx].cpu().numpy().astype(np.complex128))
     assert O.rel_l2_rows(y[idx].cpu().numpy(), ref).max() <= tol(n)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("prec,n,m", [("c64", 64, 16), ("c64", 256, 8), ("c64", 1024, 4), ("c64", 2048, 4), ("c64", 4096, 4),
+                                      ("c128", 128, 8), ("c128", 256, 4), ("c128", 1024, 4), ("c128", 2048, 4)])
+def test_partly_filled_column_tiles(gpu, prec, n, m):
+    """The last column tile with every number of columns, of infinities beside it
+    none: sequences past the last one are computed on that one's elements."""
+    import genfft_amd as G
+    p, ndt, tdt, tol = PREC[prec]
+    for cols in [*range(1, m), *range(2 * m + 1, 3 * m)]:
+        x = torch.randn(n, cols + 1, dtype=tdt, device=gpu)
+        x[:, cols] = float("inf")  # the pitch's gap
+        y = torch.full((n, cols + 2), 7 + 5j, dtype=tdt, device=gpu)
+        f = G.FFTVert(n, tdt)
+        for inv in (False, True):
+            f.transform(y, cols + 2, x, cols + 1, cols, inv)
+            v = x[:, :cols].cpu().numpy().astype(np.complex128)
+            ref = np.fft.ifft(v, axis=0) * n if inv else np.fft.fft(v, axis=0)
+            got = y.cpu().numpy()
+            assert O.rel_l2_rows(np.ascontiguousarray(got[:, :cols].T), np.ascontiguousarray(ref.T)).max() <= tol(n), cols
+            assert np.all(got[:, cols:] == 7 + 5j)
+
+
+@pytest.mark.parametrize("prec,n,cols,m", [
+    (0, 256, 3968, "16"), (0, 256, 2560, "8"), (0, 256, 3959, "8"), (0, 512, 2816, "16"), (0, 2048, 1408, "8"),
+    (0, 2048, 1403, "4"), (0, 128, 7936, "32"), (0, 64, 14336, "16"), (1, 128, 3584, "8"), (1, 1024, 1408, "8"),
+    (0, 4096, 2048, "8"), (0, 4096, 1024, "4"), (0, 4096, 2052, "4")])
+def test_column_tile_widths(prec, n, cols, m):
+    """Whole columns on whole lines take the wide tile from two thirds of a round
+    of the CUs on, short ones and partial lines from a full round."""
+    st, text = explain(desc(C.GFFT_COLS, prec, n, cols, 1, ins=cols, outs=cols))
+    t = tiles(text)
+    assert st == 0 and len(t) == 1 and field(t[0], "M") == m, text
+
+
+def test_half_lines_are_streamed():
+    """Rows of a matrix a multiple of 64 bytes apart are stored like whole lines
+    (plain=0), from 8 to 16 MiB of 32 bytes; complex64 1024 rows past 40 MiB."""
+    for n, cols, plain in ((2048, 5000, "0"), (2048, 5004, "1"), (2048, 5001, "1"), (256, 5000, "0"), (256, 5004, "0"),
+                           (256, 12804, "1"), (256, 5002, "1"), (1024, 5000, "1"), (1024, 5608, "0"), (512, 12808, "0")):
+        st, text = explain(desc(C.GFFT_COLS, 0, n, cols, 1, ins=cols, outs=cols))
+        t = tiles(text)
+        assert st == 0 and [field(x, "plain") for x in t] == [plain], (n, cols, text)
