@@ -725,6 +725,7 @@ constexpr int64_t kCachedBytes = (int64_t)128 << 20;
 // 4.89 / 4.94, 256 x 12804, 25 MiB, 13.2 / 15.3).
 constexpr int64_t kHalfLines1024 = (int64_t)40 << 20;
 constexpr int64_t kSectorsLeast = (int64_t)8 << 20, kSectorsMost = (int64_t)16 << 20;
+constexpr int64_t kHalfLinesLds = (int64_t)20 << 20;
 // Rows from which a register-held tile per row beats the four-step (MI355X, us
 // per call at 64 / 96 / 128 / 256 rows: c64 32768 points 18.1 / 18.3 / 19.5 /
 // 32 against 16.0 / 23.3 / 28 / 54, c128 16384 points 17.4 / 18.2 / 20.9 / 33
@@ -858,7 +859,8 @@ struct Builder {
             const bool out_pieces = outp == PAT_ROW || (k->M * (int64_t)csize >= 128 && pieces(out_elem) && pieces(out_outer) &&
                                                         pieces(out_outer2) && pieces(out_off_el));
             const bool row_pass = inp == PAT_ROW && outp == PAT_ROW && first && !last && p->d.kind == GFFT_C2C_2D;
-            const bool dirty = row_pass && p->d.n2 <= kShortColumn && bytes > kDirtyLeast && bytes <= kDirtyMost;
+            const bool short_column = p->d.n2 <= kShortColumn || p->d.n2 > max_len(prec, PAT_COL, PAT_COL);
+            const bool dirty = row_pass && short_column && bytes > kDirtyLeast && bytes <= kDirtyMost;
             const bool near_rows = !first && in_buf == out_buf && bytes <= kOneL2Bytes && n_outer1 >= 8;
             const bool short_cols = inp == PAT_COL && outp == PAT_COL && k->L <= kFewRows && bytes >= kFewRowsLeast;
             l.own_lines = (inp == PAT_COL || outp == PAT_COL) && in_lines && out_lines;
@@ -1203,9 +1205,16 @@ struct Builder {
     // complex 2D transform, which keep tiles of 4 columns at 4096 rows (8 columns
     // ran one 4096 x 4096 plane in 126 us instead of 145, FFTVert of 6000 such
     // columns in 110 instead of 156).
-    int col_variant(int L, int64_t cols, int64_t batch, bool plane, bool lines) const
+    int col_variant(int L, int64_t cols, int64_t batch, bool plane, int64_t pitch) const
     {
         if (store) return -1;
+        const bool lines = pitch % 128 == 0, halves = pitch % 64 == 0;
+        // LDS tiles load 16 bytes a lane, which tells where the runs start at half
+        // lines and the loads are most of a short launch (c64 256 x 9208 LDS /
+        // registers 9.4 / 9.9 us, 128 x 9208 6.3 / 6.6; 256 x 12808 12.8 / 11.9)
+        if (!prec && (L == 128 || L == 256) && halves && !lines && cols * L * batch * 8 > kSectorsLeast &&
+            cols * L * batch * 8 <= kHalfLinesLds)
+            return -1;
         int cnt = 0, best = -1;
         const KernelEntry *tab = tile_table(prec, 0, &cnt);
         auto tiles = [&](int m) { return (cols + m - 1) / m * batch; };
@@ -1229,7 +1238,12 @@ struct Builder {
                 (best < 0 || better(tab[i].M, tab[best].M))) best = i;
         if (best < 0) return -1;
         const KernelEntry *d = find_tile(prec, L, PAT_COL, PAT_COL, 0, opts.pipe_mask);
-        return d && d->M > tab[best].M && tiles(d->M) >= p->num_cus ? -1 : best;
+        // the default tile where it is wider: from one full round on, but not with a
+        // second one nearly empty whose stores are plain (c64 2048 rows, 16 / 8
+        // columns a tile: x 4700, 294 of the wide ones, 62.9 / 48.4 us, x 5301 65.3 /
+        // 60.2, x 6501, 407, 69.9 / 75.7)
+        if (!d || d->M <= tab[best].M || tiles(d->M) < p->num_cus) return best;
+        return d->reg && !halves && tiles(d->M) > p->num_cus && tiles(d->M) * 8 <= (int64_t)p->num_cus * 11 ? best : -1;
     }
 
     // Column FFTs of length `rows` down `cols` columns, `batch` matrices.
@@ -1255,8 +1269,7 @@ struct Builder {
         if (rows <= maxcol)
             return tile((int)rows, PAT_COL, PAT_COL, 0, in_buf, 0, out_buf, 0, cols, batch, 1, 0, in_dist, 1,
                         in_pitch, 0, out_dist, 1, out_pitch, TW_NONE, 0, first, last, 
-                        col_variant((int)rows, cols, batch, p->d.kind == GFFT_C2C_2D,
-                                    (in_pitch | out_pitch) * (int64_t)csize % 128 == 0));
+                        col_variant((int)rows, cols, batch, p->d.kind == GFFT_C2C_2D, (in_pitch | out_pitch) * (int64_t)csize));
         // rows = A * B, sub-pass 1 over n2 (length B, rows n1 + A*n2) with
         // twiddle W_rows^(n1*k2) into scratch, sub-pass 2 over n1 (length A)
         // writing row k2 + B*k1.

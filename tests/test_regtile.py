@@ -380,7 +380,8 @@ def test_partly_filled_column_tiles(gpu, prec, n, m):
 @pytest.mark.parametrize("prec,n,cols,m", [
     (0, 256, 3968, "16"), (0, 256, 2560, "8"), (0, 256, 3959, "8"), (0, 512, 2816, "16"), (0, 2048, 1408, "8"),
     (0, 2048, 1403, "4"), (0, 128, 7936, "32"), (0, 64, 14336, "16"), (1, 128, 3584, "8"), (1, 1024, 1408, "8"),
-    (0, 4096, 2048, "8"), (0, 4096, 1024, "4"), (0, 4096, 2052, "4")])
+    (0, 4096, 2048, "8"), (0, 4096, 1024, "4"), (0, 4096, 2052, "4"), (0, 2048, 4700, "8"), (0, 2048, 5301, "8"),
+    (0, 2048, 5800, "16"), (0, 2048, 4800, "16")])
 def test_column_tile_widths(prec, n, cols, m):
     """Whole columns on whole lines take the wide tile from two thirds of a round
     of the CUs on, short ones and partial lines from a full round."""
@@ -397,3 +398,15 @@ def test_half_lines_are_streamed():
         st, text = explain(desc(C.GFFT_COLS, 0, n, cols, 1, ins=cols, outs=cols))
         t = tiles(text)
         assert st == 0 and [field(x, "plain") for x in t] == [plain], (n, cols, text)
+
+
+def test_short_passes_by_pitch_and_size():
+    """Half-line columns of 128 and 256 rows run on the LDS tiles (256 threads)
+    between 8 and 20 MiB; the rows before sub-passes of 64 or 128 points are
+    streamed where all of them would be dirty at the end."""
+    for n, cols, nt in ((256, 9208, "256"), (256, 12808, "512"), (128, 9208, "256"), (256, 9200, "512"), (256, 9204, "512")):
+        t = tiles(explain(desc(C.GFFT_COLS, 0, n, cols, 1, ins=cols, outs=cols))[1])
+        assert field(t[0], "NT") == nt, (n, cols)
+    for w, h, batch, plain in ((128, 8192, 2, "0"), (128, 8192, 4, "1"), (256, 8192, 1, "0"), (256, 4096, 2, "1")):
+        t = tiles(explain(desc(C.GFFT_C2C_2D, 0, w, h, batch))[1])
+        assert field(t[0], "plain") == plain, (w, h, batch)
