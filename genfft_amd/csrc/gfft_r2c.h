@@ -115,13 +115,15 @@ struct RowsEntry {
     KernelEntry entry;
     int mode;
     int64_t most;  // input bytes up to which this shape is taken (0: any)
+    int64_t most_full;  // the same for full spectra
     void (*fn)(RealRowsArgs);
 };
 
-// The kernel of n/2 = L for `bytes` of input (nullptr: none).  `lds`: only
-// tiles kept in LDS; `long_row`: the register-held tile of a row one length
+// The kernel of n/2 = L for `bytes` of input (nullptr: none).  `full`: a full
+// spectrum is written; `lds`: only tiles kept in LDS; `long_row`: the register-held tile of a row one length
 // past the c2c row tiles.
-const RowsEntry *real_rows_entry(int prec, int L, int mode, int64_t bytes, bool lds = false, bool long_row = false);
+const RowsEntry *real_rows_entry(int prec, int L, int mode, int64_t bytes, bool full = false, bool lds = false,
+                                 bool long_row = false);
 hipError_t launch_real_rows(const RowsEntry *e, const RealRowsArgs &a, int64_t grid, hipStream_t s,
                             hipEvent_t stop = nullptr);
 

@@ -257,13 +257,13 @@ __global__ void __launch_bounds__(NT, 4) real_rows_reg_kernel(RealRowsArgs a)
 template <typename T, int MODE, int L, int M, int NT, int... RS>
 constexpr RowsEntry lds_rows()
 {
-    return {entry_shape<T, L, M, NT, LAY_SEQ, PAT_ROW, PAT_ROW, RS...>(), MODE, 0, &real_rows_kernel<T, L, M, NT, MODE, RS...>};
+    return {entry_shape<T, L, M, NT, LAY_SEQ, PAT_ROW, PAT_ROW, RS...>(), MODE, 0, 0, &real_rows_kernel<T, L, M, NT, MODE, RS...>};
 }
 
 template <typename T, int MODE, int HINT, int L, int M, int NT, int... RS>
-constexpr RowsEntry reg_rows(int64_t most = 0)
+constexpr RowsEntry reg_rows(int64_t most = 0, int64_t most_full = 0)
 {
-    return {reg_shape<T, L, M, NT, PAT_ROW, PAT_ROW, RS...>(), MODE, most, &real_rows_reg_kernel<T, L, M, NT, MODE, HINT, RS...>};
+    return {reg_shape<T, L, M, NT, PAT_ROW, PAT_ROW, RS...>(), MODE, most, most_full ? most_full : most, &real_rows_reg_kernel<T, L, M, NT, MODE, HINT, RS...>};
 }
 
 template <typename T, int MODE, int HINT, int L, int NT, int... RS>
@@ -287,21 +287,26 @@ constexpr RowsEntry long_rows()
 // The spectrum side of a short r2c writes two runs of bins per row in opposite
 // directions, which past the caches merge into whole lines less well than the
 // LDS tile's one run: f32 n = 512 lost from 32 MiB on (131072 rows 119 -> 169
-// us), f64 n = 1024 at 1 GiB (406 -> 425 us), hence kSmall and kCached.
-// Eight elements per thread were faster than sixteen up to n = 2048.
+// us), f64 n = 1024 at 1 GiB (406 -> 425 us), hence kSmall and kCached.  A full
+// spectrum's four runs lose earlier, at an output past the Infinity Cache (LDS
+// / registers: f64 n = 1024 x 24000 114 / 129 us, 2048 x 16000 147 / 161, 4096 x
+// 8000 147 / 154; x a third of them 22-40% faster in registers), hence kFull.
+// Eight elements per thread were faster than sixteen up to n = 2048, and for f64
+// r2c n = 8192 (62 rows 10.5 -> 9.4 us, the LDS tile 10.1).
 // The LDS tiles follow the c2c row-tile shapes; from L = 2 (n = 4) on, so
 // short real transforms are one launch as well (n = 2 runs as a copy and the
 // unpack).  Lengths whose register-held tiles hold several rows keep an LDS
-// one for layouts past 32-bit offsets.
+// one for layouts past 32-bit offsets, those with a limit one beyond it.
 constexpr int F = RR_R2C, B = RR_C2R;
 constexpr int64_t kSmall = (int64_t)16 << 20, kCached = (int64_t)512 << 20;
+constexpr int64_t kFull = (int64_t)96 << 20;
 const RowsEntry kRowsF32[] = {
     reg_rows<float, F, HINT_LD, 64, 8, 64, 4, 4, 4>(kSmall),
     reg_rows<float, F, HINT_LD, 128, 4, 64, 8, 4, 4>(kSmall),
     reg_rows<float, F, HINT_LD, 256, 2, 64, 8, 8, 4>(kSmall),
-    reg_rows<float, F, HINT_LD, 512, 1, 64, 8, 4, 4, 4>(),
+    reg_rows<float, F, HINT_LD, 512, 1, 64, 8, 4, 4, 4>(0, (int64_t)160 << 20),
     reg_rows<float, F, HINT_LD, 1024, 1, 128, 8, 8, 4, 4>(),
-    reg_rows<float, F, HINT_LD, 2048, 1, 128, 16, 16, 8>(),
+    reg_rows<float, F, HINT_LD, 2048, 1, 128, 16, 16, 8>(0, kFull),
     reg_rows<float, F, HINT_LD, 4096, 1, 256, 8, 8, 8, 8>(),
     reg_rows<float, F, HINT_LD, 8192, 1, 512, 16, 8, 8, 8>(),
     reg_rows<float, F, HINT_LD, 16384, 1, 512, 32, 32, 16>(),
@@ -325,14 +330,14 @@ const RowsEntry kRowsF32[] = {
 const RowsEntry kRowsF64[] = {
     reg_rows<double, F, HINT_LD, 128, 4, 64, 8, 4, 4>(kSmall),
     reg_rows<double, F, HINT_LD, 256, 2, 64, 8, 8, 4>(kSmall),
-    reg_rows<double, F, HINT_LD, 512, 1, 64, 8, 4, 4, 4>(kCached),
-    reg_rows<double, F, HINT_LD, 1024, 1, 128, 8, 8, 4, 4>(kCached),
-    reg_rows<double, F, HINT_LD, 2048, 1, 256, 8, 8, 8, 4>(),
-    reg_rows<double, F, HINT_LD, 4096, 1, 256, 16, 4, 8, 8>(),
+    reg_rows<double, F, HINT_LD, 512, 1, 64, 8, 4, 4, 4>(kCached, kFull),
+    reg_rows<double, F, HINT_LD, 1024, 1, 128, 8, 8, 4, 4>(kCached, kFull),
+    reg_rows<double, F, HINT_LD, 2048, 1, 256, 8, 8, 8, 4>(0, kFull),
+    reg_rows<double, F, HINT_LD, 4096, 1, 512, 8, 8, 4, 4, 4>(),
     reg_rows<double, F, HINT_LD, 8192, 1, 512, 16, 8, 8, 8>(),
     long_rows<double, F, HINT_LD, 16384, 1024, 16, 16, 8, 8>(),
     reg_rows<double, B, HINT_ST, 128, 4, 64, 4, 4, 8>(kSmall),
-    reg_rows<double, B, HINT_ST, 256, 2, 64, 4, 8, 8>(kCached),
+    reg_rows<double, B, HINT_ST, 256, 2, 64, 4, 8, 8>((int64_t)192 << 20),
     reg_rows<double, B, HINT_ST, 512, 1, 64, 4, 4, 4, 8>(),
     reg_rows<double, B, HINT_ST, 1024, 1, 128, 4, 4, 8, 8>(),
     reg_rows<double, B, HINT_ST, 2048, 1, 256, 4, 8, 8, 8>(),
@@ -348,12 +353,12 @@ const RowsEntry kRowsF64[] = {
 };
 
 template <size_t K>
-const RowsEntry *rows_find(const RowsEntry (&tab)[K], int L, int mode, int64_t bytes, bool lds, bool long_row)
+const RowsEntry *rows_find(const RowsEntry (&tab)[K], int L, int mode, int64_t bytes, bool full, bool lds, bool long_row)
 {
     for (size_t i = 0; i < K; i++) {
         const KernelEntry &e = tab[i].entry;
-        if (e.L == L && tab[i].mode == mode && !(lds && e.reg) && (e.long_row != 0) == long_row &&
-            (!tab[i].most || bytes <= tab[i].most))
+        const int64_t most = full ? tab[i].most_full : tab[i].most;
+        if (e.L == L && tab[i].mode == mode && !(lds && e.reg) && (e.long_row != 0) == long_row && (!most || bytes <= most))
             return &tab[i];
     }
     return nullptr;
@@ -361,9 +366,10 @@ const RowsEntry *rows_find(const RowsEntry (&tab)[K], int L, int mode, int64_t b
 
 }  // namespace
 
-const RowsEntry *real_rows_entry(int prec, int L, int mode, int64_t bytes, bool lds, bool long_row)
+const RowsEntry *real_rows_entry(int prec, int L, int mode, int64_t bytes, bool full, bool lds, bool long_row)
 {
-    return prec ? rows_find(kRowsF64, L, mode, bytes, lds, long_row) : rows_find(kRowsF32, L, mode, bytes, lds, long_row);
+    return prec ? rows_find(kRowsF64, L, mode, bytes, full, lds, long_row)
+                : rows_find(kRowsF32, L, mode, bytes, full, lds, long_row);
 }
 
 hipError_t launch_real_rows(const RowsEntry *e, const RealRowsArgs &a, int64_t grid, hipStream_t s, hipEvent_t stop)

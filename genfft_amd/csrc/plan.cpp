@@ -1366,7 +1366,7 @@ struct Builder {
     bool long_real_rows(int64_t n, int64_t rows) const
     {
         return !store && opts.r2c_fuse && !no_long_rows && rows >= kLongRows && is_pow2(n) && n <= INT32_MAX &&
-               real_rows_entry(prec, (int)(n / 2), RR_R2C, 0, false, true);
+               real_rows_entry(prec, (int)(n / 2), RR_R2C, 0, false, false, true);
     }
 
     // `rows` real transforms of length n in one launch: mode RR_R2C reads
@@ -1376,11 +1376,12 @@ struct Builder {
     int real_rows(int mode, int64_t n, int64_t rows, int in_buf, int64_t in_off_el, int64_t in_row, int out_buf,
                   int64_t out_off_el, int64_t out_row, bool half, bool long_row = false)
     {
-        const RowsEntry *re = real_rows_entry(prec, (int)(n / 2), mode, rows * (n / 2) * (int64_t)csize, false, long_row);
+        const RowsEntry *re = real_rows_entry(prec, (int)(n / 2), mode, rows * (n / 2) * (int64_t)csize,
+                                              mode == RR_R2C && !half, false, long_row);
         // 32-bit byte offsets within a tile; a full spectrum spans n bins
         if (re && re->entry.reg && !(tile_offsets_fit(PAT_ROW, n / 2 + 1, re->entry.M, in_row, 1, csize) &&
                                      tile_offsets_fit(PAT_ROW, n, re->entry.M, out_row, 1, csize)))
-            re = real_rows_entry(prec, (int)(n / 2), mode, 0, true);
+            re = real_rows_entry(prec, (int)(n / 2), mode, 0, false, true);
         if (!re) return fail(GFFT_ERR_UNSUPPORTED, "no real-row kernel for n=%lld", (long long)n);
         if (long_row) long_rows = true;
         const KernelEntry *fe = &re->entry;

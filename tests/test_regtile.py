@@ -410,3 +410,40 @@ def test_short_passes_by_pitch_and_size():
     for w, h, batch, plain in ((128, 8192, 2, "0"), (128, 8192, 4, "1"), (256, 8192, 1, "0"), (256, 4096, 2, "1")):
         t = tiles(explain(desc(C.GFFT_C2C_2D, 0, w, h, batch))[1])
         assert field(t[0], "plain") == plain, (w, h, batch)
+
+
+@pytest.mark.parametrize("prec,n,rows,half,m", [
+    (0, 1024, 40000, False, "1"), (0, 1024, 45000, False, "8"), (0, 1024, 60000, True, "1"), (0, 4096, 6000, False, "1"),
+    (0, 4096, 6500, False, "2"), (0, 4096, 16000, True, "1"), (1, 1024, 12000, False, "1"), (1, 1024, 13000, False, "4"),
+    (1, 1024, 30000, True, "1"), (1, 2048, 6500, False, "2"), (1, 2048, 6500, True, "1")])
+def test_large_full_spectra_take_the_lds_rows(prec, n, rows, half, m):
+    """Full spectra past the Infinity Cache are written in one run a row."""
+    st, text = explain(desc(C.GFFT_R2C, prec, n, 0, rows, flags=C.GFFT_FLAG_HALF if half else 0))
+    line = [ln for ln in text.splitlines() if ln.startswith("real_rows")]
+    assert st == 0 and len(line) == 1 and field(line[0], "M") == m, text
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,rows,full", [(4096, 6200, True), (1024, 12700, True), (2048, 6300, True), (8192, 3, True),
+                                         (8192, 257, False)])
+def test_f64_real_rows_at_the_limits(gpu, n, rows, full):
+    """Either side of kFull, and the 8192-point rows, against numpy."""
+    import genfft_amd as G
+    for b in (rows - 120 if rows > 1000 else rows, rows):
+        x = torch.randn(b, n, dtype=torch.float64, device=gpu)
+        bins = n if full else n // 2 + 1
+        y = torch.full((b, bins), 7 + 5j, dtype=torch.complex128, device=gpu)
+        f = G.RealFFT(n, torch.float64)
+        f.forward(y, x, not full)
+        at = [0, b // 2, b - 1]
+        ref = np.fft.fft(x[at].cpu().numpy())[:, :bins]
+        assert O.rel_l2_rows(y[at].cpu().numpy(), np.ascontiguousarray(ref)).max() <= O.tol_c128(n)
+        assert _worst_rows(y, torch.fft.fft(x)[:, :bins]) <= 2 * O.tol_c128(n)
+        if not full:
+            z = torch.empty_like(x)
+            f.inverse(z, y)
+            assert float(((z / n - x).norm(dim=1) / x.norm(dim=1)).max()) <= 2 * O.tol_c128(n)
+
+
+def _worst_rows(y, ref):
+    return float(((y - ref).abs().square().sum(-1) / ref.abs().square().sum(-1)).max().sqrt())
