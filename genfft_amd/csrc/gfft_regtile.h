@@ -217,7 +217,7 @@ __device__ __forceinline__ void reg_passes(T *plane, cx<T> (&v)[M * L / NT], con
             }
         }
 #pragma unroll
-        for (int e = 0; e < A::W; e++) dft<R>(x + e * R);
+        for (int e = 0; e < A::W; e++) dft<R, (M * L / NT < 32)>(x + e * R);
     }
     if constexpr (sizeof...(RS) > 0) {
         constexpr int R2 = first_radix<RS...>();
