@@ -652,6 +652,9 @@ struct gfft_plan_s {
     // the workspace they were sized for, and no staging copy is needed.
     std::vector<gfft::Launch> alt;
     bool alt_hazard = false;
+    // The launch of a call without an automatic scale, where another tile is
+    // the faster one then (none: `launches`).
+    std::vector<gfft::Launch> unscaled;
     int64_t in_step = 0, out_step = 0, in_step2 = 0, out_step2 = 0;
     void *stage = nullptr;  // copy of an input that overlaps the output (allocated on first use)
     std::mutex host_mu;
@@ -902,6 +905,26 @@ struct Builder {
             if (most && bytes > most) v = -1;
         }
         return v >= 0 || store ? v : narrow_row_variant(prec, n, rows, p->num_cus);
+    }
+
+    // Short 16-bit rows that find no scale of their own are faster on the LDS
+    // tiles, which load 16 bytes a lane, where both sides just fill the Infinity
+    // Cache (MI355X, MiB a side, us LDS / registers: FP16 32 points 64 29.1 / 27.4, 90
+    // 40.0 / 47.7, 128 56.0 / 69.4; FP16 128 points 64 29.0 / 26.0, 90 40.8 / 43.4, 128
+    // 56.4 / 63.5, 160 71.2 / 71.2; BF16, whose conversions the LDS tiles do twice, 32
+    // points 128 64.9 / 73.4, 128 points 110 56.6 / 56.4, 140 70.8 / 68.9).
+    bool lds_when_unscaled(int64_t n, int64_t batch) const
+    {
+        const int64_t bytes = n * batch * (int64_t)csize;
+        if (n > (store == 1 ? 128 : 64)) return false;
+        return bytes > ((int64_t)(n <= 64 ? 72 : 88) << 20) && bytes <= (int64_t)150 << 20;
+    }
+    int lds_rows_h(int n, int64_t batch, int64_t in_dist, int64_t out_dist)
+    {
+        int cnt = 0;
+        const KernelEntry *tab = tile_table(prec, store, &cnt), *k = find_tile(prec, n, PAT_ROW, PAT_ROW, 0, 3, -1, store, true);
+        return tile(n, PAT_ROW, PAT_ROW, 0, B_IN, 0, B_OUT, 0, batch, 1, 1, 0, 0, in_dist, 1, 0, 0, out_dist, 1, TW_NONE, 0,
+                    true, true, k ? (int)(k - tab) : -1);
     }
 
     // Register-held row tile for `batch` rows of length n, one past the LDS
@@ -1518,6 +1541,13 @@ int build_plan(gfft_plan_s *p, bool dry, const PlanOpts *forced = nullptr, bool 
         p->in_step = id * (int64_t)cs;
         p->out_step = od * (int64_t)cs;
         st = b.c2c_1d(n, batch, B_IN, 0, id, B_OUT, 0, od, true, true);
+        if (!st && b.store && p->launches.size() == 1 && p->launches[0].k->reg && b.lds_when_unscaled(n, batch)) {
+            std::vector<Launch> own;
+            own.swap(p->launches);
+            st = b.lds_rows_h((int)n, batch, id, od);
+            p->unscaled.swap(p->launches);
+            p->launches.swap(own);
+        }
         break;
     }
     case GFFT_R2C: {
@@ -1892,7 +1922,8 @@ int validate_list(const gfft_plan_s *p, const std::vector<Launch> &launches);
 
 int validate(const gfft_plan_s *p)
 {
-    const int st = validate_list(p, p->launches);
+    int st = validate_list(p, p->launches);
+    if (!st) st = validate_list(p, p->unscaled);
     return st ? st : validate_list(p, p->alt);
 }
 
@@ -2055,21 +2086,22 @@ int validate_list(const gfft_plan_s *p, const std::vector<Launch> &launches)
     return GFFT_OK;
 }
 
-int describe_launches(const std::vector<Launch> &launches, const std::string &head, char *buf, size_t len);
+std::string launches_text(const std::vector<Launch> &launches, const std::string &head);
+int copy_text(const std::string &s, char *buf, size_t len);
 
 int describe(const gfft_plan_s *p, char *buf, size_t len)
 {
     char line[256];
     snprintf(line, sizeof(line), "plan in_bytes=%zu out_bytes=%zu scratch_bytes=%zu\n", p->in_bytes,
              p->out_bytes, p->scratch_bytes);
-    if (p->alt.empty()) return describe_launches(p->launches, line, buf, len);
-    int st = describe_launches(p->launches, line, buf, len);
-    if (st) return st;
-    const std::string head = std::string(buf) + "on overlapping buffers:\n";
-    return describe_launches(p->alt, head, buf, len);
+    std::string text = launches_text(p->launches, line);
+    if (!p->unscaled.empty()) text = launches_text(p->unscaled, text + "without an automatic scale:\n");
+    if (!p->alt.empty()) text = launches_text(p->alt, text + "on overlapping buffers:\n");
+    return copy_text(text, buf, len);
 }
 
-int describe_launches(const std::vector<Launch> &launches, const std::string &head, char *buf, size_t len)
+// `head` and a line for each launch.
+std::string launches_text(const std::vector<Launch> &launches, const std::string &head)
 {
     std::string s = head;
     char line[1024];
@@ -2163,6 +2195,11 @@ int describe_launches(const std::vector<Launch> &launches, const std::string &he
         }
         s += line;
     }
+    return s;
+}
+
+int copy_text(const std::string &s, char *buf, size_t len)
+{
     if (s.size() + 1 > len) return fail(GFFT_ERR_INVALID_ARG, "describe buffer too small (%zu bytes needed)", s.size() + 1);
     memcpy(buf, s.c_str(), s.size() + 1);
     return GFFT_OK;
@@ -2186,7 +2223,8 @@ int run_launches(const std::vector<Launch> &launches, int prec, int xcd_remap, c
 // The launches this call runs, and whether its buffers overlap in a way their
 // order can corrupt (see gfft_plan_s::overlap_hazard), so that the input has
 // to be staged.
-const std::vector<Launch> &route(const gfft_plan_s *p, const void *in, const void *out, bool *stage)
+const std::vector<Launch> &route(const gfft_plan_s *p, const void *in, const void *out, bool *stage,
+                                 bool automatic_scale = false)
 {
     const uintptr_t i0 = (uintptr_t)in, o0 = (uintptr_t)out;
     const bool shifted = i0 < o0 + p->out_bytes && o0 < i0 + p->in_bytes &&
@@ -2198,7 +2236,7 @@ const std::vector<Launch> &route(const gfft_plan_s *p, const void *in, const voi
                                    l.out_steps | (l.out_buf == B_OUT ? o0 : i0)) < 0;
     alt = alt && !p->alt.empty();
     *stage = shifted && (alt ? p->alt_hazard : p->overlap_hazard);
-    return alt ? p->alt : p->launches;
+    return alt ? p->alt : !automatic_scale && !p->unscaled.empty() ? p->unscaled : p->launches;
 }
 
 // Whether the plan's one launch holds every transform whole in a workgroup's
@@ -2225,7 +2263,7 @@ int run(gfft_plan_s *p, const void *in, void *out, int direction, hipStream_t s,
         return fail(GFFT_ERR_INVALID_ARG, "plan created with GFFT_FLAG_NO_WORKSPACE holds no workspace: "
                                           "run it with gfft_execute_noalloc");
     bool stage = false;
-    const std::vector<Launch> &launches = route(p, in, out, &stage);
+    const std::vector<Launch> &launches = route(p, in, out, &stage, scale.automatic != nullptr);
     if ((!p->scratch || !uses_scratch(launches)) && !stage)  // no shared workspace: calls on any streams are independent
         return run_launches(launches, p->prec, p->xcd_remap, in, out, p->scratch, direction, s, events, scale);
     std::lock_guard<std::mutex> lk(p->order.mu);
@@ -3526,7 +3564,7 @@ int gfft_batch_plan_describe(gfft_batch_plan plan, char *buf, size_t len)
     char head[256];
     snprintf(head, sizeof(head), "batch jobs=%lld scratch_bytes=%zu offsets_even=%d\n", (long long)plan->count,
              plan->scratch_bytes, (int)plan->offsets_even);
-    return describe_launches(plan->launches, head, buf, len);
+    return copy_text(launches_text(plan->launches, head), buf, len);
 }
 
 }  // extern "C"

@@ -5,6 +5,9 @@ complex64, 1e-15*log2 N complex128) at the edges of the shapes: tiles with
 missing sequences, padded pitches, the smallest batch that takes a row past
 the LDS tiles, and overlapping buffers there.
 """
+import ctypes
+import re
+
 import numpy as np
 import pytest
 import torch
@@ -481,3 +484,47 @@ def test_rounding_is_no_larger_than_before(gpu, kind, n, count, was):
         ref = torch.fft.fft(x.to(torch.complex128))
     err = float((y.to(torch.complex128) - ref).norm() / ref.norm())
     assert err <= 1.003 * was, err
+
+
+def test_short_half_rows_without_a_scale():
+    """The LDS tile where both sides just fill the Infinity Cache and the call
+    finds no scale of its own; the register-held one finds it."""
+    for n, mb, two, bf in ((32, 64, False, False), (32, 90, True, True), (64, 128, True, True), (128, 128, True, False),
+                           (128, 80, False, False), (128, 160, False, False), (256, 128, False, False)):
+        st, text = explain(desc(C.GFFT_C2C, C.GFFT_BF16, n, 0, (mb << 20) // (4 * n)))
+        assert st == 0 and ("without an automatic scale:" in text) == bf, (n, mb)
+        st, text = explain(desc(C.GFFT_C2C, C.GFFT_F16, n, 0, (mb << 20) // (4 * n)))
+        assert st == 0 and ("without an automatic scale:" in text) == two, (n, mb)
+        if two:
+            own, given = [ln for ln in text.splitlines() if ln.startswith("tile")]
+            assert field(own, "NT") != field(given, "NT") or field(own, "M") != field(given, "M")
+
+
+def test_description_needs_one_buffer():
+    """A buffer of the length a short one is told holds the whole text."""
+    lib = C.lib()
+    d = desc(C.GFFT_C2C, 0, 1 << 16, 0, 300)
+    assert lib.gfft_plan_explain(ctypes.byref(d), ctypes.create_string_buffer(80), 80) != 0
+    need = int(re.search(r"\((\d+) bytes needed", lib.gfft_last_error().decode()).group(1))
+    buf = ctypes.create_string_buffer(need)
+    assert lib.gfft_plan_explain(ctypes.byref(d), buf, need) == 0
+    assert "xcd_four_step" in buf.value.decode() and "on overlapping buffers:" in buf.value.decode()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fmt", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("n,mb", [(32, 73), (64, 100), (128, 149), (256, 101)])
+def test_short_half_rows_both_ways(gpu, fmt, n, mb):
+    """With no scale and the automatic one."""
+    import genfft_amd as G
+    batch = (mb << 20) // (4 * n)
+    x = (torch.randn(batch, n, 2, device=gpu) * 0.1).to(fmt)
+    v = torch.view_as_complex(x[:1000].float()).to(torch.complex128)
+    ref = torch.fft.fft(v)
+    eps = 2.0 ** (-10 if fmt == torch.float16 else -7)
+    (plain, _), (auto, scales) = G.fft16(x), G.fft16(x, scale="auto")
+    for y in (plain, auto):
+        got = torch.view_as_complex(y[:1000].float()).to(torch.complex128)
+        assert float((got - ref).norm() / ref.norm()) <= eps
+    assert bool((scales == 1).all())
+    assert float((auto.float() - plain.float()).norm() / plain.float().norm()) <= eps  # every row
