@@ -324,7 +324,7 @@ const RowsEntry kRowsF32[] = {
 #define BOTH(...) lds_rows<float, F, __VA_ARGS__>(), lds_rows<float, B, __VA_ARGS__>()
     BOTH(2, 1024, 128, 2), BOTH(4, 1024, 256, 4), BOTH(8, 512, 256, 8), BOTH(16, 256, 256, 16), BOTH(32, 128, 256, 8, 4),
     BOTH(64, 64, 256, 8, 8), BOTH(128, 32, 256, 16, 8), BOTH(256, 16, 256, 16, 16), BOTH(512, 8, 256, 8, 8, 8),
-    BOTH(1024, 4, 256, 16, 16, 4), BOTH(2048, 2, 256, 16, 16, 8),
+    lds_rows<float, F, 2048, 2, 256, 16, 16, 8>(),
 #undef BOTH
 };
 const RowsEntry kRowsF64[] = {
@@ -346,8 +346,8 @@ const RowsEntry kRowsF64[] = {
     long_rows<double, B, HINT_ST, 16384, 1024, 8, 8, 16, 16>(),
 #define BOTH(...) lds_rows<double, F, __VA_ARGS__>(), lds_rows<double, B, __VA_ARGS__>()
     BOTH(2, 512, 64, 2), BOTH(4, 512, 128, 4), BOTH(8, 256, 128, 8), BOTH(16, 128, 128, 16), BOTH(32, 64, 128, 8, 4),
-    BOTH(64, 32, 128, 8, 8), BOTH(128, 16, 128, 16, 8), BOTH(256, 8, 256, 8, 8, 4), BOTH(512, 4, 256, 8, 8, 8),
-    BOTH(1024, 2, 256, 8, 4, 8, 4),
+    BOTH(64, 32, 128, 8, 8), BOTH(128, 16, 128, 16, 8), BOTH(256, 8, 256, 8, 8, 4),
+    lds_rows<double, F, 512, 4, 256, 8, 8, 8>(), lds_rows<double, F, 1024, 2, 256, 8, 4, 8, 4>(),
     lds_rows<double, F, 2048, 1, 256, 8, 8, 8, 4>(),
 #undef BOTH
 };
