@@ -2804,8 +2804,10 @@ std::vector<PlanOpts> tune_candidates(int prec, int64_t n)
         }
     int nx = 0;
     const XcdEntry *xcd = xcd_entries(&nx);
-    for (int i = 0; i < nx; i++)  // untuned: both passes in one launch, batch permitting
-        if (xcd[i].prec == prec && ((int64_t)1 << xcd[i].lg) == n) out.push_back(PlanOpts{});
+    // untuned: both passes in one launch, batch permitting (once, whatever rings
+    // the length is listed with)
+    if (std::any_of(xcd, xcd + nx, [&](const XcdEntry &e) { return e.prec == prec && ((int64_t)1 << e.lg) == n; }))
+        out.push_back(PlanOpts{});
     const int lg = ilog2(n), maxcol = max_len(prec, PAT_COL, PAT_COL), maxtr = max_len(prec, PAT_ROW, PAT_COL);
     for (int l1 = 1; l1 < lg; l1++) {
         const int64_t N1 = (int64_t)1 << l1, N2 = (int64_t)1 << (lg - l1);

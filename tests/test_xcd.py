@@ -328,3 +328,14 @@ def test_alignments(gpu, monkeypatch, prec, n, batch, pin, pout, shift_in, shift
     two = shift_out and prec == "c64" and n in (1 << 18, 1 << 19)
     if not pin and not pout:
         assert len(plan.profile(x, out)) == (2 if two else 1)
+
+
+@pytest.mark.gpu
+def test_untuned_candidate_is_listed_once(gpu):
+    """2^20 has two rings; the autotuner times its untuned plan once."""
+    import genfft_amd as G
+    try:
+        rep = G.autotune(1 << 20, 26, torch.complex64, reps=1)
+        assert sum(c["n1_log2"] == 0 and c["row_variant"] < 0 for c in rep["candidates"]) == 1
+    finally:
+        C.check(C.lib().gfft_tuning_clear())
