@@ -3,8 +3,9 @@
 // Two launches write the whole intermediate to HBM and read it back.  Here each
 // XCD takes whole transforms, its workgroups running the column tiles of one
 // and, a few transforms later, its transposing row tiles; the intermediate in
-// between lives in a ring of 48-160 MB (8-16 transforms per XCD) that the 256 MB
-// Infinity Cache holds, so HBM moves the input and the output only.  Tiles hand
+// between passes through a ring of 48-256 MiB (3-18 transforms per XCD) that is
+// reused before the Infinity Cache has to write all of it out: the traffic past
+// the L2 is that of two launches, at 6.7 TB/s where those reach 5.3.  Tiles hand
 // over within one XCD, whose L2 is common to them, which needs no cache
 // write-back.
 #pragma once

@@ -1,21 +1,25 @@
 // kern_xcd.hip -- both passes of a four-step in one persistent launch, each
 // transform on one XCD (see gfft_xcd.h).
 //
-// What bounds it: how many tiles are in flight.  Four workgroups of 256 threads
-// (or two of 512) hold 4 MB of tiles per XCD, as much as its L2, so the ring's
-// traffic goes on to the Infinity Cache (counters: reads and writes past the L2
-// are those of two launches), and a row tile must come that many tasks after its
-// column tiles not to wait: with `lag` 2 instead of 10, c64 2^16 x 2048 takes
-// 0.83-2.1 ms instead of 0.63.  MI355X against two launches, ms at 1 GiB / us at
-// 238 MiB: c64 2^16 0.75 -> 0.63 / 198 -> 170, 2^17 0.80 -> 0.64 / 205 -> 168,
-// 2^18 0.78 -> 0.64 / 201 -> 174, 2^19 0.86 -> 0.66 / 211 -> 178, 2^20 0.81 -> 0.64 /
-// 215 -> 187; c128 2^15 0.80 -> 0.65 / 208 -> 166, 2^16 0.81 -> 0.64 / 210 -> 165,
-// 2^17 0.85 -> 0.70 / 219 -> 181, 2^18 0.84 -> 0.68 / 213 -> 191 (one pass over HBM
-// at a copy's rate: 0.39 / 91).  Near the smallest batches: c64 2^16 x 145 76 -> 70
-// us, 2^17 x 81 84 -> 73, 2^20 x 25 191 -> 175, c128 2^18 x 41 156 -> 143: it is
-// taken wherever its ring fits the workspace the two launches would have.  Longer
-// transforms' rings leave the Infinity Cache; c128 2^19 gained 4% at 1 GiB and
-// nothing at 238 MiB and stays on two launches.
+// What bounds it: the traffic past the L2, which is that of two launches (2.0 GiB
+// read and 2.0 written for 1 GiB of c64 2^20 or 2^16: 6.7 TB/s, where copies that
+// stay in the Infinity Cache reach 7), and for the shortest lengths the turns of
+// an XCD's counters.  Four workgroups of 256 threads (or two of 512) hold 4 MB of
+// tiles per XCD, as much as its L2, so the ring's traffic goes on to the Infinity
+// Cache, and a row tile must come that many tasks after its column tiles not to
+// wait: with `lag` 2 instead of 10, c64 2^16 x 2048 takes 0.83-2.1 ms instead of
+// 0.62.  MI355X against two launches, ms at 1 GiB / us at an eighth to a half of it:
+// c64 2^16 0.75 -> 0.62 / 118 -> 103 (x 260), 2^17 0.79 -> 0.64 / 146 -> 122 (x 164),
+// 2^18 0.77 -> 0.65 / 264 -> 233 (x 164), 2^19 0.85 -> 0.65 / 429 -> 348 (x 130), 2^20
+// 0.82 -> 0.64 / 441 -> 335 (x 64); c128 2^15 0.76 -> 0.63 / 131 -> 113 (x 290), 2^16
+// 0.81 -> 0.63 / 157 -> 119 (x 162), 2^17 0.85 -> 0.70 / 300 -> 250 (x 171), 2^18 0.83
+// -> 0.68 / 290 -> 248 (x 84); a 1 GiB copy takes 0.39.  Near the smallest batches:
+// c64 2^16 x 146 73.6 -> 69.9 us, x 190 85.1 -> 84.7, 2^17 x 82 80.5 -> 73.3, 2^20 x 26
+// 191 -> 182, c128 2^15 x 112 59.4 -> 59.8, 2^18 x 42 158 -> 142: it is taken wherever
+// its ring fits the workspace the two launches would have (but for layouts
+// whose runs share lines, see the table).  Longer transforms' rings leave the
+// Infinity Cache; c128 2^19 gained 4% at 1 GiB and nothing at 238 MiB and stays
+// on two launches.
 #include "gfft_regtile.h"
 #include "gfft_xcd.h"
 

@@ -647,9 +647,11 @@ struct gfft_plan_s {
     // members, or rows) and in_step2 / out_step2 (2D images).
     bool overlap_hazard = false;
     // The launches of the same plan without register-held long rows and
-    // one-launch four-steps (none: it has none).  They read every input before they write an output wherever
-    // the four-step does, so a call on overlapping buffers runs these, through
-    // the workspace they were sized for, and no staging copy is needed.
+    // one-launch four-steps (none: it has none).  They read every input before
+    // they write an output wherever the four-step does, so a call on
+    // overlapping buffers runs these, through the workspace they were sized for,
+    // and no staging copy is needed; so does one whose addresses are a layout
+    // that the one launch is not taken for (xcd_hints).
     std::vector<gfft::Launch> alt;
     bool alt_hazard = false;
     // The launch of a call without an automatic scale, where another tile is
@@ -928,8 +930,8 @@ struct Builder {
     }
 
     // Register-held row tile for `batch` rows of length n, one past the LDS
-    // row tiles, or -1 (four-step).  One workgroup owns a row, so below half
-    // the CUs the four-step's shorter tiles spread a small batch wider.
+    // row tiles, or -1 (four-step).  One workgroup owns a row, so below
+    // kLongRows of them the four-step's shorter tiles spread a small batch wider.
     int long_row_variant(int64_t n, int64_t batch) const
     {
         if (store || no_long_rows || opts.dual || opts.n1_log2) return -1;
@@ -1291,7 +1293,7 @@ struct Builder {
         const int maxcol = max_len(prec, PAT_COL, PAT_COL, store);
         if (rows <= maxcol)
             return tile((int)rows, PAT_COL, PAT_COL, 0, in_buf, 0, out_buf, 0, cols, batch, 1, 0, in_dist, 1,
-                        in_pitch, 0, out_dist, 1, out_pitch, TW_NONE, 0, first, last, 
+                        in_pitch, 0, out_dist, 1, out_pitch, TW_NONE, 0, first, last,
                         col_variant((int)rows, cols, batch, p->d.kind == GFFT_C2C_2D, (in_pitch | out_pitch) * (int64_t)csize));
         // rows = A * B, sub-pass 1 over n2 (length B, rows n1 + A*n2) with
         // twiddle W_rows^(n1*k2) into scratch, sub-pass 2 over n1 (length A)
@@ -2516,11 +2518,13 @@ int check_noalloc_fit(const gfft_plan_s *p)
 // Uneven batches: transforms of mixed power-of-two lengths at arbitrary
 // offsets, each with its own direction.
 //   lengths 1 .. MixCfg::TOT   one persistent mixed-size launch (device work
-//                              queue), preceded by a one-thread counter reset;
-//   longer lengths            per length class, the single-pass or four-step
-//                              tile launches with job tables along the
-//                              transform index.
-// The whole list is captured once into a HIP graph and replayed.  (Captured
+//                              queue, which clears itself);
+//   longer lengths            per length class, the single-pass, one-launch or
+//                              two-launch four-step tiles with job tables
+//                              along the transform index.
+// A list of more than kFewLaunches launches is captured once into a HIP graph
+// and replayed, a shorter one is enqueued (one-launch four-steps with the reset
+// of their counters).  (Captured
 // with the classes forked onto four side streams, the replay ran slower than
 // one stream: the persistent class kernels each size their grid to the whole
 // GPU and contend when they overlap.)
