@@ -314,7 +314,6 @@ __device__ __forceinline__ void reg_tile(T *plane, const TileArgs &a, const cx<T
     // per-thread byte offset (the host admits only layouts it fits)
     {
         using A = Bfly<L, M, NT, MP, R1>;
-        const bool sw = swap_in_of(a, o);
         in += INP == PAT_ROW ? (int64_t)s0 * a.in_inner : (int64_t)s0;
         const int64_t step = (INP == PAT_ROW ? (int64_t)A::LR : (int64_t)A::LR * a.in_elem) * (int64_t)sizeof(cx<T>);
         const char *ib = reinterpret_cast<const char *>(in);
@@ -322,8 +321,9 @@ __device__ __forceinline__ void reg_tile(T *plane, const TileArgs &a, const cx<T
         for (int q = 0; q < A::N; q++) {
             // a sequence past the last one is computed on that one's elements
             // and not stored (a branch around each load instead made the one
-            // partly filled tile the slowest: c64 4096 x 107 columns 20.3 us)
-            const int s = min(A::s(tid, q), nvalid - 1), j = A::j(tid, q);
+            // partly filled tile the slowest: c64 4096 x 107 columns 20.4 us, 17.8 so);
+            // pairs stay one access, of the last two sequences
+            const int s = min(A::s(tid, q), max(nvalid - A::W, 0)), j = A::j(tid, q);
             const uint32_t to = (INP == PAT_ROW ? (uint32_t)s * (uint32_t)a.in_inner + (uint32_t)j
                                                 : (uint32_t)j * (uint32_t)a.in_elem + (uint32_t)s) * (uint32_t)sizeof(cx<T>);
             cx<T> *x = &v[q * A::W * R1];
@@ -335,26 +335,33 @@ __device__ __forceinline__ void reg_tile(T *plane, const TileArgs &a, const cx<T
                 for (int r = 0; r < R1; r++) x[r] = agent_load<T>(buffer, to, (int)(r * step));
                 continue;
             }
+            if (A::W == 1 || nvalid > 1) {
 #pragma unroll
-            for (int r = 0; r < R1; r++) {
-                const cx<T> *p = reinterpret_cast<const cx<T> *>(ib + r * step + to);
-                if (A::W == 1 || nvalid == M) {
-                    reg_load<HINT, A::W>(p, x + r, R1);
-                } else {
-                    // pairs stay one access: the last sequence alone is the second
-                    // of the pair before it (its partner's result is not stored)
-                    const bool one = s + 1 >= nvalid;
-                    cx<T> y[2];
-                    if (nvalid > 1) reg_load<HINT, 2>(p - one, y, 1);
-                    else reg_load<HINT, 1>(p, y + 1, 0);
-                    x[r] = one ? y[1] : y[0];
-                    x[R1 + r] = y[1];
+                for (int r = 0; r < R1; r++)
+                    reg_load<HINT, A::W>(reinterpret_cast<const cx<T> *>(ib + r * step + to), x + r, R1);
+            } else {
+#pragma unroll
+                for (int r = 0; r < R1; r++) {
+                    reg_load<HINT, 1>(reinterpret_cast<const cx<T> *>(ib + r * step + to), x + r, R1);
+                    x[(A::W - 1) * R1 + r] = x[r];
                 }
             }
         }
-        if (sw) {
+        // read once the loads are on their way: the wait for it would hold them up
+        // (c128 64 x 64 images 6.9 us, 6.7 so)
+        asm volatile("" ::: "memory");
+        if (swap_in_of(a, o)) {
 #pragma unroll
             for (int k = 0; k < E; k++) v[k] = swap_ri(v[k]);
+        }
+        if (A::W == 2 && (nvalid & 1)) {
+            // the last sequence is the second of the two its thread has read
+            // (the other result of that thread is not stored)
+#pragma unroll
+            for (int q = 0; q < A::N; q++)
+#pragma unroll
+                for (int r = 0; r < R1; r++)
+                    if (A::s(tid, q) >= nvalid - 1) v[q * A::W * R1 + r] = v[(q + 1) * A::W * R1 - R1 + r];
         }
     }
     reg_passes<T, L, M, NT, G, MP, MPL, MPL, 1, RS...>(plane, v, reinterpret_cast<const cx<T> *>(a.pass_tw), tid, a,
