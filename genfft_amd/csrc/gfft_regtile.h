@@ -309,6 +309,11 @@ __device__ __forceinline__ void reg_tile(T *plane, const TileArgs &a, const cx<T
     constexpr int CM = col_map<T, L, M, NT, RS...>();
     constexpr int MP = INP == PAT_ROW ? MAP_J : CM, MPL = OUTP == PAT_ROW ? MAP_J : CM;
     using G = PlaneGeom<T, L, M, R1, INP == PAT_ROW>;
+    // Columns of 4096 rows: a wave has three loads on their way, not all of them;
+    // the tiles that share their lines stay closer together (c64 us all / three:
+    // 4096 x 3000 77 / 72, 4096 x 1024 24.4 / 22.3, 4096 x 8 9.8 / 9.9; 2048 x 5000
+    // 48.0 / 49.3, 1024 x 8192 24.1 / 25.6, c128 1024 x 4096 28.7 / 31.7)
+    constexpr bool kFewLoads = INP == PAT_COL && sizeof(T) == 4 && L >= 4096;
     cx<T> v[E];
     // HBM accesses: a uniform 64-bit base for each r plus one 32-bit
     // per-thread byte offset (the host admits only layouts it fits)
@@ -337,8 +342,10 @@ __device__ __forceinline__ void reg_tile(T *plane, const TileArgs &a, const cx<T
             }
             if (A::W == 1 || nvalid > 1) {
 #pragma unroll
-                for (int r = 0; r < R1; r++)
+                for (int r = 0; r < R1; r++) {
                     reg_load<HINT, A::W>(reinterpret_cast<const cx<T> *>(ib + r * step + to), x + r, R1);
+                    if constexpr (kFewLoads) asm volatile("s_waitcnt vmcnt(2)" ::: "memory");
+                }
             } else {
 #pragma unroll
                 for (int r = 0; r < R1; r++) {
