@@ -719,6 +719,21 @@ constexpr int64_t kOneL2Bytes = (int64_t)8 << 20;
 // x 1048576 108 / 101; 128 rows x 32768 11.1 / 12.7).
 constexpr int kFewRows = 64;
 constexpr int64_t kFewRowsLeast = (int64_t)16 << 20;
+// So do columns whose rows are `lines` (of 128 bytes) apart when one, two or
+// four of them come to 1024 +- 40 lines, an odd multiple of 8: every such step
+// down a column comes back to almost the same place in 128 KiB (found by a sweep
+// of pitches; us hardware's order / neighbours on one XCD; c64 256 rows, lines 500
+// 9.25 / 8.26, 508 8.91 / 8.32, 524 10.14 / 9.23, 1000 13.3 / 12.1, 250 6.05 / 5.42, but
+// 499 7.88 / 8.23, 501 7.92 / 8.21, 504 7.88 / 8.31, 512 8.03 / 9.00; 512 rows, 492
+// 13.2 / 12.7, 500 14.8 / 13.0, 508 15.2 / 13.5, 532 17.4 / 16.7, but 484 12.6 / 12.5,
+// 496 12.5 / 12.7; c128 512 rows, 250 10.2 / 9.1, 254 10.1 / 9.3, 252 8.9 / 9.1; 128
+// rows, 1000 8.24 / 7.97, 1016 8.45 / 8.10, 500 5.5 / 5.5, 516 6.00 / 6.31).
+inline bool crowded(int L, int64_t pitch_bytes)
+{
+    if (L < 128 || pitch_bytes % 128) return false;
+    const int64_t lines = pitch_bytes / 128, low = lines & -lines;
+    return low >= (L < 256 ? 8 : 2) && low <= 8 && lines / low >= 123 && lines / low <= 133;
+}
 // Row batches of at most this many bytes a side take the `cached` row tiles
 // (c64 2048 points on MI355X: 64 MiB 59.8 -> 55.8 us, 128 MiB 101.3 -> 101.4).
 constexpr int64_t kCachedBytes = (int64_t)128 << 20;
@@ -869,7 +884,9 @@ struct Builder {
             const bool near_rows = !first && in_buf == out_buf && bytes <= kOneL2Bytes && n_outer1 >= 8;
             const bool short_cols = inp == PAT_COL && outp == PAT_COL && k->L <= kFewRows && bytes >= kFewRowsLeast;
             l.own_lines = (inp == PAT_COL || outp == PAT_COL) && in_lines && out_lines;
-            l.row_order = near_rows || short_cols;
+            const bool crowd = inp == PAT_COL && outp == PAT_COL &&
+                               (crowded(k->L, in_elem * (int64_t)csize) || crowded(k->L, out_elem * (int64_t)csize));
+            l.row_order = near_rows || short_cols || crowd;
             l.plain = k->fn_plain &&
                       (!out_pieces || near_rows || (!last && !dirty && bytes <= (row_pass ? kKeptRowBytes : kKeptBytes)));
         }
@@ -2115,7 +2132,7 @@ std::string launches_text(const std::vector<Launch> &launches, const std::string
             snprintf(line, sizeof(line),
                      "%s L=%d M=%d NT=%d layout=%d inp=%d outp=%d lds=%d pipe=%d grid=%lld rad=%d,%d,%d,%d tiles=%d "
                      "n_inner=%d tiles_inner=%d n_outer1=%d in=%s+%lld out=%s+%lld "
-                     "in_strides=%lld,%lld,%lld,%lld out_strides=%lld,%lld,%lld,%lld tw=%d first=%d last=%d vin=%d vout=%d runs=%d lines=%d plain=%d\n",
+                     "in_strides=%lld,%lld,%lld,%lld out_strides=%lld,%lld,%lld,%lld tw=%d first=%d last=%d vin=%d vout=%d runs=%d lines=%d plain=%d order=%d\n",
                      l.k->long_row ? "long_row" : "tile", l.k->L, l.k->M, l.k->NT, l.k->layout, l.k->inp, l.k->outp,
                      l.k->lds_bytes, l.k->persistent, (long long)l.grid, l.k->rad[0],
                      l.k->nrad > 1 ? l.k->rad[1] : 0, l.k->nrad > 2 ? l.k->rad[2] : 0,
@@ -2124,7 +2141,7 @@ std::string launches_text(const std::vector<Launch> &launches, const std::string
                      (long long)a.in_outer2, (long long)a.in_outer, (long long)a.in_inner, (long long)a.in_elem,
                      (long long)a.out_outer2, (long long)a.out_outer, (long long)a.out_inner,
                      (long long)a.out_elem, a.tw_mode, (int)l.first, (int)l.last, (int)l.vin_ok, (int)l.vout_ok, a.runs, (int)l.own_lines,
-                     (int)l.plain);
+                     (int)l.plain, (int)l.row_order);
             break;
         }
         case LT_DUAL: {

@@ -403,6 +403,26 @@ def test_half_lines_are_streamed():
         assert st == 0 and [field(x, "plain") for x in t] == [plain], (n, cols, text)
 
 
+def test_pitches_that_crowd_keep_neighbours_together():
+    """From 256 rows on, columns whose row distance is 2, 4 or 8 times an odd
+    number of 123 to 133 lines of 128 bytes take the tile order that keeps
+    neighbours on one XCD (order=1)."""
+    for prec, n, lines, order in ((0, 256, 500, "1"), (0, 512, 492, "1"), (0, 512, 532, "1"), (0, 256, 1000, "1"),
+                                  (0, 1024, 250, "1"), (1, 512, 254, "1"), (0, 512, 484, "0"), (0, 512, 540, "0"),
+                                  (0, 256, 504, "0"), (0, 256, 512, "0"), (0, 256, 501, "0"), (0, 128, 500, "0"), (0, 128, 1000, "1"),
+                                  (1, 512, 256, "0"), (0, 512, 125, "0")):
+        cols = lines * (8 if prec else 16)
+        t = tiles(explain(desc(C.GFFT_COLS, prec, n, cols, 1, ins=cols, outs=cols))[1])
+        assert [field(x, "order") for x in t] == [order], (prec, n, lines)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("prec,n,cols,pin,pout", [
+    ("c64", 256, 8000, 0, 0), ("c64", 512, 4063, 1, 33), ("c128", 512, 2000, 48, 0)])
+def test_columns_at_those_pitches(gpu, prec, n, cols, pin, pout):
+    test_columns_vs_float64(gpu, prec, n, cols, pin, pout)
+
+
 def test_short_passes_by_pitch_and_size():
     """Half-line columns of 128 and 256 rows run on the LDS tiles (256 threads)
     between 8 and 20 MiB; the rows before sub-passes of 64 or 128 points are
